@@ -132,24 +132,26 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
     ctx->kf_split = ctx->kf_split_ok;
     ctx->kforce_lds_split = kforce_lds_bytes(K, KF_SPLIT_WAVES, ctx->kf_chunk_split);
     std::vector<int> gcol;
-    std::vector<int4> mf_tiles, mf_rt, mf_rt_small, ks_col;
-    std::vector<int2> ks_unit;
+    std::vector<int4> mf_tiles, mf_rt, mf_rt_small, ks_col, ks_slot, ks_slot_ph;
     {
         const char *kv = std::getenv("QTP_KSPACE");
         const bool want_mf = !(kv && std::strcmp(kv, "vector") == 0);
         ctx->kf_mf_ok = 2 * K <= 4 * MF_MAXKS && ctx->G > 0 && ctx->AC % 4 == 0 &&
-                        build_mf_layout(g, gcol, mf_tiles, ctx->mf_Mp, ctx->mf_nks, ks_col, ks_unit);
+                        build_mf_layout(g, gcol, mf_tiles, ctx->mf_Mp, ctx->mf_nks, ks_col,
+                                        ks_slot, ctx->ks_cap, ks_slot_ph);
         ctx->kf_mf = ctx->kf_mf_ok && want_mf;
         if (ctx->kf_mf_ok) {
             mf_rt = mf_tile_order(mf_tiles, MF_WAVES);
             mf_rt_small = mf_tile_order(mf_tiles, MF_WAVES_SMALL);
             ctx->mf_nrt = (int)mf_rt.size();
             ctx->mf_nrt_small = (int)mf_rt_small.size();
-            ctx->ks_nunit = (int)ks_unit.size();
             ctx->kforce_mf_lds = kforce_mf_lds_bytes(K, ctx->mf_nks, MF_WAVES);
             ctx->kforce_mf_lds_small = kforce_mf_lds_bytes(K, ctx->mf_nks, MF_WAVES_SMALL);
-            ctx->ks_ncol4 = (int)ks_col.size();
-            ctx->ksum_mf_lds = ksum_mf_lds_bytes(K, ctx->AC, ctx->ks_ncol4, ctx->ks_nunit);
+            ctx->ks_nslot = (int)ks_slot.size();
+            ctx->ks_nslot_ph = (int)ks_slot_ph.size();
+            ctx->phase_lds = std::max(std::max(sizeof(RsLds<4>), sizeof(NlLds)),
+                                      ksum_mf_lds_bytes(K, PH_SUB));
+            ctx->ksum_mf_lds = ksum_mf_lds_bytes(K, ctx->AC);
         }
         if (ctx->kf_mf) ctx->kf_split = false;
     }
@@ -186,7 +188,11 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
         const bool hi = ctx->mf_nks > MF_KS_LO;
         bool ok = ctx->ksum_mf_lds <= 160 * 1024 && ctx->kforce_mf_lds <= 160 * 1024;
         if (ok && ctx->ksum_mf_lds > 64 * 1024)
-            ok = hipFuncSetAttribute((const void *)k_ksum_mf,
+            ok = hipFuncSetAttribute(ctx->ks_cap == 1   ? (const void *)k_ksum_mf<1>
+                                     : ctx->ks_cap == 2 ? (const void *)k_ksum_mf<2>
+                                     : ctx->ks_cap == 3 ? (const void *)k_ksum_mf<3>
+                                     : ctx->ks_cap == 4 ? (const void *)k_ksum_mf<4>
+                                                        : (const void *)k_ksum_mf<KS_ACC>,
                                      hipFuncAttributeMaxDynamicSharedMemorySize,
                                      (int)ctx->ksum_mf_lds) == hipSuccess;
         if (ok && ctx->kforce_mf_lds > 64 * 1024)
@@ -229,7 +235,8 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
                         (st = dalloc(ctx, &ctx->mf_rt, ctx->mf_nrt)) ||
                         (st = dalloc(ctx, &ctx->mf_rt_small, ctx->mf_nrt_small)) ||
                         (st = dalloc(ctx, &ctx->ks_col, ks_col.size())) ||
-                        (st = dalloc(ctx, &ctx->ks_unit, ks_unit.size())))) ||
+                        (st = dalloc(ctx, &ctx->ks_slot, ks_slot.size())) ||
+                        (st = dalloc(ctx, &ctx->ks_slot_ph, ks_slot_ph.size())))) ||
         (st = alloc_all(ctx)))
         return st;
     if (ctx->kf_mf_ok &&
@@ -238,7 +245,9 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
          hipMemcpy(ctx->mf_rt_small, mf_rt_small.data(), mf_rt_small.size() * sizeof(int4),
                    hipMemcpyHostToDevice) ||
          hipMemcpy(ctx->ks_col, ks_col.data(), ks_col.size() * sizeof(int4), hipMemcpyHostToDevice) ||
-         hipMemcpy(ctx->ks_unit, ks_unit.data(), ks_unit.size() * sizeof(int2), hipMemcpyHostToDevice))) {
+         hipMemcpy(ctx->ks_slot, ks_slot.data(), ks_slot.size() * sizeof(int4), hipMemcpyHostToDevice) ||
+         hipMemcpy(ctx->ks_slot_ph, ks_slot_ph.data(), ks_slot_ph.size() * sizeof(int4),
+                   hipMemcpyHostToDevice))) {
         ctx->err = "constant upload failed";
         return QTP_ERR_HIP;
     }
@@ -263,7 +272,7 @@ void qtp_destroy(qtp_ctx *ctx)
     void *ptrs[] = {ctx->q, ctx->p, ctx->F, ctx->fph, ctx->disp, ctx->m_atom, ctx->sqm_atom,
                     ctx->charge, ctx->point, ctx->list, ctx->fpoint, ctx->flist, ctx->cnt,
                     ctx->flag, ctx->status, ctx->nreb, ctx->qpm, ctx->vpart, ctx->vout, ctx->rpart, ctx->rs_sites, ctx->rs_box, ctx->rs_far, ctx->nl_bm, ctx->cell_of, ctx->crank, ctx->cstart, ctx->member, ctx->cell_pos,
-                    ctx->spart, ctx->sprime, ctx->flj, ctx->fspl, ctx->spl_coef, ctx->fpm, ctx->fk2, ctx->wm, ctx->gcol, ctx->mf_rt, ctx->mf_rt_small, ctx->ks_col, ctx->ks_unit, ctx->Ve, ctx->epart,
+                    ctx->spart, ctx->sprime, ctx->flj, ctx->fspl, ctx->spl_coef, ctx->fpm, ctx->fk2, ctx->wm, ctx->gcol, ctx->mf_rt, ctx->mf_rt_small, ctx->ks_col, ctx->ks_slot, ctx->ks_slot_ph, ctx->Ve, ctx->epart,
                     ctx->scal, ctx->out, ctx->heat, ctx->heat_step, ctx->step_ctr, ctx->groups,
                     ctx->gcf, ctx->grk, ctx->tiles, ctx->Cm, ctx->mode, ctx->nq, ctx->np,
                     ctx->ppart, ctx->hpart, ctx->dev, ctx->obs, ctx->obs_out, ctx->ntrace, ctx->trace,

@@ -75,7 +75,8 @@ struct qtp_ctx {
     // 1 always, 0 never (k_prop_fwd + k_prop_inv)
     int prop_fused = -1;
     int ep_cap = 0;   // allocated stride of the energy partials
-    int mf_Mp = 0, mf_nks = 0, mf_nrt = 0, mf_nrt_small = 0, ks_nunit = 0, ks_ncol4 = 0;
+    int mf_Mp = 0, mf_nks = 0, mf_nrt = 0, mf_nrt_small = 0, ks_nslot = 0, ks_cap = 6, ks_nslot_ph = 0;
+    size_t phase_lds = 0;  // k_phase_pairs
     size_t kforce_mf_lds = 0, kforce_mf_lds_small = 0, ksum_mf_lds = 0;
 
     // device state (planar SoA)
@@ -104,7 +105,8 @@ struct qtp_ctx {
     int4 *mf_rt = nullptr;  // k_kforce_mf row-tile table (MF_WAVES waves)
     int4 *mf_rt_small = nullptr;  // and for MF_WAVES_SMALL
     int4 *ks_col = nullptr; // k_ksum_mf column table
-    int2 *ks_unit = nullptr;
+    int4 *ks_slot = nullptr;  // and its slot groups
+    int4 *ks_slot_ph = nullptr;  // slot groups of k_phase_pairs
     double *scal = nullptr, *out = nullptr, *heat = nullptr, *heat_step = nullptr;
     unsigned long long *step_ctr = nullptr;
     // constants

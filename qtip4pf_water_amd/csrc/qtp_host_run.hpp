@@ -8,14 +8,13 @@
 // force phase: E single-bead evaluations (forces.cpp:468-630)
 // ---------------------------------------------------------------------------
 // Launch shape of k_ksum_mf for E evaluations: blocks per chunk group (a
-// multiple of the count that keeps KS_MAXU units per wave; more when the
-// launch has few blocks, or as tuned), chunks per block (as tuned, else the
-// most of 1, 2, 4, 8 that still leaves 2048 blocks), chunk groups.
+// multiple of the count that gives each wave at most one slot group, more when
+// the launch has few blocks, or as tuned), chunks per block (as tuned, else
+// the most of 1, 2, 4, 8 that still leaves 2048 blocks), chunk groups.
 static void ksum_mf_shape(const qtp_ctx *ctx, int E, int *usplit, int *cpb, int *ncg)
 {
-    const int per = KS_MAXU * KS_WAVES;
-    const int req = std::max(1, (ctx->ks_nunit + per - 1) / per);
-    const int umax = std::min(4, std::max(1, ctx->ks_nunit / (req * KS_WAVES)));
+    const int req = std::max(1, (ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES);
+    const int umax = std::min(4, std::max(1, ctx->ks_nslot / req));
     const int mult = ctx->ks_usplit > 0 ? std::min(ctx->ks_usplit, umax)
                                         : ((long)E * ctx->nac * req < 128 ? umax : 1);
     *usplit = req * mult;
@@ -45,6 +44,153 @@ struct SplineScope {
 };
 
 
+// What every real-space tile of a launch at `pos` shares.
+static RsArgs rs_args(const qtp_ctx *ctx, const double *pos, double *vp)
+{
+    RsArgs a{};
+    a.pos = pos;
+    a.pstride = 3L * ctx->NAP;
+    a.charge = ctx->charge;
+    a.n_atoms = ctx->n_atoms;
+    a.NAP = ctx->NAP;
+    a.nblk = ctx->nblk;
+    a.gamma = ctx->ff.gamma_vs;
+    a.half1mg = ctx->ff.half1mg;
+    a.tiles = ctx->tiles;
+    a.ntile = a.nt = ctx->ntile;
+    a.box = ctx->box;
+    a.ew = ctx->ew;
+    a.rpart = ctx->rpart;
+    a.epart = ctx->epart;
+    a.ep_stride = ctx->ep_stride;
+    a.ep_off = ctx->ep_real;
+    a.vpart = vp;
+    a.cf = rs_coef();
+    a.sites = ctx->rs_sites;
+    a.bbox = ctx->rs_box;
+    a.rfar = ctx->rs_far;
+    a.fx = rs_fix(ctx->box, std::sqrt(ctx->ew.rcut_sq));
+    return a;
+}
+
+static KsArgs ks_args(const qtp_ctx *ctx, const double *pos, int sub, int gsites, int ncg, int usplit)
+{
+    KsArgs a{};
+    a.pos = pos;
+    a.pstride = 3L * ctx->NAP;
+    a.charge = ctx->charge;
+    a.n_atoms = ctx->n_atoms;
+    a.NAP = ctx->NAP;
+    a.gamma = ctx->ff.gamma_vs;
+    a.half1mg = ctx->ff.half1mg;
+    a.ew = ctx->ew;
+    a.kcol = ctx->ks_col;
+    a.kslot = ctx->ks_slot;
+    a.nslot = ctx->ks_nslot;
+    a.G = ctx->G;
+    a.sub = sub;
+    a.gsites = gsites;
+    a.ncg = ncg;
+    a.usplit = usplit;
+    a.spart = ctx->spart;
+    return a;
+}
+
+static SrArgs sr_args(const qtp_ctx *ctx, int nparts, double *vp)
+{
+    SrArgs a{};
+    a.spart = ctx->spart;
+    a.nac = nparts;
+    a.G = ctx->G;
+    a.groups = ctx->groups;
+    a.gcf = ctx->gcf;
+    a.sprime = ctx->sprime;
+    a.epart = ctx->epart;
+    a.ep_stride = ctx->ep_stride;
+    a.ep_off = ctx->ep_k;
+    a.grk = ctx->grk;
+    a.q4 = 0.25 / ctx->ew.kappa2;
+    a.vpart = vp;
+    a.wm = ctx->kf_mf ? ctx->wm : nullptr;
+    a.Mp = ctx->mf_Mp;
+    a.NN = 4 * ctx->mf_nks;
+    a.gcol = ctx->gcol;
+    a.bkz = ctx->ew.bk[2];
+    a.pform = ctx->kf_mf ? 1 : 0;
+    return a;
+}
+
+static LjArgs lj_args(const qtp_ctx *ctx, const double *pos, int lmode, int lbase, double *vp)
+{
+    LjArgs a{};
+    a.pos = pos;
+    a.pstride = 3L * ctx->NAP;
+    a.n_mols = ctx->n_mols;
+    a.NAP = ctx->NAP;
+    a.fpoint = ctx->fpoint;
+    a.flist = ctx->flist;
+    a.fcap = ctx->fcap;
+    a.lmode = lmode;
+    a.lbase = lbase;
+    a.box = ctx->box;
+    a.ff = ctx->ff;
+    a.flj = ctx->flj;
+    a.epart = ctx->epart;
+    a.ep_stride = ctx->ep_stride;
+    a.ep_off = ctx->ep_lj;
+    a.vpart = vp;
+    return a;
+}
+
+static HeatArgs heat_args(const qtp_ctx *ctx, bool with_heat)
+{
+    HeatArgs h{};
+    if (with_heat) {
+        h.part = ctx->ppart;
+        h.hpart = ctx->hpart;
+        h.heat_acc = ctx->heat;
+        h.heat_step = ctx->heat_step;
+        h.ntile = ctx->ptile;
+        h.nh = ctx->P * ctx->ptile;
+    }
+    return h;
+}
+
+static NlArgs nlist_args(const qtp_ctx *ctx, int force_all, bool with_heat, const unsigned long long *ctr)
+{
+    NlArgs a{};
+    a.n_mols = ctx->n_mols;
+    a.NAP = ctx->NAP;
+    a.NMP = ctx->NMP;
+    a.q = ctx->q;
+    a.box = ctx->box;
+    a.r_skin_sq = ctx->ff.r_skin_sq;
+    a.skin = ctx->drv.r_skin - ctx->drv.lj_rcut;
+    a.force_all = force_all;
+    a.every = ctr ? ctx->rebuild_every : 0;
+    a.step_ctr = ctr;
+    a.list_size = ctx->list_size;
+    a.fcap = ctx->fcap;
+    a.disp = ctx->disp;
+    a.flag = ctx->flag;
+    a.nreb = ctx->nreb;
+    a.point = ctx->point;
+    a.fpoint = ctx->fpoint;
+    a.list = ctx->list;
+    a.flist = ctx->flist;
+    a.status = ctx->status;
+    a.heat = heat_args(ctx, with_heat);
+    return a;
+}
+
+// Whether a phase takes the one-stream form (k_phase_pairs,
+// k_phase_reduce): the default launch choices without tile culling or splines.
+static bool phase_fused(const qtp_ctx *ctx)
+{
+    return !ctx->timing && ctx->kf_mf && !ctx->rs_cull && !ctx->spl_on && ctx->rs_split == 0 &&
+           ctx->rs_waves == 4 && ctx->rs_carg != 0 && ctx->ks_usplit == 0 && ctx->ks_cpb == 0;
+}
+
 // vout (optional): per-evaluation virial W_ab = sum_i r_i (x) F_i in the
 // minimum-image pair form (6 components xx yy zz xy xz yz), at fixed Ewald
 // parameters.
@@ -62,7 +208,8 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     // before kforce, with a share of the real-space tiles after them.  With
     // per-kernel timing on, everything stays on one stream so each launch is
     // timed alone.
-    const bool fork = !ctx->timing;
+    const bool fused = phase_fused(ctx);
+    const bool fork = !ctx->timing && !fused;
     hipStream_t sk = fork ? ctx->s2 : s;
     // real-space tiles: the first nt_a on this stream, the other nt_b (a
     // tunable share, in eighths) on the second stream after the LJ kernel,
@@ -75,14 +222,12 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     // lost more than the launch gained)
     const bool carg = ctx->rs_carg >= 0 ? ctx->rs_carg == 1
                                         : (long)E * ctx->ntile >= RS_CARG_BLOCKS;
-    const RsCoef cf = rs_coef();
+    RsArgs ra = rs_args(ctx, pos, vp);
     auto launch_rs = [&](hipStream_t st, int t0, int nt) {
         TimeScope ts(ctx, "realspace");
-#define QTP_RS_LAUNCH_W(VIR, CARG, CULL, W)                                                        \
-    k_realspace<VIR, CARG, CULL, W><<<E * nt, 64 * W, 0, st>>>(                                    \
-        pos, N3, ctx->charge, ctx->n_atoms, ctx->NAP, ctx->nblk, g, h, ctx->tiles, ctx->ntile,     \
-        t0, nt, ctx->box, ctx->ew, ctx->rpart, ctx->epart, ctx->ep_stride, ctx->ep_real, vp, cf, \
-        ctx->rs_sites, ctx->rs_box, ctx->rs_far)
+        ra.t0 = t0;
+        ra.nt = nt;
+#define QTP_RS_LAUNCH_W(VIR, CARG, CULL, W) k_realspace<VIR, CARG, CULL, W><<<E * nt, 64 * W, 0, st>>>(ra)
 #define QTP_RS_LAUNCH(VIR, CARG, CULL)                                                             \
     do {                                                                                           \
         if (ctx->rs_waves == 2) QTP_RS_LAUNCH_W(VIR, CARG, CULL, 2);                              \
@@ -116,6 +261,45 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
             ctx->tiles, ctx->ntile, ctx->nblk, E, ctx->rs_box, ctx->box, ctx->ew, ctx->rs_far,
             ctx->epart, ctx->ep_stride, ctx->ep_real, vp);
     }
+    if (fused) {
+        int usplit, cpb, ncg;
+        ksum_mf_shape(ctx, E, &usplit, &cpb, &ncg);
+        usplit = (ctx->ks_nslot_ph + 3) / 4;
+        KsArgs ka = ks_args(ctx, pos, PH_SUB, cpb * ctx->AC, ncg, usplit);
+        ka.kslot = ctx->ks_slot_ph;
+        ka.nslot = ctx->ks_nslot_ph;
+        // a list check deferred by the step: only the LJ blocks read the lists
+        NlArgs na{};
+        int n_nl = 0;
+        if (ctx->lists_defer) {
+            ctx->lists_defer = false;
+            na = nlist_args(ctx, 0, ctx->lists_heat, ctx->lists_ctr);
+            na.keep_disp = 1;
+            n_nl = ctx->P + (ctx->lists_heat ? 1 : 0);
+        }
+        const int n_ks = E * ncg * usplit, n_rs = E * ctx->ntile, n_lj = E * ctx->nmb;
+        const bool early = n_lj <= PH_LJ_EARLY;
+        const int n_lj1 = early ? n_lj : 0;
+        const int n_lj2 = early && n_nl == 0 ? 0 : n_lj;
+        const int grid_a = n_nl + n_ks + n_lj1 + n_rs;
+        const SrArgs sa = sr_args(ctx, ncg, vp);
+        const LjArgs la = lj_args(ctx, pos, lmode, lbase, vp);
+#define QTP_PHASE(VIR, LPM)                                                                    \
+    do {                                                                                       \
+        k_phase_pairs<VIR, LPM><<<grid_a, 256, ctx->phase_lds, s>>>(ra, ka, la, na, n_nl, n_ks,  \
+                                                                    n_lj1, n_rs);              \
+        k_phase_reduce<VIR, LPM><<<n_lj2 + E * ctx->ngr, 256, 0, s>>>(sa, la, na, n_nl, n_lj2, \
+                                                                      early);                  \
+    } while (0)
+        if (ctx->lj_lpm == 64) {
+            if (vout) QTP_PHASE(true, 64);
+            else QTP_PHASE(false, 64);
+        } else {
+            if (vout) QTP_PHASE(true, 16);
+            else QTP_PHASE(false, 16);
+        }
+#undef QTP_PHASE
+    } else {
     if (fork) {
         HIPCHK(hipEventRecord(ctx->ev_fork, s));
         HIPCHK(hipStreamWaitEvent(sk, ctx->ev_fork, 0));
@@ -125,10 +309,16 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
         if (ctx->kf_mf) {
             int usplit, cpb, ncg;
             ksum_mf_shape(ctx, E, &usplit, &cpb, &ncg);
-            k_ksum_mf<<<E * ncg * usplit, 64 * KS_WAVES, ctx->ksum_mf_lds, sk>>>(
-                pos, N3, ctx->charge, ctx->n_atoms, ctx->NAP, g, h, ctx->ew, ctx->ks_col,
-                ctx->ks_ncol4, ctx->ks_unit, ctx->ks_nunit, ctx->G, ctx->AC, ctx->nac, cpb, usplit,
-                ctx->spart);
+            const KsArgs ka = ks_args(ctx, pos, ctx->AC, cpb * ctx->AC, ncg, usplit);
+#define QTP_KS_MF(CAP) k_ksum_mf<CAP><<<E * ncg * usplit, 64 * KS_WAVES, ctx->ksum_mf_lds, sk>>>(ka)
+            switch (ctx->ks_cap) {
+            case 1: QTP_KS_MF(1); break;
+            case 2: QTP_KS_MF(2); break;
+            case 3: QTP_KS_MF(3); break;
+            case 4: QTP_KS_MF(4); break;
+            default: QTP_KS_MF(KS_ACC); break;
+            }
+#undef QTP_KS_MF
         } else
             k_ksum<<<E * ctx->ngc * ctx->nac, 256, ctx->ksum_lds, sk>>>(
                 pos, N3, ctx->charge, ctx->n_atoms, ctx->NAP, g, h, ctx->ew, ctx->groups, ctx->G,
@@ -142,12 +332,7 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
             int usplit, cpb;
             ksum_mf_shape(ctx, E, &usplit, &cpb, &nparts);
         }
-        k_sreduce<<<E * ctx->ngr, 256, 0, sk>>>(ctx->spart, nparts, ctx->G, ctx->groups, ctx->gcf,
-                                                 ctx->sprime, ctx->epart, ctx->ep_stride, ctx->ep_k,
-                                                 ctx->grk, 0.25 / ctx->ew.kappa2, vp,
-                                                 ctx->kf_mf ? ctx->wm : nullptr,
-                                                 ctx->mf_Mp, 4 * ctx->mf_nks, ctx->gcol,
-                                                 ctx->ew.bk[2], ctx->kf_mf ? 1 : 0);
+        k_sreduce<<<E * ctx->ngr, 256, 0, sk>>>(sr_args(ctx, nparts, vp));
     }
     // a list check deferred by the step (only the LJ kernel reads the lists)
     if (ctx->lists_defer) {
@@ -156,11 +341,8 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     }
     {
         TimeScope ts(ctx, "ljintra");
-#define QTP_LJ_LAUNCH(VIR, LPM)                                                                    \
-    k_ljintra<VIR, LPM><<<E * ctx->nmb, 256, 0, sk>>>(pos, N3, ctx->n_mols, ctx->NAP, ctx->fpoint, \
-                                                      ctx->flist, ctx->fcap, lmode, lbase,         \
-                                                      ctx->box, ctx->ff, ctx->flj, ctx->epart,     \
-                                                      ctx->ep_stride, ctx->ep_lj, vp)
+        const LjArgs la = lj_args(ctx, pos, lmode, lbase, vp);
+#define QTP_LJ_LAUNCH(VIR, LPM) k_ljintra<VIR, LPM><<<E * ctx->nmb, 256, 0, sk>>>(la)
         if (ctx->lj_lpm == 64) {
             if (vout) QTP_LJ_LAUNCH(true, 64);
             else QTP_LJ_LAUNCH(false, 64);
@@ -185,6 +367,7 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     if (fork) HIPCHK(hipEventRecord(ctx->ev_join, sk));
     launch_rs(s, 0, nt_a);
     if (fork) HIPCHK(hipStreamWaitEvent(s, ctx->ev_join, 0));
+    }
     {
         TimeScope ts(ctx, "kforce");
         // tiles the CULL form skipped: their (zero) slots are not read
@@ -313,23 +496,11 @@ static int run_lists(qtp_ctx *ctx, int force_all, bool with_heat, const unsigned
     const int every = ctr ? ctx->rebuild_every : 0;
     hipStream_t s = st ? st : ctx->stream;
     const int P = ctx->P;
-    HeatArgs heat{};
-    if (with_heat) {
-        heat.part = ctx->ppart;
-        heat.hpart = ctx->hpart;
-        heat.heat_acc = ctx->heat;
-        heat.heat_step = ctx->heat_step;
-        heat.ntile = ctx->ptile;
-        heat.nh = ctx->P * ctx->ptile;
-    }
+    const HeatArgs heat = heat_args(ctx, with_heat);
     const bool cells = use_cells(ctx);
     if (ctx->n_mols <= NL_FUSED_MAXMOL && !cells) {
         TimeScope ts(ctx, "nlist");
-        k_nlist_bead<<<P + (with_heat ? 1 : 0), 1024, 0, s>>>(ctx->n_mols, ctx->NAP, ctx->NMP, ctx->q, ctx->box,
-                                        ctx->ff.r_skin_sq, ctx->drv.r_skin - ctx->drv.lj_rcut, force_all,
-                                        every, ctr, ctx->list_size, ctx->fcap, ctx->disp, ctx->flag, ctx->nreb,
-                                        ctx->point, ctx->fpoint, ctx->list, ctx->flist,
-                                        ctx->status, heat);
+        k_nlist_bead<<<P + (with_heat ? 1 : 0), 1024, 0, s>>>(nlist_args(ctx, force_all, with_heat, ctr));
         HIPCHK(hipGetLastError());
         return QTP_OK;
     }
@@ -469,8 +640,17 @@ static int run_class_step(qtp_ctx *ctx, unsigned long long *ctr, bool resident =
         CHK(run_nn_forces(ctx, ctx->s3));
         HIPCHK(hipEventRecord(ctx->ev_nn_join, ctx->s3));
     }
-    CHK(run_lists(ctx, 0, false, resident ? ctr : nullptr));
-    CHK(run_phase(ctx, ctx->q, 1, 0, 0, ctx->fph, nullptr));
+    // the one-stream phase checks the lists in its first launch
+    if (phase_fused(ctx) && ctx->n_mols <= NL_FUSED_MAXMOL && !use_cells(ctx)) {
+        ctx->lists_defer = true;
+        ctx->lists_heat = false;
+        ctx->lists_ctr = resident ? ctr : nullptr;
+    } else {
+        CHK(run_lists(ctx, 0, false, resident ? ctr : nullptr));
+    }
+    const int st = run_phase(ctx, ctx->q, 1, 0, 0, ctx->fph, nullptr);
+    ctx->lists_defer = false;
+    CHK(st);
     if (with_nn && !nn_fork) CHK(run_nn_forces(ctx, s));
     if (nn_fork) HIPCHK(hipStreamWaitEvent(s, ctx->ev_nn_join, 0));
     {

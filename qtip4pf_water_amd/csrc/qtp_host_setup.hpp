@@ -128,11 +128,13 @@ static void build_groups(qtp_ctx *ctx, std::vector<int4> &g, std::vector<double>
 // false when a (kx, ky) pair appears in two runs or a column's kz are not
 // consecutive (then the vector kernels are used).
 // k_ksum_mf: kcol per sorted column (kx | ky << 16, first group, first kz,
-// last kz), padded to a multiple of four with empty columns; units (tile of
-// four columns, n-tile) for every n = 2 kz + 0/1 that a tile's columns reach.
+// last kz), padded to a multiple of four with empty columns; kslot: the slot
+// groups (first column tile, tiles, n-tiles N), consecutive tiles whose columns
+// reach N tiles of n = 2 kz + 0/1 (the sort keeps equal N together).
 static bool build_mf_layout(const std::vector<int4> &g, std::vector<int> &gcol,
                             std::vector<int4> &tiles, int &Mp, int &nks, std::vector<int4> &kcol,
-                            std::vector<int2> &kunit)
+                            std::vector<int4> &kslot, int &ks_cap,
+                            std::vector<int4> &kslot_ph)
 {
     struct Col {
         int kx, ky, kzmax, g0, kz0;
@@ -178,9 +180,35 @@ static bool build_mf_layout(const std::vector<int4> &g, std::vector<int> &gcol,
         const Col &c = cols[ord[i]];
         kcol[i] = make_int4(c.kx | (c.ky << 16), c.g0, c.kz0, c.kzmax);
     }
-    kunit.clear();
-    for (int t = 0; t < nq; ++t)
-        for (int u = 0; u <= (2 * kcol[4 * t].w + 1) / 16; ++u) kunit.push_back(make_int2(t, u));
+    // CAP of k_ksum_mf: the least of blocks x (factor tables + the fullest
+    // wave's products, two waves to a SIMD) per chunk; about 3000 cycles for
+    // the tables, 64 a product, 16 k-steps
+    kslot.clear();
+    auto slots = [&](int cap) {
+        std::vector<int4> v;
+        for (int t = 0; t < nq;) {
+            const int N = ((2 * kcol[4 * t].w + 1) >> 4) + 1;
+            int k = 1;
+            while (k < std::max(1, cap / N) && t + k < nq && ((2 * kcol[4 * (t + k)].w + 1) >> 4) + 1 == N) ++k;
+            v.push_back(make_int4(t, k, N, 0));
+            t += k;
+        }
+        return v;
+    };
+    kslot_ph = slots(PH_CAP);
+    double best = 0.0;
+    for (int cap : {6, 4, 3, 2, 1}) {
+        std::vector<int4> v = slots(cap);
+        const size_t blocks = (v.size() + KS_WAVES - 1) / KS_WAVES;
+        int most = 0;
+        for (const int4 &u : v) most = std::max(most, std::max(1, cap / u.z) * u.z);
+        const double cost = (double)blocks * (3000.0 + 2.0 * 64.0 * 16.0 * most);
+        if (kslot.empty() || cost < best) {
+            best = cost;
+            ks_cap = cap;
+            kslot = v;
+        }
+    }
     return true;
 }
 

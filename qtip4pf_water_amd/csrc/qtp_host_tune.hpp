@@ -148,7 +148,7 @@ int tune_time(qtp_ctx *ctx, int n, float *ms)
 std::vector<TuneCfg> tune_candidates(const qtp_ctx *ctx)
 {
     std::vector<TuneCfg> out;
-    const int umax = std::min(4, std::max(1, ctx->ks_nunit / KS_WAVES));
+    const int umax = std::min(4, std::max(1, ctx->ks_nslot / ((ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES)));
     for (int rsw : {4, 2})
         for (int lpm : {16, 64})
             for (int kmf = ctx->kf_mf_ok ? 1 : 0; kmf >= 0; --kmf)

@@ -27,6 +27,66 @@ __device__ __forceinline__ void kw_table(double2 *row, double r, double bk, doub
     }
 }
 
+// sin and cos of x for the factor tables: x = n pi/2 + r with pi/2 in three
+// parts (each fma rounds once, to the size of the small difference, so r is as
+// accurate as x for every n that a double holds exactly), then the Taylor series of sin and
+// cos to degrees 17 and 18 on |r| <= pi/4 (truncation below 1e-17).  About 40
+// vector instructions; the library's reduction for any size of x takes more
+// than twice that.
+__constant__ double SINCOS_COEF[20] = {
+    0.6366197723675814,                                               // 2 / pi
+    1.5707963267341256, 6.077100506303966e-11, 2.0222662487959506e-21,  // pi / 2
+    1.0 / 355687428096000.0, -1.0 / 1307674368000.0, 1.0 / 6227020800.0, -1.0 / 39916800.0,
+    1.0 / 362880.0, -1.0 / 5040.0, 1.0 / 120.0, -1.0 / 6.0,           // sin: 1/17! ... -1/3!
+    -1.0 / 6402373705728000.0, 1.0 / 20922789888000.0, -1.0 / 87178291200.0, 1.0 / 479001600.0,
+    -1.0 / 3628800.0, 1.0 / 40320.0, -1.0 / 720.0, 1.0 / 24.0};       // cos: -1/18! ... 1/4!
+__device__ __forceinline__ void sincos_table(double x, double &sn, double &cs)
+{
+    // the coefficients by scalar loads at an offset the compiler cannot see
+    // through: kept out of registers across the caller's loop (as literals they
+    // were held there, and k_ksum_mf spilled a hundred registers)
+    int o = 0;
+    asm volatile("" : "+s"(o));
+    const double *C = SINCOS_COEF + o;
+    const double n = rint(x * C[0]);
+    double r = fma(-n, C[1], x);
+    r = fma(-n, C[2], r);
+    r = fma(-n, C[3], r);
+    // beyond 2^53 quarter turns x says nothing about its phase: 0, so that the
+    // factors stay on the unit circle (inf and NaN give NaN)
+    if (!(fabs(r) <= 1.0)) r -= r;
+    const double z = r * r;
+    double s = C[4], c = C[12];
+#pragma unroll
+    for (int k = 1; k < 8; ++k) {
+        s = fma(s, z, C[4 + k]);
+        c = fma(c, z, C[12 + k]);
+    }
+    s = fma(s * z, r, r);
+    c = fma(fma(c, z, -0.5), z, 1.0);
+    const int q = (int)fma(-4.0, floor(0.25 * n), n);  // n mod 4, exact for any n
+    const double a = (q & 1) ? c : s, b = (q & 1) ? s : c;
+    sn = (q & 2) ? -a : a;
+    cs = ((q + 1) & 2) ? -b : b;
+}
+
+// One site's factors e^{i m b r} q, m = 0 .. K-1, by the recurrence of
+// forces.cpp:212-245 (q: the charge in the x table, 1 in the others, 0 for a
+// site that does not exist): put(m, Re, Im).
+template <class Put>
+__device__ __forceinline__ void mf_factors(double br, double q, int K, Put put)
+{
+    double sn, cs;
+    sincos_table(br, sn, cs);
+    double cm = q, sm = 0.0;
+    for (int m = 0; m < K; ++m) {
+        put(m, cm, sm);
+        const double c = fma(cs, cm, -(sn * sm));
+        sm = fma(cs, sm, sn * cm);
+        cm = c;
+    }
+}
+
 constexpr int KF_REC = 9;   // doubles per k-group record read by k_kforce
 
 // Reciprocal-space structure factors (kwald, forces.cpp:180-448), partial
@@ -90,58 +150,125 @@ __global__ __launch_bounds__(256) void k_ksum(const double *__restrict__ pos, lo
 //   at site j,  Zt[2 kz], Zt[2 kz + 1] = Re, Im Z(kz)
 // form one matrix product over the sites; k_sreduce combines them into the
 // eight sums of each group (A = X Y, B = X Y*: Ar = F0 - F1, Ai = F2 + F3,
-// Br = F0 + F1, Bi = F3 - F2).  A unit = 16 rows (four columns in
-// k_kforce_mf's sorted order) x 16 values of n (n-tile 0 or 1); each lane
-// forms its A operand F_p with one product of two table entries.
-// A block takes cpb consecutive chunks (a chunk group) and a slice of the
-// units: it builds each chunk's factor tables in turn and keeps its units'
-// accumulators in registers across the chunks (at most KS_MAXU units per
-// wave), so one partial per group and chunk group is written: cpb times
-// fewer partials to write here and to read in k_sreduce.
+// Br = F0 + F1, Bi = F3 - F2).  A column tile = 16 rows (four columns in
+// k_kforce_mf's sorted order) x N 16-wide tiles of n, the ones its columns
+// reach (1 to 3); each lane forms its A operand F_p with one product of two
+// table entries.  A wave takes a slot group: up to max(1, CAP / N) column tiles
+// of the same N, at most max(CAP, 3) accumulators.  Per k-step of four sites it
+// reads each tile's two A factors and the N B operands once for its products:
+// 7, 8 or 13 LDS reads for six products at N = 3, 2, 1.  (One accumulator at a time took 18 and was
+// bound by the LDS: 4096 H2O x 32 beads, |n| <= 18, 697 -> 628 us.)
+// A block takes cpb consecutive chunks (a chunk group) and KS_WAVES slot
+// groups: it builds each chunk's factor tables in turn and keeps the
+// accumulators in registers across the chunks, so one partial per group and
+// chunk group is written: cpb times fewer partials to write here and to read
+// in k_sreduce.
 // Output per group and chunk group: Re/Im Z times F0..F3, in that order.
 // kcol[c] = (kx | ky << 16, first group, first kz, last kz) per sorted
-// column (padding columns: first kz > last kz).  usplit blocks share a chunk
-// group, each taking 1/usplit of the units (the host makes the slices fit
-// KS_MAXU units per wave).
+// column (padding columns: first kz > last kz); kslot[i] = (first column tile,
+// tiles, N) of slot group i.  usplit blocks share a chunk group, each taking
+// 1/usplit of the slot groups (at most KS_WAVES).
 // grid: E * ncg * usplit (ncg = ceil(nac / cpb)), 64 * KS_WAVES threads,
-// ksum_mf_lds_bytes(K, AC, ncol4, nunit).
+// ksum_mf_lds_bytes(K, AC).
 constexpr int KS_WAVES = 8;
-constexpr int KS_MAXU = 6;  // units per wave of one block (accumulator registers)
+constexpr int KS_ACC = 6;  // largest CAP (1, 2, 3, 4 or 6)
 // LDS rows of AC + 2 entries: the B operands of a quarter-wave (16 rows n at
 // one site) and the A factors of a tile's columns then fall in different banks.
-// The column and unit tables are staged in LDS behind the factor tables.
 // z-factor rows of k_ksum_mf: 2 K entries padded to whole 16-row n tiles
 // (at least two)
 __host__ __device__ inline int ksum_mf_zrows(int K) { return 2 * K <= 32 ? 32 : ((2 * K + 15) / 16) * 16; }
-inline size_t ksum_mf_lds_bytes(int K, int AC, int ncol4, int nunit)
+inline size_t ksum_mf_lds_bytes(int K, int AC)
 {
-    return ((size_t)4 * K + ksum_mf_zrows(K)) * (AC + 2) * 8 + (size_t)ncol4 * 16 +
-           (size_t)nunit * 8;
+    return ((size_t)4 * K + ksum_mf_zrows(K)) * (AC + 2) * 8;
 }
 
-__global__ __launch_bounds__(64 * KS_WAVES) void k_ksum_mf(
-    const double *__restrict__ pos, long pstride, const double *__restrict__ charge, int n_atoms,
-    int NAP, double gamma, double half1mg, Ewald ew, const int4 *__restrict__ kcol, int ncol4,
-    const int2 *__restrict__ kunit, int nunit, int G, int AC, int nac, int cpb, int usplit,
-    double *__restrict__ spart)
+// The wave's slot group over the staged sites: T column tiles of N n-tiles.
+template <int N, int T>
+__device__ __forceinline__ void ks_slots(const double *Td, const double *Zr, const int *ox, const int *oy,
+                                         int zstep, int AC, mf_v4d *acc)
 {
-    extern __shared__ double smem[];
+    const double *px[T], *py[T], *pz[N];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        px[t] = Td + ox[t];
+        py[t] = Td + oy[t];
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) pz[n] = Zr + n * zstep;
+    // two k-steps of loads in flight where the registers allow it (a loop of
+    // N = 3, T = 2 alone: 61.8 TFLOP/s with one, 70.5 with two)
+    constexpr int U = 2 * T + N > 8 ? 1 : 2;
+#pragma unroll U
+    for (int s4 = 0; s4 < AC; s4 += 4) {
+        double b[N], a[T];
+#pragma unroll
+        for (int n = 0; n < N; ++n) b[n] = pz[n][s4];
+#pragma unroll
+        for (int t = 0; t < T; ++t) a[t] = px[t][2 * s4] * py[t][2 * s4];
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+            for (int n = 0; n < N; ++n)
+                acc[t * N + n] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[t], b[n], acc[t * N + n], 0, 0, 0);
+    }
+}
+// The slot group's partials: lane n = 16 n-tile + j16, product gq, column
+// 4 tile + reg.
+template <int N, int T>
+__device__ __forceinline__ void ks_write(const int4 *__restrict__ kcol, int t0, int j16, int gq,
+                                         int nt, const mf_v4d *acc, double *__restrict__ out)
+{
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        if (t >= nt) break;
+#pragma unroll
+        for (int reg = 0; reg < 4; ++reg) {
+            const int4 cr = kcol[4 * (t0 + t) + reg];
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                const int kz = (16 * n + j16) >> 1;
+                if (kz >= cr.z && kz <= cr.w)
+                    out[(long)(cr.y + kz - cr.z) * 8 + gq * 2 + (j16 & 1)] = acc[t * N + n][reg];
+            }
+        }
+    }
+}
+struct KsArgs {
+    const double *pos;
+    long pstride;
+    const double *charge;
+    int n_atoms, NAP;
+    double gamma, half1mg;
+    Ewald ew;
+    const int4 *kcol, *kslot;
+    int nslot, G;
+    int sub;                  // sites staged at a time (a multiple of 4)
+    int gsites, ncg, usplit;  // sites per chunk group (a multiple of 4), groups, blocks per group
+    double *spart;
+};
+
+// Block `b` of a launch; its 64 WAVES threads, ksum_mf_lds_bytes(K, sub) of LDS
+// at smem.  The k-steps of a chunk group run over its sites in order whatever
+// `sub` is, so the partials do not depend on it.
+template <int CAP, int WAVES>
+__device__ __forceinline__ void ks_block(double *smem, int b, const KsArgs &A)
+{
+    const int n_atoms = A.n_atoms, NAP = A.NAP, nslot = A.nslot, G = A.G, SC = A.sub;
+    const int usplit = A.usplit;
+    const double gamma = A.gamma, half1mg = A.half1mg;
+    const Ewald &ew = A.ew;
+    const double *__restrict__ charge = A.charge;
+    const int4 *__restrict__ kcol = A.kcol;
     const int K = ew.K;
-    const int RS = AC + 2;           // LDS row stride
+    const int RS = SC + 2;           // LDS row stride
     const int ZN = ksum_mf_zrows(K);
-    double2 *T = (double2 *)smem;    // [2][K][RS] x (charge folded), y factors
+    // smem: [2][K][RS] (Re, Im) pairs of the x (charge folded) and y factors
     double *Zt = smem + 4 * K * RS;  // [ZN][RS]
-    int4 *sc = (int4 *)(Zt + ZN * RS);  // [ncol4] column table
-    int2 *su = (int2 *)(sc + ncol4);    // [nunit] unit table
-    const int ncg = (nac + cpb - 1) / cpb;
-    const int per_e = ncg * usplit;
-    const int e = blockIdx.x / per_e, r = blockIdx.x - e * per_e;
+    const int per_e = A.ncg * usplit;
+    const int e = b / per_e, r = b - e * per_e;
     const int cg = r / usplit, us = r - cg * usplit;
-    const int u0 = us * nunit / usplit, u1 = (us + 1) * nunit / usplit;
-    const int ac0 = cg * cpb, ac1 = min(nac, ac0 + cpb);
-    const double *X = pos + (long)e * pstride;
-    for (int t = threadIdx.x; t < ncol4; t += blockDim.x) sc[t] = kcol[t];
-    for (int t = threadIdx.x; t < nunit; t += blockDim.x) su[t] = kunit[t];
+    const int s0 = cg * A.gsites, s1 = min(s0 + A.gsites, (n_atoms + 3) & ~3);
+    const double *X = A.pos + (long)e * A.pstride;
     const int lane = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j16 = lane & 15, gq = lane >> 4;
@@ -149,74 +276,66 @@ __global__ __launch_bounds__(64 * KS_WAVES) void k_ksum_mf(
     // a = Re for p = 0, 2, b = Re for p = 0, 3 (Im otherwise)
     const int pp = lane & 3;
     const int xa = (pp == 1 || pp == 3) ? 1 : 0, yb = (pp == 1 || pp == 2) ? 1 : 0;
-    const double *Td = (const double *)T;
-    mf_v4d acc[KS_MAXU];
+    const double *Td = smem;
+    const double *Zr = Zt + j16 * RS + gq;  // site 4 s + gq, row j16 of an n-tile
+    constexpr int T1 = CAP, T2 = CAP / 2 > 0 ? CAP / 2 : 1, T3 = CAP / 3 > 0 ? CAP / 3 : 1;
+    constexpr int ACC = CAP > 3 ? CAP : 3;
+    // the wave's slot group (N = 0: none); a short one repeats its first tile
+    // in the slots it does not fill.  Read behind the first chunk's tables, so
+    // that their loads do not wait for it.
+    const int u = us * nslot / usplit + w;
+    int4 sl = make_int4(0, 0, 0, 0);
+    int N = 0, NT = 0, ox[T1], oy[T1];
+    mf_v4d acc[ACC];
 #pragma unroll
-    for (int k = 0; k < KS_MAXU; ++k) acc[k] = mf_v4d{0.0, 0.0, 0.0, 0.0};
-    for (int ac = ac0; ac < ac1; ++ac) {
-        if (ac > ac0) __syncthreads();  // the previous chunk's tables are read
-        for (int t = threadIdx.x; t < 3 * AC; t += blockDim.x) {
-            // factor tables by the recurrence of kw_table (forces.cpp:212-245)
+    for (int k = 0; k < ACC; ++k) acc[k] = mf_v4d{0.0, 0.0, 0.0, 0.0};
+    for (int sb = s0; sb < s1; sb += SC) {
+        const int AC = min(SC, s1 - sb);
+        if (sb > s0) __syncthreads();  // the previous sites' tables are read
+        for (int t = threadIdx.x; t < 3 * AC; t += 64 * WAVES) {
             const int d = t / AC, j = t - d * AC;
-            const int atom = ac * AC + j;
-            const bool va = atom < n_atoms;
-            double sn = 0.0, cs = 0.0, qf = 0.0;
-            if (va) {
+            const int atom = sb + j;
+            double br = 0.0, qf = 0.0;
+            if (atom < n_atoms) {
                 qf = d == 0 ? charge[atom] : 1.0;
-                sincos(ew.bk[d] * site_coord(X, NAP, atom, d, gamma, half1mg), &sn, &cs);
+                br = ew.bk[d] * site_coord(X, NAP, atom, d, gamma, half1mg);
             }
-            double cm = 1.0, sm = 0.0;
-            for (int m = 0; m < K; ++m) {
-                if (m > 0) {
-                    const double cn = cs * cm - sn * sm;
-                    const double snn = sn * cm + cs * sm;
-                    cm = cn;
-                    sm = snn;
-                }
-                const double c = va ? cm * qf : 0.0, s = va ? sm * qf : 0.0;
-                if (d < 2) {
-                    T[(d * K + m) * RS + j] = make_double2(c, s);
-                } else {
-                    Zt[(2 * m) * RS + j] = c;
-                    Zt[(2 * m + 1) * RS + j] = s;
-                }
-            }
+            // x, y: (Re, Im) pairs in rows of RS; z: rows of Re and of Im
+            double *row = d < 2 ? smem + 2 * (d * K * RS + j) : Zt + j;
+            const int im = d < 2 ? 1 : RS;
+            mf_factors(br, qf, K, [&](int m, double c, double s) {
+                row[2 * m * RS] = c;
+                row[2 * m * RS + im] = s;
+            });
             if (d == 2)
-                for (int n = 2 * K; n < ZN; ++n) Zt[n * RS + j] = 0.0;
+                for (int n = 2 * K; n < ZN; ++n) row[n * RS] = 0.0;
+        }
+        if (sb == s0) {
+            if (u < (us + 1) * nslot / usplit) sl = A.kslot[u];
+            N = __builtin_amdgcn_readfirstlane(sl.z), NT = __builtin_amdgcn_readfirstlane(sl.y);
+#pragma unroll
+            for (int t = 0; t < T1; ++t) {
+                const int ck = N ? kcol[4 * (sl.x + (t < NT ? t : 0)) + (j16 >> 2)].x : 0;
+                ox[t] = 2 * ((ck & 0xffff) * RS + gq) + xa;
+                oy[t] = 2 * ((K + (ck >> 16)) * RS + gq) + yb;
+            }
         }
         __syncthreads();
-#pragma unroll
-        for (int k = 0; k < KS_MAXU; ++k) {
-            const int u = u0 + w + k * KS_WAVES;
-            if (u >= u1) break;
-            const int2 un = su[u];
-            const int ck = sc[4 * un.x + (j16 >> 2)].x;
-            const int kx = ck & 0xffff, ky = ck >> 16;
-            const double *Xr = Td + 2 * (kx * RS + gq) + xa;  // site 4 s + gq
-            const double *Yr = Td + 2 * ((K + ky) * RS + gq) + yb;
-            const double *Zr = Zt + (16 * un.y + j16) * RS + gq;
-            mf_v4d a4 = acc[k];
-#pragma unroll 4
-            for (int s4 = 0; s4 < AC; s4 += 4)
-                a4 = __builtin_amdgcn_mfma_f64_16x16x4f64(Xr[2 * s4] * Yr[2 * s4], Zr[s4], a4, 0, 0, 0);
-            acc[k] = a4;
-        }
+        if (N == 3) ks_slots<3, T3>(Td, Zr, ox, oy, 16 * RS, AC, acc);
+        else if (N == 2) ks_slots<2, T2>(Td, Zr, ox, oy, 16 * RS, AC, acc);
+        else if (N == 1) ks_slots<1, T1>(Td, Zr, ox, oy, 16 * RS, AC, acc);
     }
-    double *out = spart + ((long)e * ncg + cg) * G * 8;
-#pragma unroll
-    for (int k = 0; k < KS_MAXU; ++k) {
-        const int u = u0 + w + k * KS_WAVES;
-        if (u >= u1) break;
-        const int2 un = su[u];
-        // lane: n = 16 n-tile + j16, product gq, column 4 tile + reg
-        const int n = 16 * un.y + j16, kz = n >> 1;
-#pragma unroll
-        for (int reg = 0; reg < 4; ++reg) {
-            const int4 cr = sc[4 * un.x + reg];
-            if (kz >= cr.z && kz <= cr.w)
-                out[(long)(cr.y + kz - cr.z) * 8 + gq * 2 + (n & 1)] = acc[k][reg];
-        }
-    }
+    double *out = A.spart + ((long)e * A.ncg + cg) * G * 8;
+    if (N == 3) ks_write<3, T3>(kcol, sl.x, j16, gq, NT, acc, out);
+    else if (N == 2) ks_write<2, T2>(kcol, sl.x, j16, gq, NT, acc, out);
+    else if (N == 1) ks_write<1, T1>(kcol, sl.x, j16, gq, NT, acc, out);
+}
+
+template <int CAP>
+__global__ __launch_bounds__(64 * KS_WAVES, 4) void k_ksum_mf(const KsArgs A)
+{
+    extern __shared__ double smem[];
+    ks_block<CAP, KS_WAVES>(smem, blockIdx.x, A);
 }
 
 // Sum the partial structure factors, energy per group (forces.cpp:274, 315,
@@ -236,20 +355,37 @@ __global__ __launch_bounds__(64 * KS_WAVES) void k_ksum_mf(
 // times +-kz b_z, as the v weight of the other part of the same variant pair.
 // Only these entries are ever written; the rest of W stays zero.
 constexpr int SR_GPB = 32;  // groups per block
-__global__ __launch_bounds__(256) void k_sreduce(const double *__restrict__ spart, int nac, int G,
-                                                 const int4 *__restrict__ groups,
-                                                 const double *__restrict__ gcf,
-                                                 double *__restrict__ sprime,
-                                                 double *__restrict__ epart, int ep_stride,
-                                                 int ep_off, const double4 *__restrict__ grk,
-                                                 double q4, double *__restrict__ vpart,
-                                                 double *__restrict__ wm, int Mp, int NN,
-                                                 const int *__restrict__ gcol, double bkz,
-                                                 int pform)
+struct SrArgs {
+    const double *spart;
+    int nac, G;
+    const int4 *groups;
+    const double *gcf;
+    double *sprime, *epart;
+    int ep_stride, ep_off;
+    const double4 *grk;
+    double q4;
+    double *vpart, *wm;
+    int Mp, NN;
+    const int *gcol;
+    double bkz;
+    int pform;
+};
+__device__ __forceinline__ void sreduce_block(double *sh, int block, const SrArgs &A)
 {
-    __shared__ double sh[16];
+    const double *__restrict__ spart = A.spart;
+    const int nac = A.nac, G = A.G, ep_stride = A.ep_stride, ep_off = A.ep_off, Mp = A.Mp, NN = A.NN;
+    const int pform = A.pform;
+    const int4 *__restrict__ groups = A.groups;
+    const double *__restrict__ gcf = A.gcf;
+    const double4 *__restrict__ grk = A.grk;
+    const int *__restrict__ gcol = A.gcol;
+    const double q4 = A.q4, bkz = A.bkz;
+    double *__restrict__ sprime = A.sprime;
+    double *__restrict__ epart = A.epart;
+    double *__restrict__ vpart = A.vpart;
+    double *__restrict__ wm = A.wm;
     const int nb = (G + SR_GPB - 1) / SR_GPB;
-    const int e = blockIdx.x / nb, gb = blockIdx.x - e * nb;
+    const int e = block / nb, gb = block - e * nb;
     const int g = gb * SR_GPB + (threadIdx.x >> 3);
     const int v = threadIdx.x & 7;
     const bool live = g < G;
@@ -348,6 +484,11 @@ __global__ __launch_bounds__(256) void k_sreduce(const double *__restrict__ spar
             if (threadIdx.x == 0) vpart[((long)e * 6 + c) * ep_stride + ep_off + gb] = vs;
         }
     }
+}
+__global__ __launch_bounds__(256) void k_sreduce(const SrArgs A)
+{
+    __shared__ double sh[16];
+    sreduce_block(sh, blockIdx.x, A);
 }
 
 // Reciprocal-space forces (forces.cpp:276-279, 319-324, 368-373, 434-442),

@@ -13,21 +13,51 @@ namespace qtp {
 // its energy is halved.
 // grid: E * ceil(n_mols / (256 / LPM)), 256 threads.
 constexpr int LJ_BATCH = 4;
-template <bool VIR, int LPM>
-__global__ __launch_bounds__(256) void k_ljintra(const double *__restrict__ pos, long pstride,
-                                                 int n_mols, int NAP,
-                                                 const int *__restrict__ fpoint,
-                                                 const int *__restrict__ flist, long fcap,
-                                                 int lmode, int lbase, Box box, FF ff,
-                                                 double *__restrict__ flj,
-                                                 double *__restrict__ epart, int ep_stride,
-                                                 int ep_off, double *__restrict__ vpart)
+struct LjArgs {
+    const double *pos;
+    long pstride;
+    int n_mols, NAP;
+    const int *fpoint, *flist;
+    long fcap;
+    int lmode, lbase;
+    Box box;
+    FF ff;
+    double *flj, *epart;
+    int ep_stride, ep_off;
+    double *vpart;
+};
+// The evaluation that block `block` of nblocks works on, and whether it is the
+// evaluation's first block.
+template <int LPM>
+__device__ __forceinline__ int lj_eval(int block, int nblocks, const LjArgs &A)
 {
-    __shared__ double sh[16];
+    constexpr int MPB = 256 / LPM;
+    return xcd_remap(block, nblocks) / ((A.n_mols + MPB - 1) / MPB);
+}
+template <int LPM>
+__device__ __forceinline__ bool lj_eval_first(int block, int nblocks, const LjArgs &A)
+{
+    constexpr int MPB = 256 / LPM;
+    return xcd_remap(block, nblocks) % ((A.n_mols + MPB - 1) / MPB) == 0;
+}
+template <bool VIR, int LPM>
+__device__ __forceinline__ void lj_block(double *sh, int block, int nblocks, const LjArgs &A)
+{
+    const double *__restrict__ pos = A.pos;
+    const long pstride = A.pstride, fcap = A.fcap;
+    const int n_mols = A.n_mols, NAP = A.NAP, lmode = A.lmode, lbase = A.lbase;
+    const int ep_stride = A.ep_stride, ep_off = A.ep_off;
+    const int *__restrict__ fpoint = A.fpoint;
+    const int *__restrict__ flist = A.flist;
+    const Box &box = A.box;
+    const FF &ff = A.ff;
+    double *__restrict__ flj = A.flj;
+    double *__restrict__ epart = A.epart;
+    double *__restrict__ vpart = A.vpart;
     constexpr int MPB = 256 / LPM;
     double v6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
     const int nmb = (n_mols + MPB - 1) / MPB;
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int bid = xcd_remap(block, nblocks);
     const int e = bid / nmb, mb = bid - e * nmb;
     const int gi = threadIdx.x / LPM, t = threadIdx.x % LPM;
     const int i = mb * MPB + gi;
@@ -172,6 +202,12 @@ __global__ __launch_bounds__(256) void k_ljintra(const double *__restrict__ pos,
             if (threadIdx.x == 0) vpart[((long)e * 6 + c) * ep_stride + ep_off + mb] = v;
         }
     }
+}
+template <bool VIR, int LPM>
+__global__ __launch_bounds__(256) void k_ljintra(const LjArgs A)
+{
+    __shared__ double sh[16];
+    lj_block<VIR, LPM>(sh, blockIdx.x, gridDim.x, A);
 }
 
 // Splined pair potentials of the fast-CMD path (forces.cpp:634-691,

@@ -7,11 +7,18 @@ namespace qtp {
 // rwald :141-177).  One block of W wavefronts (W = 2 or 4) per 64x64 tile
 // (I<=J) of the site pair matrix; wave w takes the 64/W j-columns
 // c0 = w 64/W ... c0 + 64/W - 1 against all 64 i.
-// Pass 1 (lane <-> i) marks each lane's in-cutoff columns (a bit mask).
-// The wave then lays its in-cutoff pairs out in an LDS queue column by
-// column (a ballot per column; within a column, rows ascending), and pass 2
-// gives every lane the same number of consecutive queue entries: lanes stay
-// busy however unevenly the pairs fall.  Consecutive entries mostly share
+// Pass 1 (lane <-> i) tests a column per turn in fixed point (RsFix: the
+// box is a power of two, so differences wrap to the minimum image by
+// themselves) with a slightly larger cutoff and appends the column's pairs to
+// an LDS queue (the comparison is the ballot; within a column, rows
+// ascending).  Pass 2 gives every lane the same number of consecutive queue
+// entries: lanes stay busy however unevenly the pairs fall.  It makes the
+// exact FP64 cutoff test; the few pairs that fail it are zeroed on a branch
+// that is seldom taken.  The kernel issues vector instructions in about two
+// thirds of its cycles and uses the LDS in more than half: the FP64 form of
+// pass 1 took a third of the instructions.  Measured alone, FP64 -> fixed
+// point: 216 H2O x 32 beads 34.9 -> 31.1 us, 512 x 32 at r_c 10.9 A 105 -> 98
+// us, 1000 x 16 at 12 A 153 -> 141 us.  Consecutive entries mostly share
 // the column j, so a lane keeps the j reaction in registers and adds it to
 // the LDS column array when j changes; i forces go to the wave's own LDS
 // rows with ds_add_f64.  Columns belong to one wave and every wave has its
@@ -59,6 +66,61 @@ __device__ __forceinline__ double periodic_gap(double a0, double a1, double b0, 
     f = fma(-L, floor(f * invL), f);
     const double back = L - f - (a1 - a0) - (b1 - b0);
     return fmax(0.0, fmin(f, back));
+}
+
+// Fixed-point coordinates of pass 1.  Cubic boxes: 16 bits per coordinate in
+// units of L / 2^16, the squared distance by two packed dot products (five
+// instructions a pair); |d| comes out at most sqrt(3) units too large, so
+// r2u is (r_c + 2 units)^2.  Other boxes: 32 bits per coordinate in units of
+// L_d / 2^32, differences converted to FP32 and scaled by w (12 instructions);
+// r2f is (r_c (1 + 1e-5))^2, the margin far above the FP32 rounding.  The FP64
+// test took 15 plus the select of a mask bit.
+struct RsFix {
+    float w[3], r2f;
+    unsigned r2u;
+    int cubic;
+};
+inline RsFix rs_fix(const Box &box, double rcut)
+{
+    RsFix f;
+    for (int d = 0; d < 3; ++d) f.w[d] = (float)(box.L[d] * (1.0 / 4294967296.0));
+    const double r = rcut * (1.0 + 1e-5);
+    f.r2f = (float)(r * r);
+    f.cubic = box.L[0] == box.L[1] && box.L[1] == box.L[2];
+    const double u = rcut / box.L[0] * 65536.0 + 2.0;
+    // only used for cubic boxes, where r_c <= L / 2: below 2^31
+    f.r2u = f.cubic ? (unsigned)(u * u) + 1u : 0u;
+    return f;
+}
+typedef short rs_s16x2 __attribute__((ext_vector_type(2)));
+// (x | y << 16, z) of a cubic box, or (x, y, z) of 32 bits each
+__device__ __forceinline__ uint4 rs_fixed(double x, double y, double z, const Box &b, int cubic)
+{
+    const double fx = __builtin_amdgcn_fract(x * b.inv[0]);
+    const double fy = __builtin_amdgcn_fract(y * b.inv[1]);
+    const double fz = __builtin_amdgcn_fract(z * b.inv[2]);
+    if (cubic) {
+        const unsigned ux = (unsigned)fma(fx, 65536.0, 0.5), uy = (unsigned)fma(fy, 65536.0, 0.5),
+                       uz = (unsigned)fma(fz, 65536.0, 0.5);
+        return make_uint4((ux & 0xffffu) | (uy << 16), uz & 0xffffu, 0u, 0u);
+    }
+    return make_uint4((unsigned)(fx * 4294967296.0), (unsigned)(fy * 4294967296.0),
+                      (unsigned)(fz * 4294967296.0), 0u);
+}
+__device__ __forceinline__ bool rs_near16(uint2 a, uint2 b, unsigned r2u)
+{
+    const rs_s16x2 xy = __builtin_bit_cast(rs_s16x2, a.x) - __builtin_bit_cast(rs_s16x2, b.x);
+    const rs_s16x2 z = __builtin_bit_cast(rs_s16x2, a.y) - __builtin_bit_cast(rs_s16x2, b.y);
+    // at most 3 * 2^30: read as unsigned
+    const int r = __builtin_amdgcn_sdot2(z, z, __builtin_amdgcn_sdot2(xy, xy, 0, false), false);
+    return (unsigned)r < r2u;
+}
+__device__ __forceinline__ bool rs_near32(uint4 a, uint4 b, const RsFix &f)
+{
+    const float dx = (float)(int)(a.x - b.x) * f.w[0];
+    const float dy = (float)(int)(a.y - b.y) * f.w[1];
+    const float dz = (float)(int)(a.z - b.z) * f.w[2];
+    return fmaf(dx, dx, fmaf(dy, dy, dz * dz)) < f.r2f;
 }
 
 // Index of tile (I, J), I <= J, in the real-space tile list (I-major upper
@@ -158,31 +220,75 @@ __global__ __launch_bounds__(256) void k_tilefar(const int2 *__restrict__ tiles,
     }
 }
 
+// LDS of one tile's block.
+template <int W>
+struct RsLds {
+    double4 sI[64], sJ[64];  // x, y, z, charge
+    // fixed-point sites of J and I: 8 bytes each (cubic) or 16
+    uint4 uJ[64], uI[64];
+    double fj[3][64];
+    double fi[W][3][64];
+    double ewv[W];
+    double wv[W][6];
+    unsigned short qe[W][64 * (64 / W)];
+};
+// What a launch passes to every tile.
+struct RsArgs {
+    const double *pos;
+    long pstride;
+    const double *charge;
+    int n_atoms, NAP, nblk;
+    double gamma, half1mg;
+    const int2 *tiles;
+    int ntile, t0, nt;
+    Box box;
+    Ewald ew;
+    double *rpart, *epart;
+    int ep_stride, ep_off;
+    double *vpart;
+    RsCoef cf;
+    const double4 *sites;
+    const double *bbox;
+    const unsigned char *rfar;
+    RsFix fx;
+};
+
+// The tile of block `block` of nblocks (XCD-remapped), by its 64 W threads.
 template <bool VIR, bool CARG, bool CULL, int W>
-__global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__ pos, long pstride,
-                                                      const double *__restrict__ charge, int n_atoms,
-                                                      int NAP, int nblk, double gamma, double half1mg,
-                                                      const int2 *__restrict__ tiles, int ntile,
-                                                      int t0, int nt,
-                                                      Box box, Ewald ew,
-                                                      double *__restrict__ rpart,
-                                                      double *__restrict__ epart, int ep_stride,
-                                                      int ep_off, double *__restrict__ vpart,
-                                                      const RsCoef cf,
-                                                      const double4 *__restrict__ sites,
-                                                      const double *__restrict__ bbox,
-                                                      const unsigned char *__restrict__ rfar)
+__device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, const RsArgs &A)
 {
     static_assert(W == 2 || W == 4, "two or four waves per tile");
     constexpr int CPW = 64 / W;  // columns per wave
-    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int n_atoms = A.n_atoms, NAP = A.NAP, nblk = A.nblk, ntile = A.ntile, t0 = A.t0, nt = A.nt;
+    const int ep_stride = A.ep_stride, ep_off = A.ep_off;
+    const double gamma = A.gamma, half1mg = A.half1mg;
+    const Box &box = A.box;
+    const Ewald &ew = A.ew;
+    const RsCoef &cf = A.cf;
+    const RsFix &fx = A.fx;
+    const double *__restrict__ charge = A.charge;
+    const double4 *__restrict__ sites = A.sites;
+    const double *__restrict__ bbox = A.bbox;
+    double *__restrict__ rpart = A.rpart;
+    double *__restrict__ epart = A.epart;
+    double *__restrict__ vpart = A.vpart;
+    auto &sI = L.sI;
+    auto &sJ = L.sJ;
+    auto &uJ = L.uJ;
+    auto &uI = L.uI;
+    auto &fj = L.fj;
+    auto &fi = L.fi;
+    auto &qe = L.qe;
+    auto &ewv = L.ewv;
+    auto &wv = L.wv;
+    const int bid = xcd_remap(block, nblocks);
     const int e = bid / nt, t = t0 + (bid - e * nt);
     // a tile k_tilefar skipped (its partials zeroed there)
-    if (CULL && rfar[(long)e * ntile + t]) return;
-    const int I = tiles[t].x, J = tiles[t].y;
+    if (CULL && A.rfar[(long)e * ntile + t]) return;
+    const int I = A.tiles[t].x, J = A.tiles[t].y;
     const int l = threadIdx.x & 63;
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const double *X = pos + (long)e * pstride;
+    const double *X = A.pos + (long)e * A.pstride;
     const long base_e = (long)e * nblk * 3 * NAP;
     // CULL: the live 8 x 8 cluster pairs of the wave's columns, from the
     // cluster boxes alone, so their loads overlap the staging of the sites:
@@ -203,12 +309,6 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
                           J * 64 + 8 * cj < n_atoms && (I != J || cj >= ci);
         todo = __ballot(live) & (((CPW == 64 ? 0ull : 1ull << CPW) - 1ull) << (CPW * w));
     }
-    __shared__ double4 sI[64], sJ[64];  // x, y, z, charge
-    __shared__ double fj[3][64];
-    __shared__ double fi[W][3][64];
-    __shared__ unsigned short qe[W][64 * CPW];
-    __shared__ double ewv[W];
-    __shared__ double wv[W][6];
     if (w < 2) {
         const int s = (w == 0 ? J : I) * 64 + l;
         double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
@@ -219,6 +319,12 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
                              site_coord(X, NAP, s, 1, gamma, half1mg),
                              site_coord(X, NAP, s, 2, gamma, half1mg), charge[s]);
         (w == 0 ? sJ : sI)[l] = v;
+        uint4 *us = w == 0 ? uJ : uI;
+        const uint4 u = rs_fixed(v.x, v.y, v.z, box, fx.cubic);
+        if (fx.cubic)
+            ((uint2 *)us)[l] = make_uint2(u.x, u.y);
+        else
+            us[l] = u;
         if (w == 0) {
             fj[0][l] = 0.0;
             fj[1][l] = 0.0;
@@ -230,8 +336,16 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
     fi[w][2][l] = 0.0;
     __syncthreads();
     const int c0 = CPW * w;
-    const int i = I * 64 + l;
     int total = 0;
+    // append the pairs of `in` (one per lane) to the wave's queue
+    auto push = [&](unsigned long long bal, int il, int c) {
+        if ((bal >> l) & 1ull) {
+            const int r = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+            qe[w][total + r] = (unsigned short)(il | (c << 6));
+        }
+        total += __popcll(bal);
+    };
     if constexpr (CULL) {
         // pass 1 over the live cluster pairs: each one's 64 site pairs take
         // one lane each; the queue holds a cluster pair's entries by column,
@@ -241,50 +355,29 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
             todo &= todo - 1ull;
             const int il = 8 * (bit & 7) + (l & 7);
             const int jl = 8 * (bit >> 3) + (l >> 3);
-            const double4 a = sI[il], b = sJ[jl];
-            const double dx = mimg_fast(a.x - b.x, box.L[0], box.inv[0]);
-            const double dy = mimg_fast(a.y - b.y, box.L[1], box.inv[1]);
-            const double dz = mimg_fast(a.z - b.z, box.L[2], box.inv[2]);
-            const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
+            const bool close = fx.cubic ? rs_near16(((const uint2 *)uI)[il], ((const uint2 *)uJ)[jl], fx.r2u)
+                                        : rs_near32(uI[il], uJ[jl], fx);
             const int ii = I * 64 + il, j = J * 64 + jl;
-            const bool on = j > ii && j < n_atoms && rsq < ew.rcut_sq;
-            const unsigned long long bal = __ballot(on);
-            if (on) {
-                const int r = __builtin_amdgcn_mbcnt_hi(
-                    (unsigned)(bal >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-                qe[w][total + r] = (unsigned short)(il | ((jl - c0) << 6));
-            }
-            total += __popcll(bal);
+            push(__ballot(close && j > ii && j < n_atoms), il, jl - c0);
         }
     } else {
-        // pass 1: in-cutoff columns of row i (j > i; j < n_atoms)
-        unsigned int mask = 0u;
-        if (i < n_atoms) {
-            const double4 a = sI[l];
+        // pass 1, column by column: rows that exist, j > i in diagonal tiles
+        const int nrow = min(64, n_atoms - I * 64), ncol = n_atoms - J * 64;
+        const unsigned long long rows = nrow == 64 ? ~0ull : (1ull << nrow) - 1ull;
+        auto keep = [&](unsigned long long bal, int jl) {
+            if (I == J) bal &= (1ull << jl) - 1ull;
+            return jl < ncol ? bal & rows : 0ull;
+        };
+        if (fx.cubic) {
+            const uint2 a = ((const uint2 *)uI)[l];
 #pragma unroll
-            for (int c = 0; c < CPW; ++c) {
-                const int jl = c0 + c;
-                const int j = J * 64 + jl;
-                const double4 b = sJ[jl];
-                const double dx = mimg_fast(a.x - b.x, box.L[0], box.inv[0]);
-                const double dy = mimg_fast(a.y - b.y, box.L[1], box.inv[1]);
-                const double dz = mimg_fast(a.z - b.z, box.L[2], box.inv[2]);
-                const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
-                if (j > i && j < n_atoms && rsq < ew.rcut_sq) mask |= 1u << c;
-            }
-        }
-        // the wave's pair queue, column-major: column c's rows at off_c + (the
-        // lane's rank among the column's set lanes)
+            for (int c = 0; c < CPW; ++c)
+                push(keep(__ballot(rs_near16(a, ((const uint2 *)uJ)[c0 + c], fx.r2u)), c0 + c), l, c);
+        } else {
+            const uint4 a = uI[l];
 #pragma unroll
-        for (int c = 0; c < CPW; ++c) {
-            const bool on = (mask >> c) & 1u;
-            const unsigned long long bal = __ballot(on);
-            if (on) {
-                const int r = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                                        __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-                qe[w][total + r] = (unsigned short)(l | (c << 6));
-            }
-            total += __popcll(bal);
+            for (int c = 0; c < CPW; ++c)
+                push(keep(__ballot(rs_near32(a, uJ[c0 + c], fx)), c0 + c), l, c);
         }
     }
     __syncthreads();
@@ -310,10 +403,19 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
             b = sJ[jl];
         }
         const double4 a = sI[il];
-        const double dx = mimg_fast(a.x - b.x, box.L[0], box.inv[0]);
-        const double dy = mimg_fast(a.y - b.y, box.L[1], box.inv[1]);
-        const double dz = mimg_fast(a.z - b.z, box.L[2], box.inv[2]);
-        const double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
+        double dx = mimg_fast(a.x - b.x, box.L[0], box.inv[0]);
+        double dy = mimg_fast(a.y - b.y, box.L[1], box.inv[1]);
+        double dz = mimg_fast(a.z - b.z, box.L[2], box.inv[2]);
+        double rsq = fma(dx, dx, fma(dy, dy, dz * dz));
+        double qq = a.w * b.w;
+        // the exact cutoff: a pair of pass 1's margin (or with a NaN) adds nothing
+        const bool out = !(rsq < ew.rcut_sq);
+        if (__builtin_expect(__ballot(out) != 0ull, 0)) {
+            if (out) {
+                dx = dy = dz = qq = 0.0;
+                rsq = ew.rcut_sq;
+            }
+        }
         const double rinv = rsqrt_pos(rsq);
         double ex, ec;
         if constexpr (CARG) {
@@ -327,7 +429,6 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
         // same molecule: -erf (forces.cpp:158-166); a molecule's three sites
         // lie in one 64-site block or two consecutive ones
         if (near && (I * 64 + il) / 3 == (J * 64 + jl) / 3) ec -= 1.0;
-        const double qq = a.w * b.w;
         const double ep = qq * rinv * ec;
         const double pf = (ep + qq * ew.pref2k * ex) * (rinv * rinv);
         en += ep;
@@ -386,6 +487,13 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const double *__restrict__
         for (int k = 0; k < W; ++k) s += ewv[k];
         epart[(long)e * ep_stride + ep_off + t] = s;
     }
+}
+
+template <bool VIR, bool CARG, bool CULL, int W>
+__global__ __launch_bounds__(64 * W) void k_realspace(const RsArgs A)
+{
+    __shared__ RsLds<W> L;
+    rs_tile<VIR, CARG, CULL, W>(L, blockIdx.x, gridDim.x, A);
 }
 
 }  // namespace qtp

@@ -895,7 +895,7 @@ __global__ __launch_bounds__(256) void k_nl_fill(int n_mols, int NAP, const doub
 
 // Rebuild test (update.cpp:356-385) and, when it fires, the bead's Verlet
 // lists (neighbour.cpp:12-62) in one launch: one block of 1024 threads per
-// bead.  Row counts live in LDS (n_mols <= NL_MAXMOL), rows are handled one
+// bead.  Row counts live in LDS (n_mols <= NL_FUSED_MAXMOL), rows are handled one
 // per wavefront with ballot + prefix-popcount compaction; the distance test
 // is bit-for-bit neighbour.cpp:42-53.   grid: P.
 // (a1, a2) <- the two largest of {a1 >= a2} and {b1 >= b2}
@@ -908,7 +908,6 @@ __device__ __forceinline__ void top2_merge(double &a1, double &a2, double b1, do
         a1 = b1;
     }
 }
-constexpr int NL_MAXMOL = 4096;
 // Above this size the rebuild runs on the four-kernel path (k_check,
 // k_nl_count, k_nl_scan, k_nl_fill: a wavefront per molecule row instead of
 // one block per bead), whose rebuild steps are far shorter at thousands of
@@ -922,26 +921,87 @@ struct HeatArgs {
     double *heat_acc, *heat_step;
     int ntile, nh;
 };
-__global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NMP,
-                                                     const double *__restrict__ q, Box box,
-                                                     double r_skin_sq, double skin, int force_all,
-                                                     int every,
-                                                     const unsigned long long *__restrict__ step_ctr,
-                                                     int list_size, long fcap,
-                                                     double *__restrict__ disp,
-                                                     int *__restrict__ flag,
-                                                     double *__restrict__ nreb,
-                                                     int *__restrict__ point,
-                                                     int *__restrict__ fpoint,
-                                                     int *__restrict__ list,
-                                                     int *__restrict__ flist,
-                                                     int *__restrict__ status, HeatArgs heat)
+struct NlArgs {
+    int n_mols, NAP, NMP;
+    const double *q;
+    Box box;
+    double r_skin_sq, skin;
+    int force_all, every;
+    const unsigned long long *step_ctr;
+    int list_size;
+    long fcap;
+    double *disp;
+    int *flag;
+    double *nreb;
+    int *point, *fpoint, *list, *flist, *status;
+    int keep_disp;  // leave a rebuilt bead's displacements for a later launch to zero
+    HeatArgs heat;
+};
+struct NlLds {
+    double s1[16], s2[16];
+    int ch[NL_FUSED_MAXMOL], cf[NL_FUSED_MAXMOL];
+    int flag, tot[2];
+};
+// Whether bead b's lists are rebuilt this step: its two largest O
+// displacements (update.cpp:356-385), or forced.  By a block of NT threads;
+// the same value in every thread.
+template <int NT>
+__device__ __forceinline__ int list_flag(double *s1, double *s2, int *flag, int b, const NlArgs &A)
 {
-    __shared__ double s1[16], s2[16];
-    __shared__ int ch[NL_MAXMOL], cf[NL_MAXMOL];
-    __shared__ int s_flag, s_tot[2];
-    const int b = blockIdx.x, tid = threadIdx.x;
-    if (heat.part && b == (int)gridDim.x - 1) {  // the extra last block: the heat sum only
+    const double *D = A.disp + (long)b * 3 * A.NMP;
+    const int tid = threadIdx.x;
+    double m1 = 0.0, m2 = 0.0;
+    for (int i = tid; i < A.n_mols; i += NT) {
+        const double dx = D[i], dy = D[A.NMP + i], dz = D[2 * A.NMP + i];
+        const double d2 = dx * dx + dy * dy + dz * dz;
+        if (d2 > m1) {
+            m2 = m1;
+            m1 = d2;
+        } else if (d2 > m2) {
+            m2 = d2;
+        }
+    }
+    // top two of the block: within each wave by shuffles, then over the waves
+    for (int o = 32; o > 0; o >>= 1) {
+        const double b1 = __shfl_xor(m1, o, 64), b2 = __shfl_xor(m2, o, 64);
+        top2_merge(m1, m2, b1, b2);
+    }
+    if ((tid & 63) == 0) {
+        s1[tid >> 6] = m1;
+        s2[tid >> 6] = m2;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double t1 = s1[0], t2 = s2[0];
+        for (int ww = 1; ww < NT / 64; ++ww) top2_merge(t1, t2, s1[ww], s2[ww]);
+        int f = A.force_all || (sqrt(t1) + sqrt(t2) > A.skin);
+        if (A.every > 0 && A.step_ctr && (A.step_ctr[0] + 1ull) % (unsigned long long)A.every == 0ull)
+            f = 1;
+        *flag = f;
+    }
+    __syncthreads();
+    return *flag;
+}
+// Bead `block` of nblocks by NT threads.
+template <int NT>
+__device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, const NlArgs &A)
+{
+    const int n_mols = A.n_mols, NAP = A.NAP, NMP = A.NMP, list_size = A.list_size;
+    const double *__restrict__ q = A.q;
+    const Box &box = A.box;
+    const double r_skin_sq = A.r_skin_sq;
+    const long fcap = A.fcap;
+    double *__restrict__ disp = A.disp;
+    int *__restrict__ flag = A.flag;
+    double *__restrict__ nreb = A.nreb;
+    int *__restrict__ point = A.point;
+    int *__restrict__ fpoint = A.fpoint;
+    int *__restrict__ list = A.list;
+    int *__restrict__ flist = A.flist;
+    int *__restrict__ status = A.status;
+    const HeatArgs &heat = A.heat;
+    const int b = block, tid = threadIdx.x;
+    if (heat.part && b == nblocks - 1) {  // the extra last block: the heat sum only
         if (tid < 64) {
             const double ke = wave_sum_array(heat.part, heat.ntile);
             const double h = wave_sum_array(heat.hpart, heat.nh);
@@ -954,45 +1014,17 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NM
         return;
     }
     double *D = disp + (long)b * 3 * NMP;
-    // --- two largest O displacements
-    double m1 = 0.0, m2 = 0.0;
-    for (int i = tid; i < n_mols; i += 1024) {
-        const double dx = D[i], dy = D[NMP + i], dz = D[2 * NMP + i];
-        const double d2 = dx * dx + dy * dy + dz * dz;
-        if (d2 > m1) {
-            m2 = m1;
-            m1 = d2;
-        } else if (d2 > m2) {
-            m2 = d2;
-        }
-    }
-    // top two of the block: within each wave by shuffles, then over the 16 waves
-    for (int o = 32; o > 0; o >>= 1) {
-        const double b1 = __shfl_xor(m1, o, 64), b2 = __shfl_xor(m2, o, 64);
-        top2_merge(m1, m2, b1, b2);
-    }
-    if ((tid & 63) == 0) {
-        s1[tid >> 6] = m1;
-        s2[tid >> 6] = m2;
-    }
-    __syncthreads();
+    const int f = list_flag<NT>(S.s1, S.s2, &S.flag, b, A);
     if (tid == 0) {
-        double t1 = s1[0], t2 = s2[0];
-        for (int ww = 1; ww < 16; ++ww) top2_merge(t1, t2, s1[ww], s2[ww]);
-        int f = force_all || (sqrt(t1) + sqrt(t2) > skin);
-        if (every > 0 && step_ctr && (step_ctr[0] + 1ull) % (unsigned long long)every == 0ull)
-            f = 1;
-        s_flag = f;
         flag[b] = f;
         if (f && nreb) nreb[b] += 1.0;
     }
-    __syncthreads();
-    if (!s_flag) return;
+    if (!f) return;
     // --- counts
     const double *Q = q + (long)b * 3 * NAP;
     const int lane = tid & 63, w = tid >> 6;
     const unsigned long long below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    for (int i = w; i < n_mols; i += 16) {
+    for (int i = w; i < n_mols; i += NT / 64) {
         const double xi = Q[3 * i], yi = Q[NAP + 3 * i], zi = Q[2 * NAP + 3 * i];
         int nh = 0, nf = 0;
         for (int j0 = 0; j0 < n_mols; j0 += 64) {
@@ -1008,8 +1040,8 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NM
             nh += __popcll(__ballot(in && j > i));
         }
         if (lane == 0) {
-            ch[i] = nh;
-            cf[i] = nf;
+            S.ch[i] = nh;
+            S.cf[i] = nf;
         }
     }
     __syncthreads();
@@ -1018,7 +1050,7 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NM
         int carry_h = 0, carry_f = 0;
         for (int i0 = 0; i0 < n_mols; i0 += 64) {
             const int i = i0 + lane;
-            const int vh = i < n_mols ? ch[i] : 0, vf = i < n_mols ? cf[i] : 0;
+            const int vh = i < n_mols ? S.ch[i] : 0, vf = i < n_mols ? S.cf[i] : 0;
             int ih = vh, iff = vf;
             for (int o = 1; o < 64; o <<= 1) {
                 const int th = __shfl_up(ih, o, 64), tf = __shfl_up(iff, o, 64);
@@ -1028,34 +1060,35 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NM
                 }
             }
             if (i < n_mols) {
-                ch[i] = carry_h + ih - vh;
-                cf[i] = carry_f + iff - vf;
+                S.ch[i] = carry_h + ih - vh;
+                S.cf[i] = carry_f + iff - vf;
             }
             carry_h += __shfl(ih, 63, 64);
             carry_f += __shfl(iff, 63, 64);
         }
         if (lane == 0) {
-            s_tot[0] = carry_h;
-            s_tot[1] = carry_f;
+            S.tot[0] = carry_h;
+            S.tot[1] = carry_f;
         }
     }
     __syncthreads();
-    const int nh_tot = s_tot[0], nf_tot = s_tot[1];
+    const int nh_tot = S.tot[0], nf_tot = S.tot[1];
     if (tid == 0 && (nh_tot > list_size || (long)nf_tot > fcap)) atomicOr(status, 1);
-    for (int i = tid; i < n_mols; i += 1024) {
-        point[(long)b * n_mols + i] = ch[i];
-        fpoint[(long)b * (n_mols + 1) + i] = cf[i];
+    for (int i = tid; i < n_mols; i += NT) {
+        point[(long)b * n_mols + i] = S.ch[i];
+        fpoint[(long)b * (n_mols + 1) + i] = S.cf[i];
     }
     if (tid == 0) fpoint[(long)b * (n_mols + 1) + n_mols] = nf_tot;
     int *L = list + (long)b * list_size;
     int *FL = flist + (long)b * fcap;
-    for (int k = nh_tot + tid; k < list_size; k += 1024) L[k] = 0;
-    for (int t = tid; t < 3 * NMP; t += 1024) D[t] = 0.0;
+    for (int k = nh_tot + tid; k < list_size; k += NT) L[k] = 0;
+    if (!A.keep_disp)
+        for (int t = tid; t < 3 * NMP; t += NT) D[t] = 0.0;
     // --- fill
-    for (int i = w; i < n_mols; i += 16) {
+    for (int i = w; i < n_mols; i += NT / 64) {
         const double xi = Q[3 * i], yi = Q[NAP + 3 * i], zi = Q[2 * NAP + 3 * i];
-        int kh = ch[i];
-        long kf = cf[i];
+        int kh = S.ch[i];
+        long kf = S.cf[i];
         for (int j0 = 0; j0 < n_mols; j0 += 64) {
             const int j = j0 + lane;
             bool in = false;
@@ -1079,6 +1112,94 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(int n_mols, int NAP, int NM
             kh += __popcll(bh);
         }
     }
+}
+__global__ __launch_bounds__(1024) void k_nlist_bead(const NlArgs A)
+{
+    __shared__ NlLds L;
+    nlist_block<1024>(L, blockIdx.x, gridDim.x, A);
+}
+
+// ---------------------------------------------------------------------------
+// A force phase in three launches on one stream (the third is k_kforce_mf).
+// With the k-space and LJ kernels on a second stream a phase spent 5 us on the
+// fork and 9 us on the join (a kernel starts that long after the last event of
+// another queue; 0-1 us after its predecessor on its own queue).  The FP64
+// matrix instructions and the FP64 vector instructions of different blocks
+// take turns on the same units, so two launches side by side gain no
+// arithmetic rate either.  us a step, two streams -> this form: 216 H2O
+// classical 47 -> 37, 512 classical with the learned correction 79 -> 68, 216
+// x 32 154 -> 148, 512 x 32 447 -> 409, 990 x 16 566 -> 539.
+// ---------------------------------------------------------------------------
+// First launch, 256 threads, LDS for the largest role: n_nl blocks of list
+// checks and rebuilds of a step (and its heat sum); n_ks blocks of structure
+// factors; n_lj of LJ and intramolecular terms; n_rs real-space tiles.  The
+// roles with the longer latency come first when all blocks fit the chip at
+// once (512 classical 68 against 70 us a step) and the fuller real-space
+// blocks otherwise (512 x 32 409 against 418).
+// The LJ blocks here of a step's first phase (n_nl > 0) test their bead's
+// displacements themselves: a bead whose lists this launch rebuilds is left to
+// k_phase_reduce, which also zeroes its displacements (nothing may change
+// them while both roles read them).
+constexpr int PH_CAP = 2;   // k_ksum_mf's CAP here: few accumulators, so that six
+                            // waves fit a SIMD (four: 512 x 32 469 us a step)
+constexpr int PH_SUB = 32;  // sites whose factor tables are staged at a time: about
+                            // the LDS of a real-space block
+constexpr int PH_RESIDENT = 256 * 6;  // blocks the chip holds at once
+// With at most this many LJ blocks (two a CU: a launch of their own would be
+// all latency) they run in the first launch, beside the real-space tiles;
+// with more, in the second (216 x 32, 432 blocks: 148 us a step in the first,
+// 152 in the second; 512 x 32, 1024 blocks: 414 and 409).
+constexpr int PH_LJ_EARLY = 512;
+struct LjLds {
+    double sh[16], s1[16], s2[16];
+    int flag;
+};
+template <bool VIR, int LPM>
+__global__ __launch_bounds__(256, 6) void k_phase_pairs(const RsArgs rs, const KsArgs ks,
+                                                        const LjArgs lj, const NlArgs nl, int n_nl,
+                                                        int n_ks, int n_lj, int n_rs)
+{
+    extern __shared__ double smem[];
+    int b = blockIdx.x;
+    if (b < n_nl) {
+        nlist_block<256>(*(NlLds *)smem, b, n_nl, nl);
+        return;
+    }
+    b -= n_nl;
+    const bool rs_last = n_ks + n_lj + n_rs <= PH_RESIDENT;
+    if (rs_last ? b >= n_ks + n_lj : b < n_rs) {
+        rs_tile<VIR, true, false, 4>(*(RsLds<4> *)smem, rs_last ? b - n_ks - n_lj : b, n_rs, rs);
+        return;
+    }
+    if (!rs_last) b -= n_rs;
+    if (b < n_ks) {
+        ks_block<PH_CAP, 4>(smem, b, ks);
+        return;
+    }
+    LjLds &L = *(LjLds *)smem;
+    b -= n_ks;
+    if (n_nl > 0 && list_flag<256>(L.s1, L.s2, &L.flag, lj_eval<LPM>(b, n_lj, lj), nl)) return;
+    lj_block<VIR, LPM>(L.sh, b, n_lj, lj);
+}
+// Second launch, 256 threads: n_lj blocks for the LJ and intramolecular terms,
+// of every bead or (rebuilt_only) of the beads whose lists the first launch
+// rebuilt; the rest: reduction of the structure factors.  n_nl > 0: a step's
+// first phase, whose rebuilt beads' displacements are zeroed here.
+template <bool VIR, int LPM>
+__global__ __launch_bounds__(256) void k_phase_reduce(const SrArgs sr, const LjArgs lj, const NlArgs nl,
+                                                      int n_nl, int n_lj, int rebuilt_only)
+{
+    __shared__ double sh[16];
+    const int b = blockIdx.x;
+    if (b >= n_lj) {
+        sreduce_block(sh, b - n_lj, sr);
+        return;
+    }
+    const int e = lj_eval<LPM>(b, n_lj, lj);
+    const bool rebuilt = n_nl > 0 && nl.flag[e];
+    if (rebuilt || !rebuilt_only) lj_block<VIR, LPM>(sh, b, n_lj, lj);
+    if (rebuilt && lj_eval_first<LPM>(b, n_lj, lj))
+        for (int t = threadIdx.x; t < 3 * nl.NMP; t += 256) nl.disp[(long)e * 3 * nl.NMP + t] = 0.0;
 }
 
 // ---------------------------------------------------------------------------
