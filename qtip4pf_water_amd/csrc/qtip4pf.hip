@@ -30,6 +30,7 @@ const char *qtp_noalloc_last_error();
 #include "qtp_host_setup.hpp"
 #include "qtp_host_nn.hpp"
 #include "qtp_host_run.hpp"
+#include "qtp_host_xfer.hpp"
 #include "qtp_host_tune.hpp"
 
 // ===========================================================================
@@ -277,9 +278,12 @@ void qtp_destroy(qtp_ctx *ctx)
                     ctx->gcf, ctx->grk, ctx->tiles, ctx->Cm, ctx->mode, ctx->nq, ctx->np,
                     ctx->ppart, ctx->hpart, ctx->dev, ctx->obs, ctx->obs_out, ctx->ntrace, ctx->trace,
                     ctx->fnn, ctx->ms, ctx->cmf_acc, ctx->cmf_n, ctx->qc, ctx->rdf_oo,
-                    ctx->rdf_oh};
+                    ctx->rdf_oh, ctx->xref};
     for (void *p : ptrs)
         if (p) hipFree(p);
+    if (ctx->xpin) hipHostFree(ctx->xpin);
+    for (hipEvent_t e : ctx->xev)
+        if (e) hipEventDestroy(e);
     if (ctx->s2) hipStreamSynchronize(ctx->s2);
     if (ctx->s3) hipStreamSynchronize(ctx->s3);
     if (ctx->ev_fork) hipEventDestroy(ctx->ev_fork);
@@ -319,13 +323,17 @@ static int get_forces_impl(qtp_ctx *ctx, const double *q, double *F, const doubl
     if (!ctx || !q || !F || !point || !list || bead < 0 || bead >= ctx->P) return QTP_ERR_ARG;
     CHK(check_finite(ctx, q + (long)bead * ctx->n_dof, ctx->n_dof, "positions"));
     CHK(upload_charges_masses(ctx, charge, nullptr));
+    CHK(check_lists(ctx, point, list, bead, 1));
     // stage the bead's positions in evaluation slot 0 of qpm, its lists in slot `bead`
-    CHK(upload_planar(ctx, ctx->qpm, q + (long)bead * ctx->n_dof, 1));
-    CHK(upload_lists(ctx, point, list, bead, 1, bead));
+    Xfer in(ctx);
+    in.planar(ctx->qpm, q + (long)bead * ctx->n_dof, 1);
+    CHK(upload_with_lists(ctx, in, point, list, bead, 1, bead));
     CHK(run_phase(ctx, ctx->qpm, 1, 0, bead, ctx->fpm, ctx->Ve));
     double e = 0.0;
-    HIPCHK(hipMemcpyAsync(&e, ctx->Ve, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CHK(download_planar(ctx, ctx->fpm, 1, F + (long)bead * ctx->n_dof));
+    Xfer res(ctx);
+    res.planar(ctx->fpm, F + (long)bead * ctx->n_dof, 1);
+    res.raw(ctx->Ve, &e, 1);
+    CHK(res.down());
     CHK(flush_timing(ctx));
     if (energy) *energy = e;
     ctx->state_set = false;
@@ -341,13 +349,17 @@ int qtp_get_forces_virial(qtp_ctx *ctx, const double *q, double *F, const double
     SplineScope sp(ctx, false);
     CHK(check_finite(ctx, q + (long)bead * ctx->n_dof, ctx->n_dof, "positions"));
     CHK(upload_charges_masses(ctx, charge, nullptr));
-    CHK(upload_planar(ctx, ctx->qpm, q + (long)bead * ctx->n_dof, 1));
-    CHK(upload_lists(ctx, point, list, bead, 1, bead));
+    CHK(check_lists(ctx, point, list, bead, 1));
+    Xfer in(ctx);
+    in.planar(ctx->qpm, q + (long)bead * ctx->n_dof, 1);
+    CHK(upload_with_lists(ctx, in, point, list, bead, 1, bead));
     CHK(run_phase(ctx, ctx->qpm, 1, 0, bead, ctx->fpm, ctx->Ve, ctx->vout));
     double e = 0.0;
-    HIPCHK(hipMemcpyAsync(&e, ctx->Ve, sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    HIPCHK(hipMemcpyAsync(virial, ctx->vout, 6 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CHK(download_planar(ctx, ctx->fpm, 1, F + (long)bead * ctx->n_dof));
+    Xfer res(ctx);
+    res.planar(ctx->fpm, F + (long)bead * ctx->n_dof, 1);
+    res.raw(ctx->Ve, &e, 1);
+    res.raw(ctx->vout, virial, 6);
+    CHK(res.down());
     CHK(flush_timing(ctx));
     if (energy) *energy = e;
     ctx->state_set = false;
@@ -362,13 +374,17 @@ static int force_eval_sc_impl(qtp_ctx *ctx, const double *q, double *F_sc, const
     const int P = ctx->P;
     CHK(check_finite(ctx, q, (long)P * ctx->n_dof, "positions"));
     CHK(upload_charges_masses(ctx, charge, mass));
-    CHK(upload_planar(ctx, ctx->q, q, P));
-    CHK(upload_lists(ctx, point, list, 0, P, 0));
+    CHK(check_lists(ctx, point, list, 0, P));
+    Xfer in(ctx);
+    in.planar(ctx->q, q, P);
+    CHK(upload_with_lists(ctx, in, point, list, 0, P, 0));
     CHK(run_sc_forces(ctx, 0, nullptr));
     double o[2];
-    HIPCHK(hipMemcpyAsync(o, ctx->out, 2 * sizeof(double), hipMemcpyDeviceToHost, ctx->stream));
-    CHK(download_planar(ctx, ctx->F, P, F_sc));
-    if (fphys) CHK(download_planar(ctx, ctx->fph, P, fphys));
+    Xfer res(ctx);
+    res.planar(ctx->F, F_sc, P);
+    if (fphys) res.planar(ctx->fph, fphys, P);
+    res.raw(ctx->out, o, 2);
+    CHK(res.down());
     CHK(flush_timing(ctx));
     if (energy) *energy = o[0];
     if (sc_pot) *sc_pot = o[1];
@@ -486,36 +502,41 @@ static int update_sc_impl(qtp_ctx *ctx, double *q, double *p, const double *mass
     const int P = ctx->P;
     CHK(check_finite(ctx, q, (long)P * ctx->n_dof, "positions"));
     CHK(upload_charges_masses(ctx, charge, mass));
-    CHK(upload_planar(ctx, ctx->q, q, P));
-    CHK(upload_planar(ctx, ctx->p, p, P));
-    CHK(upload_planar(ctx, ctx->F, F, P));
-    CHK(upload_disp(ctx, disp, 0, P));
-    CHK(upload_lists(ctx, point, list, 0, P, 0));
-    if (is_nvt)
-        HIPCHK(hipMemcpy(ctx->dev, dev, ctx->dev_cap * sizeof(double), hipMemcpyHostToDevice));
-    HIPCHK(hipMemset(ctx->status, 0, sizeof(int)));
+    CHK(check_lists(ctx, point, list, 0, P));
+    HIPCHK(hipMemsetAsync(ctx->status, 0, sizeof(int), ctx->stream));
     double h0 = heat ? *heat : 0.0;
-    HIPCHK(hipMemcpy(ctx->heat, &h0, sizeof(double), hipMemcpyHostToDevice));
+    Xfer in(ctx);
+    in.planar(ctx->q, q, P);
+    in.planar(ctx->p, p, P);
+    in.planar(ctx->F, F, P);
+    in.disp(ctx->disp, disp, P);
+    if (is_nvt) in.raw(ctx->dev, dev, ctx->dev_cap);
+    in.raw(ctx->heat, &h0, 1);
+    CHK(upload_with_lists(ctx, in, point, list, 0, P, 0));
     CHK(run_sc_step(ctx, is_nvt, 1, nullptr));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     CHK(flush_timing(ctx));
     CHK(read_status(ctx));
     double o[2];
-    HIPCHK(hipMemcpy(o, ctx->out, 2 * sizeof(double), hipMemcpyDeviceToHost));
-    HIPCHK(hipMemcpy(&h0, ctx->heat, sizeof(double), hipMemcpyDeviceToHost));
-    CHK(download_planar(ctx, ctx->q, P, q));
-    CHK(download_planar(ctx, ctx->p, P, p));
-    CHK(download_planar(ctx, ctx->F, P, F));
-    if (fphys) CHK(download_planar(ctx, ctx->fph, P, fphys));
-    CHK(download_disp(ctx, disp, 0, P));
+    Xfer res(ctx);
+    res.planar(ctx->q, q, P);
+    res.planar(ctx->p, p, P);
+    res.planar(ctx->F, F, P);
+    if (fphys) res.planar(ctx->fph, fphys, P);
+    res.disp(ctx->disp, disp, P);
+    res.raw(ctx->out, o, 2);
+    res.raw(ctx->heat, &h0, 1);
+    CHK(res.down());
     std::vector<int> fl(P);
     HIPCHK(hipMemcpy(fl.data(), ctx->flag, P * sizeof(int), hipMemcpyDeviceToHost));
     for (int b = 0; b < P; ++b)
         if (fl[b]) {
             HIPCHK(hipMemcpy(point + (long)b * ctx->n_mols, ctx->point + (size_t)b * ctx->n_mols,
                              ctx->n_mols * sizeof(int), hipMemcpyDeviceToHost));
+            // the row's used part
+            const int used = point[(long)(b + 1) * ctx->n_mols - 1];
             HIPCHK(hipMemcpy(list + (long)b * ctx->list_size, ctx->list + (size_t)b * ctx->list_size,
-                             ctx->list_size * sizeof(int), hipMemcpyDeviceToHost));
+                             used * sizeof(int), hipMemcpyDeviceToHost));
         }
     if (heat) *heat = h0;
     if (energy) *energy = o[0];
@@ -531,27 +552,31 @@ static int update_class_impl(qtp_ctx *ctx, double *q, double *p, const double *m
     if (!ctx || !q || !p || !F || !point || !list || !disp || ctx->P != 1) return QTP_ERR_ARG;
     CHK(check_finite(ctx, q, ctx->n_dof, "positions"));
     CHK(upload_charges_masses(ctx, charge, mass));
-    CHK(upload_planar(ctx, ctx->q, q, 1));
-    CHK(upload_planar(ctx, ctx->p, p, 1));
-    CHK(upload_planar(ctx, ctx->F, F, 1));
-    CHK(upload_disp(ctx, disp, 0, 1));
-    CHK(upload_lists(ctx, point, list, 0, 1, 0));
-    HIPCHK(hipMemset(ctx->status, 0, sizeof(int)));
+    CHK(check_lists(ctx, point, list, 0, 1));
+    HIPCHK(hipMemsetAsync(ctx->status, 0, sizeof(int), ctx->stream));
+    Xfer in(ctx);
+    in.planar(ctx->q, q, 1);
+    in.planar(ctx->p, p, 1);
+    in.planar(ctx->F, F, 1);
+    in.disp(ctx->disp, disp, 1);
+    CHK(upload_with_lists(ctx, in, point, list, 0, 1, 0));
     CHK(run_class_step(ctx, nullptr));
     HIPCHK(hipStreamSynchronize(ctx->stream));
     CHK(flush_timing(ctx));
     CHK(read_status(ctx));
     double o[2];
-    HIPCHK(hipMemcpy(o, ctx->out, 2 * sizeof(double), hipMemcpyDeviceToHost));
-    CHK(download_planar(ctx, ctx->q, 1, q));
-    CHK(download_planar(ctx, ctx->p, 1, p));
-    CHK(download_planar(ctx, ctx->F, 1, F));
-    CHK(download_disp(ctx, disp, 0, 1));
+    Xfer res(ctx);
+    res.planar(ctx->q, q, 1);
+    res.planar(ctx->p, p, 1);
+    res.planar(ctx->F, F, 1);
+    res.disp(ctx->disp, disp, 1);
+    res.raw(ctx->out, o, 2);
+    CHK(res.down());
     int fl = 0;
     HIPCHK(hipMemcpy(&fl, ctx->flag, sizeof(int), hipMemcpyDeviceToHost));
     if (fl) {
         HIPCHK(hipMemcpy(point, ctx->point, ctx->n_mols * sizeof(int), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(list, ctx->list, ctx->list_size * sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(list, ctx->list, point[ctx->n_mols - 1] * sizeof(int), hipMemcpyDeviceToHost));
     }
     if (energy) *energy = o[0];
     ctx->state_set = false;
@@ -838,12 +863,13 @@ int qtp_get_state(qtp_ctx *ctx, double *q, double *p, double *F, double *fphys, 
     if (!ctx) return QTP_ERR_ARG;
     HIPCHK(hipStreamSynchronize(ctx->stream));
     const int P = ctx->P;
-    if (q) CHK(download_planar(ctx, ctx->q, P, q));
-    if (p) CHK(download_planar(ctx, ctx->p, P, p));
-    if (F) CHK(download_planar(ctx, ctx->F, P, F));
-    if (fphys) CHK(download_planar(ctx, ctx->fph, P, fphys));
-    if (disp) CHK(download_disp(ctx, disp, 0, P));
-    return QTP_OK;
+    Xfer x(ctx);
+    if (q) x.planar(ctx->q, q, P);
+    if (p) x.planar(ctx->p, p, P);
+    if (F) x.planar(ctx->F, F, P);
+    if (fphys) x.planar(ctx->fph, fphys, P);
+    if (disp) x.disp(ctx->disp, disp, P);
+    return x.A.n ? x.down() : QTP_OK;
 }
 
 // ---- checkpoint / restart ------------------------------------------------------
@@ -968,13 +994,18 @@ int qtp_load_checkpoint(qtp_ctx *ctx, const char *path, const double *charge, co
     CHK(check_finite(ctx, p.data(), (long)nd, "momenta"));
     invalidate_graphs(ctx);
     CHK(upload_charges_masses(ctx, charge, mass));
-    CHK(upload_planar(ctx, ctx->q, q.data(), P));
-    CHK(upload_planar(ctx, ctx->p, p.data(), P));
-    CHK(upload_disp(ctx, disp.data(), 0, P));
     // the saved half lists, and the full lists expanded from them: each row in
     // ascending partner order, as the list kernels write it, so the force
     // sums run in the same order as before the stop
-    CHK(upload_lists(ctx, point.data(), list.data(), 0, P, 0));
+    CHK(check_lists(ctx, point.data(), list.data(), 0, P));
+    Xfer in(ctx);
+    in.planar(ctx->q, q.data(), P);
+    in.planar(ctx->p, p.data(), P);
+    in.disp(ctx->disp, disp.data(), P);
+    CHK(upload_with_lists(ctx, in, point.data(), list.data(), 0, P, 0));
+    HIPCHK(hipStreamSynchronize(ctx->stream));
+    // the rows' unused ends as they were saved
+    HIPCHK(hipMemcpy(ctx->list, list.data(), list.size() * sizeof(int), hipMemcpyHostToDevice));
     HIPCHK(hipMemset(ctx->status, 0, sizeof(int)));
     if (P >= 2) {
         CHK(run_sc_forces(ctx, 0, nullptr));

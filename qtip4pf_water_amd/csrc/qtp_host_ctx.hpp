@@ -96,6 +96,13 @@ struct qtp_ctx {
     // NL_BM_MAX_BYTES; otherwise the fill pass tests the candidates again)
     unsigned long long *nl_bm = nullptr;
     double *nreb = nullptr;
+    // transfers of the reference-shaped calls (qtp_host_xfer.hpp): the packed
+    // arrays on the device, pinned chunks, an event per chunk
+    double *xref = nullptr;
+    size_t xref_cap = 0;
+    char *xpin = nullptr;
+    hipEvent_t xev[4] = {nullptr, nullptr, nullptr, nullptr};
+    unsigned xslot = 0;
     // force-phase scratch (E <= max(P,1))
     double *qpm = nullptr, *vpart = nullptr, *vout = nullptr, *rpart = nullptr, *spart = nullptr, *sprime = nullptr;
     double *flj = nullptr, *fpm = nullptr, *Ve = nullptr, *epart = nullptr;

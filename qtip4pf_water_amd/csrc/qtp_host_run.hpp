@@ -1,6 +1,6 @@
 // qtp_host_run.hpp -- host side of the gfx950 qTIP4P/F step: launch
 // sequences (force phases, SC forces, neighbour lists, the SC and classical
-// steps) and host <-> device layout conversion.
+// steps).
 // Included once, in order, by qtip4pf.hip (one translation unit).
 #pragma once
 
@@ -678,137 +678,6 @@ static int class_initial_forces(qtp_ctx *ctx)
                                         ctx->nn ? ctx->nn->Etile : nullptr,
                                         ctx->nn ? nn_tiles(ctx->nn) : 0);
     HIPCHK(hipGetLastError());
-    return QTP_OK;
-}
-
-// ---------------------------------------------------------------------------
-// host <-> device layout conversion
-// ---------------------------------------------------------------------------
-static void to_planar(const qtp_ctx *ctx, const double *ref, int nb, std::vector<double> &out)
-{
-    const long N3 = 3L * ctx->NAP;
-    out.assign((size_t)nb * N3, 0.0);
-    for (int b = 0; b < nb; ++b)
-        for (int a = 0; a < ctx->n_atoms; ++a)
-            for (int d = 0; d < 3; ++d)
-                out[b * N3 + (long)d * ctx->NAP + a] = ref[(long)b * ctx->n_dof + 3 * a + d];
-}
-
-static void from_planar(const qtp_ctx *ctx, const std::vector<double> &pl, int nb, double *ref)
-{
-    const long N3 = 3L * ctx->NAP;
-    for (int b = 0; b < nb; ++b)
-        for (int a = 0; a < ctx->n_atoms; ++a)
-            for (int d = 0; d < 3; ++d)
-                ref[(long)b * ctx->n_dof + 3 * a + d] = pl[b * N3 + (long)d * ctx->NAP + a];
-}
-
-static int upload_planar(qtp_ctx *ctx, double *dst, const double *ref, int nb)
-{
-    std::vector<double> h;
-    to_planar(ctx, ref, nb, h);
-    HIPCHK(hipMemcpyAsync(dst, h.data(), h.size() * sizeof(double), hipMemcpyHostToDevice,
-                          ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    return QTP_OK;
-}
-
-static int download_planar(qtp_ctx *ctx, const double *src, int nb, double *ref)
-{
-    std::vector<double> h((size_t)nb * 3 * ctx->NAP);
-    HIPCHK(hipMemcpyAsync(h.data(), src, h.size() * sizeof(double), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
-    from_planar(ctx, h, nb, ref);
-    return QTP_OK;
-}
-
-// disp: reference [b][3*mol + d]  <->  device [b][d][NMP]
-static int upload_disp(qtp_ctx *ctx, const double *ref, int b0, int nb)
-{
-    std::vector<double> h((size_t)nb * 3 * ctx->NMP, 0.0);
-    for (int b = 0; b < nb; ++b)
-        for (int i = 0; i < ctx->n_mols; ++i)
-            for (int d = 0; d < 3; ++d)
-                h[((size_t)b * 3 + d) * ctx->NMP + i] = ref[(long)(b0 + b) * 3 * ctx->n_mols + 3 * i + d];
-    HIPCHK(hipMemcpy(ctx->disp + (size_t)b0 * 3 * ctx->NMP, h.data(), h.size() * sizeof(double),
-                     hipMemcpyHostToDevice));
-    return QTP_OK;
-}
-
-static int download_disp(qtp_ctx *ctx, double *ref, int b0, int nb)
-{
-    std::vector<double> h((size_t)nb * 3 * ctx->NMP);
-    HIPCHK(hipMemcpy(h.data(), ctx->disp + (size_t)b0 * 3 * ctx->NMP, h.size() * sizeof(double),
-                     hipMemcpyDeviceToHost));
-    for (int b = 0; b < nb; ++b)
-        for (int i = 0; i < ctx->n_mols; ++i)
-            for (int d = 0; d < 3; ++d)
-                ref[(long)(b0 + b) * 3 * ctx->n_mols + 3 * i + d] = h[((size_t)b * 3 + d) * ctx->NMP + i];
-    return QTP_OK;
-}
-
-// Caller's half lists (reference layout) -> device half + full lists.  Row
-// n_mols-1 is ignored as forces.cpp:489 does.
-static int upload_lists(qtp_ctx *ctx, const int *point, const int *list, int b0, int nb,
-                        int dev_b0)
-{
-    const int n = ctx->n_mols;
-    std::vector<int> fp((size_t)nb * (n + 1)), fl((size_t)nb * ctx->fcap, 0);
-    for (int bb = 0; bb < nb; ++bb) {
-        const int b = b0 + bb;
-        const int *pt = point + (long)b * n;
-        const int *ls = list + (long)b * ctx->list_size;
-        std::vector<std::vector<int>> rows(n);
-        for (int i = 0; i < n - 1; ++i) {
-            const int k0 = pt[i], k1 = pt[i + 1];
-            if (k0 < 0 || k1 > ctx->list_size || k1 < k0) {
-                ctx->err = "neighbour list: point[] out of range";
-                return QTP_ERR_ARG;
-            }
-            for (int k = k0; k < k1; ++k) {
-                const int j = ls[k];
-                if (j < 0 || j >= n) {
-                    ctx->err = "neighbour list: entry out of range";
-                    return QTP_ERR_ARG;
-                }
-                rows[j].push_back(i);
-            }
-        }
-        long pos = 0;
-        for (int i = 0; i < n; ++i) {
-            fp[(size_t)bb * (n + 1) + i] = (int)pos;
-            std::vector<int> r = rows[i];  // partners j < i (i in row j)
-            if (i < n - 1)
-                for (int k = pt[i]; k < pt[i + 1]; ++k) r.push_back(ls[k]);
-            for (int j : r) {
-                if (pos >= ctx->fcap) {
-                    ctx->err = "neighbour list: full list exceeds capacity";
-                    return QTP_ERR_LIST_OVERFLOW;
-                }
-                fl[(size_t)bb * ctx->fcap + pos++] = j;
-            }
-        }
-        fp[(size_t)bb * (n + 1) + n] = (int)pos;
-    }
-    HIPCHK(hipMemcpy(ctx->fpoint + (size_t)dev_b0 * (n + 1), fp.data(), fp.size() * sizeof(int),
-                     hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(ctx->flist + (size_t)dev_b0 * ctx->fcap, fl.data(), fl.size() * sizeof(int),
-                     hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(ctx->point + (size_t)dev_b0 * n, point + (long)b0 * n, (size_t)nb * n * sizeof(int),
-                     hipMemcpyHostToDevice));
-    HIPCHK(hipMemcpy(ctx->list + (size_t)dev_b0 * ctx->list_size, list + (long)b0 * ctx->list_size,
-                     (size_t)nb * ctx->list_size * sizeof(int), hipMemcpyHostToDevice));
-    return QTP_OK;
-}
-
-static int check_finite(qtp_ctx *ctx, const double *a, long n, const char *what)
-{
-    for (long i = 0; i < n; ++i)
-        if (!std::isfinite(a[i])) {
-            ctx->err = std::string(what) + " contains a non-finite value";
-            return QTP_ERR_NONFINITE;
-        }
     return QTP_OK;
 }
 
