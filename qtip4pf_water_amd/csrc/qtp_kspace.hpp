@@ -349,8 +349,10 @@ __global__ __launch_bounds__(64 * KS_WAVES, 4) void k_ksum_mf(const KsArgs A)
 // (E_k = c |S(k)|^2 per sign variant; the strain derivative of kwald's sum at
 // fixed Ewald parameters).
 // With wm set, the force coefficients go to k_kforce_mf's matrix instead of
-// the records: W[n][8 col + s] (n = 2 kz + 0/1 for the Re/Im z factor; s =
-// u1 u2 v1 v2 u3 u4 v3 v4, the Z-linear sums of k_kforce; col = gcol[g]).
+// the records: W[n][row] (n = 2 kz + 0/1 for the Re/Im z factor; the column's
+// rows u1 u2 u3 u4 v1 v2 v3 v4, the Z-linear sums of k_kforce, in pairs at 0,
+// 4, 8 and 12 of its 16-row tile, the second column's two further; column =
+// gcol[g]).
 // Each coefficient c_v enters twice: as the u weight of its own component and,
 // times +-kz b_z, as the v weight of the other part of the same variant pair.
 // Only these entries are ever written; the rest of W stays zero.
@@ -461,11 +463,13 @@ __device__ __forceinline__ void sreduce_block(double *sh, int block, const SrArg
         if (wm) {
             const int kz = groups[g].z;
             const int lo = v & 1, hi = (v >> 1) & 1;
-            const int row = 8 * gcol[g] + (v >> 2) * 4;
+            const int col = gcol[g];
+            // rows of the tile: 4 (2 [v] + side) + 2 (column of the pair) + 0/1
+            const int row = 16 * (col >> 1) + 4 * (v >> 2) + 2 * (col & 1);
             const double kzr = bkz * kz;
             double *W = wm + (long)e * NN * Mp;
             W[(long)(2 * kz + lo) * Mp + row + hi] = cv;
-            W[(long)(2 * kz + 1 - lo) * Mp + row + 3 - hi] = (lo == hi ? -kzr : kzr) * cv;
+            W[(long)(2 * kz + 1 - lo) * Mp + row + 8 + 1 - hi] = (lo == hi ? -kzr : kzr) * cv;
         } else {
             // record of k_kforce (9 doubles): c1..c8, then (kx, ky, kz) packed
             double *o = sprime + ((long)e * G + g) * KF_REC;
@@ -709,17 +713,20 @@ __global__ __launch_bounds__(64 * W) void k_kforce(
 // Reciprocal-space forces on FP64 matrix cores (v_mfma_f64_16x16x4f64), the
 // same sums as k_kforce (forces.cpp:276-279, 319-324, 368-373, 434-442).
 // Per evaluation, the Z-linear sums of every column and every site form one
-// product  D[8 col + s][site] = sum_n W[8 col + s][n] Zt[n][site]  with
-// Zt[2 kz][j], Zt[2 kz + 1][j] = Re, Im e^{i kz b_z z_j} and W written by
-// k_sreduce.  Columns are sorted by their largest kz, so a 16-row tile (two
-// columns) takes only the k-steps of 4 that its columns reach (tile table
-// rt: packed (kx, ky) of both columns, k-steps, first row; in the order the
-// waves take them, k-steps balanced over the waves; k-steps 0 = no tile).
-// The epilogue applies each column's A = XY, B = XY* and kx, ky per site:
-// with lane group g = lane / 16 holding rows 8 c' + g and 8 c' + g + 4 of
-// both columns of a tile (the 16x16 result layout), g = 0, 1 give the x and
-// y forces of (Ar u1 + Br u3) and (Ai u2 + Bi u4), g = 2, 3 the z force of
-// (Ar v1 + Br v3) and (Ai v2 + Bi v4).
+// product  D[row][site] = sum_n W[row][n] Zt[n][site]  with Zt[2 kz][j],
+// Zt[2 kz + 1][j] = Re, Im e^{i kz b_z z_j} and W written by k_sreduce.
+// Columns are sorted by their largest kz, so a 16-row tile (two columns) takes
+// only the k-steps of 4 that its columns reach (tile table rt: packed (kx, ky)
+// of both columns, k-steps, first row; in the order the waves take them,
+// k-steps balanced over the waves; k-steps 0 = no tile).
+// The epilogue applies each column's A = XY, B = XY* and kx, ky per site.  The
+// rows of a tile are laid out so that a lane's four results (rows g, 4 + g,
+// 8 + g, 12 + g, g = lane / 16) belong to one column (g >> 1): part g & 1 (Re,
+// Im) of the weights of A and B in the x and y forces, (u1, u3) or (u2, u4),
+// and in the z force, (v1, v3) or (v2, v4).  So each lane forms its part of A
+// and B once a tile: 11 FP64 instructions and four 8-byte LDS reads per site
+// tile next to 3 to 20 products of 64 cycles.  With the two columns' results
+// in separate registers it was 20 and eight (4096 x 32: 996 us then, 902 now).
 // Block = 48 sites (16 whole molecules: three 16-site tiles) x W waves (8,
 // or 16 when a launch has few site blocks); each wave reads the z factors of
 // the three site tiles (the B operands) from LDS and takes every W-th row
@@ -740,8 +747,8 @@ constexpr int MF_MAXKS = 12;
 
 inline size_t kforce_mf_lds_bytes(int K, int nks, int W)
 {
-    return (size_t)2 * K * MF_SITES * 16 + (size_t)4 * nks * MF_SITES * 8 +
-           (size_t)2 * W * 3 * MF_SITES * 8 + (size_t)3 * MF_SITES * 8;
+    return (size_t)4 * K * MF_SITES * 8 + (size_t)4 * nks * MF_SITES * 8 +
+           (size_t)W * 3 * MF_SITES * 8 + (size_t)3 * MF_SITES * 8;
 }
 
 // One 16-row tile of k_kforce_mf over three site tiles, NT k-steps: the A
@@ -779,11 +786,10 @@ __global__ __launch_bounds__(64 * W) void k_kforce_mf(
 {
     extern __shared__ double smem[];
     const int K = ew.K, NN = 4 * nks;
-    double2 *T = (double2 *)smem;                    // [2][K][48] x (charge folded), y factors
-    double *Zt = smem + 4 * K * MF_SITES;            // [NN][48]
-    double *red = Zt + NN * MF_SITES;                // [W][3][48] k-space wave partials
-    double *rsm = red + W * 3 * MF_SITES;     // [W][3][48] real-space slot partials
-    double *ef = rsm + W * 3 * MF_SITES;      // [3][48]
+    double *T = smem;                         // [2][K][Re, Im][48] x (charge folded), y factors
+    double *Zt = smem + 4 * K * MF_SITES;     // [NN][48], n = 2 kz + 0/1
+    double *red = Zt + NN * MF_SITES;         // [W][3][48] wave partials
+    double *ef = red + W * 3 * MF_SITES;      // [3][48]
     const int nbm = (n_atoms + MF_SITES - 1) / MF_SITES;
     const int bid = xcd_remap(blockIdx.x, gridDim.x);
     const int e = bid / nbm, ab = bid - e * nbm;
@@ -839,38 +845,28 @@ __global__ __launch_bounds__(64 * W) void k_kforce_mf(
         // factor tables by the recurrence of kw_table (forces.cpp:212-245)
         const int d = threadIdx.x / MF_SITES, j = threadIdx.x - d * MF_SITES;
         const int atom = a0 + j;
-        const bool va = atom < n_atoms;
-        double sn = 0.0, cs = 0.0, qf = 0.0;
-        if (va) {
+        double br = 0.0, qf = 0.0;
+        if (atom < n_atoms) {
             qf = d == 0 ? charge[atom] : 1.0;
-            sincos(ew.bk[d] * site_coord(X, NAP, atom, d, gamma, half1mg), &sn, &cs);
+            br = ew.bk[d] * site_coord(X, NAP, atom, d, gamma, half1mg);
         }
-        double cm = 1.0, sm = 0.0;
-        for (int m = 0; m < K; ++m) {
-            if (m > 0) {
-                const double cn = cs * cm - sn * sm;
-                const double snn = sn * cm + cs * sm;
-                cm = cn;
-                sm = snn;
-            }
-            const double c = va ? cm * qf : 0.0, s = va ? sm * qf : 0.0;
-            if (d < 2) {
-                T[(d * K + m) * MF_SITES + j] = make_double2(c, s);
-            } else {
-                Zt[(2 * m) * MF_SITES + j] = c;
-                Zt[(2 * m + 1) * MF_SITES + j] = s;
-            }
-        }
+        double *row = T + 2 * d * K * MF_SITES + j;
+        mf_factors(br, qf, K, [&](int m, double c, double s) {
+            row[2 * m * MF_SITES] = c;
+            row[(2 * m + 1) * MF_SITES] = s;
+        });
         if (d == 2)
             for (int n = 2 * K; n < NN; ++n) Zt[n * MF_SITES + j] = 0.0;
     }
     __syncthreads();
     const int j = lane & 15, gq = lane >> 4;
     const double *Zl = Zt + gq * MF_SITES + j;  // B operand of k-step t, site tile st: Zl[4t*48 + 16st]
-    const bool odd = gq & 1;
+    // the lane's column of a tile (gq >> 1) and part (gq & 1: the y factors'
+    // Re and Im change places)
+    const bool odd = gq & 1, second = gq & 2;
     const double sg = odd ? 1.0 : -1.0;
-    const bool gxy = gq < 2;
-    double acc1[3] = {0.0, 0.0, 0.0}, acc2[3] = {0.0, 0.0, 0.0};
+    const double *Xl = T + j, *Yl = Xl + (2 * K + odd) * MF_SITES, *Yo = Xl + (2 * K + !odd) * MF_SITES;
+    double ax[3] = {0.0, 0.0, 0.0}, ay[3] = {0.0, 0.0, 0.0}, az[3] = {0.0, 0.0, 0.0};
     const double *We = wm + (long)e * NN * Mp;
     for (int i = w; i < nrt; i += W) {
         const int4 r = rt[i];
@@ -913,50 +909,43 @@ __global__ __launch_bounds__(64 * W) void k_kforce_mf(
             default: mf_tile<6>(Wr2, Mp4, Zl2, d0, d1, d2); break;
             }
         }
+        const int ck = second ? r.y : r.x;
+        const int kx = ck & 0xffff, ky = ck >> 16;
+        const int xo = 2 * MF_SITES * kx, yo = 2 * MF_SITES * ky;
+        const double cx = ew.bk[0] * kx, cy = ew.bk[1] * ky;
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
-            const int ck = h ? r.y : r.x;
-            const int kx = ck & 0xffff, ky = ck >> 16;
-            const double cx = gxy ? ew.bk[0] * kx : 1.0, cy = gxy ? ew.bk[1] * ky : 0.0;
-#pragma unroll
-            for (int st = 0; st < 3; ++st) {
-                const mf_v4d &D = st == 0 ? d0 : st == 1 ? d1 : d2;
-                const double2 Xv = T[kx * MF_SITES + 16 * st + j];
-                const double2 Yv = T[(K + ky) * MF_SITES + 16 * st + j];
-                const double s1 = Xv.x * (odd ? Yv.y : Yv.x), s2 = Xv.y * (odd ? Yv.x : Yv.y);
-                const double a = fma(sg, s2, s1), b = fma(-sg, s1, s2);
-                const double ta = a * D[2 * h], tb = b * D[2 * h + 1];
-                acc1[st] = fma(-cx, ta + tb, acc1[st]);
-                acc2[st] = fma(-cy, ta - tb, acc2[st]);
-            }
+        for (int st = 0; st < 3; ++st) {
+            const mf_v4d &D = st == 0 ? d0 : st == 1 ? d1 : d2;
+            const double s1 = Xl[xo + 16 * st] * Yl[yo + 16 * st];
+            const double s2 = Xl[xo + 16 * st + MF_SITES] * Yo[yo + 16 * st];
+            const double a = fma(sg, s2, s1), b = fma(-sg, s1, s2);
+            const double t = a * D[0];
+            ax[st] = fma(-cx, fma(b, D[1], t), ax[st]);
+            ay[st] = fma(-cy, fma(-b, D[1], t), ay[st]);
+            az[st] = fma(-b, D[3], fma(-a, D[2], az[st]));
         }
     }
 #pragma unroll
     for (int st = 0; st < 3; ++st) {
-        acc1[st] += __shfl_xor(acc1[st], 16, 64);
-        acc2[st] += __shfl_xor(acc2[st], 16, 64);
-        if (gq == 0) {
-            red[(w * 3 + 0) * MF_SITES + 16 * st + j] = acc1[st];
-            red[(w * 3 + 1) * MF_SITES + 16 * st + j] = acc2[st];
-        } else if (gq == 2) {
-            red[(w * 3 + 2) * MF_SITES + 16 * st + j] = acc1[st];
-        }
+        ax[st] += __shfl_xor(ax[st], 16, 64);
+        ay[st] += __shfl_xor(ay[st], 16, 64);
+        az[st] += __shfl_xor(az[st], 16, 64);
+        ax[st] += __shfl_xor(ax[st], 32, 64);
+        ay[st] += __shfl_xor(ay[st], 32, 64);
+        az[st] += __shfl_xor(az[st], 32, 64);
     }
-    if (lane < MF_SITES) {
-        rsm[(w * 3 + 0) * MF_SITES + lane] = rx;
-        rsm[(w * 3 + 1) * MF_SITES + lane] = ry;
-        rsm[(w * 3 + 2) * MF_SITES + lane] = rz;
+    if (lane < MF_SITES) {  // lane = 16 st + j, and its real-space slots
+        red[(w * 3 + 0) * MF_SITES + lane] = rx + (gq == 0 ? ax[0] : gq == 1 ? ax[1] : ax[2]);
+        red[(w * 3 + 1) * MF_SITES + lane] = ry + (gq == 0 ? ay[0] : gq == 1 ? ay[1] : ay[2]);
+        red[(w * 3 + 2) * MF_SITES + lane] = rz + (gq == 0 ? az[0] : gq == 1 ? az[1] : az[2]);
     }
     __syncthreads();
     const int d = threadIdx.x / MF_SITES, sj = threadIdx.x - d * MF_SITES;
     if (threadIdx.x < 3 * MF_SITES) {
-        double vr = 0.0, vk = 0.0;
+        double v = 0.0;
 #pragma unroll
-        for (int ww = 0; ww < W; ++ww) {
-            vr += rsm[(ww * 3 + d) * MF_SITES + sj];
-            vk += red[(ww * 3 + d) * MF_SITES + sj];
-        }
-        ef[d * MF_SITES + sj] = vr + vk;
+        for (int ww = 0; ww < W; ++ww) v += red[(ww * 3 + d) * MF_SITES + sj];
+        ef[d * MF_SITES + sj] = v;
     }
     __syncthreads();
     if (threadIdx.x < 3 * MF_SITES && a0 + sj < n_atoms) {
