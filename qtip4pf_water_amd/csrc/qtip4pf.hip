@@ -150,7 +150,7 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
             ctx->kforce_mf_lds_small = kforce_mf_lds_bytes(K, ctx->mf_nks, MF_WAVES_SMALL);
             ctx->ks_nslot = (int)ks_slot.size();
             ctx->ks_nslot_ph = (int)ks_slot_ph.size();
-            ctx->phase_lds = std::max(std::max(sizeof(RsLds<4>), sizeof(NlLds)),
+            ctx->phase_lds = std::max(std::max(sizeof(RsLds<4>), sizeof(NlRowLds)),
                                       ksum_mf_lds_bytes(K, PH_SUB));
             ctx->ksum_mf_lds = ksum_mf_lds_bytes(K, ctx->AC);
         }

@@ -179,6 +179,8 @@ static NlArgs nlist_args(const qtp_ctx *ctx, int force_all, bool with_heat, cons
     a.list = ctx->list;
     a.flist = ctx->flist;
     a.status = ctx->status;
+    a.bm = ctx->nl_bm;
+    a.cnt = ctx->cnt;
     a.heat = heat_args(ctx, with_heat);
     return a;
 }
@@ -274,8 +276,7 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
         if (ctx->lists_defer) {
             ctx->lists_defer = false;
             na = nlist_args(ctx, 0, ctx->lists_heat, ctx->lists_ctr);
-            na.keep_disp = 1;
-            n_nl = ctx->P + (ctx->lists_heat ? 1 : 0);
+            n_nl = ctx->P * ((ctx->n_mols + NL_ROWS - 1) / NL_ROWS) + (ctx->lists_heat ? 1 : 0);
         }
         const int n_ks = E * ncg * usplit, n_rs = E * ctx->ntile, n_lj = E * ctx->nmb;
         const bool early = n_lj <= PH_LJ_EARLY;

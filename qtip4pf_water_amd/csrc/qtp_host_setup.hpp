@@ -329,9 +329,13 @@ static int alloc_all(qtp_ctx *ctx)
         CHK(dalloc(ctx, &ctx->member, (size_t)P * ctx->n_mols));
         CHK(dalloc(ctx, &ctx->cell_pos, (size_t)P * ctx->n_mols));
         CHK(dalloc(ctx, &ctx->cstart, (size_t)P * (ctx->cg.ncell + 1)));
-        const size_t nbm = (size_t)P * ctx->n_mols * ((ctx->n_mols + 63) / 64);
-        if (nbm * sizeof(unsigned long long) <= NL_BM_MAX_BYTES) CHK(dalloc(ctx, &ctx->nl_bm, nbm));
     }
+    // row bitmaps: of the cell build, and of the one-stream phase's rebuild
+    // (at most 128 KiB a bead)
+    const size_t nbm = (size_t)P * ctx->n_mols * ((ctx->n_mols + 63) / 64);
+    if (ctx->n_mols <= NL_FUSED_MAXMOL ||
+        (ctx->cells_ok && nbm * sizeof(unsigned long long) <= NL_BM_MAX_BYTES))
+        CHK(dalloc(ctx, &ctx->nl_bm, nbm));
     CHK(dalloc(ctx, &ctx->flag, P));
     CHK(dalloc(ctx, &ctx->status, 1));
     CHK(dalloc(ctx, &ctx->nreb, P));

@@ -26,8 +26,8 @@ struct LjArgs {
     int ep_stride, ep_off;
     double *vpart;
 };
-// The evaluation that block `block` of nblocks works on, and whether it is the
-// evaluation's first block.
+// The evaluation that block `block` of nblocks works on, and which of the
+// evaluation's blocks it is.
 template <int LPM>
 __device__ __forceinline__ int lj_eval(int block, int nblocks, const LjArgs &A)
 {
@@ -35,10 +35,10 @@ __device__ __forceinline__ int lj_eval(int block, int nblocks, const LjArgs &A)
     return xcd_remap(block, nblocks) / ((A.n_mols + MPB - 1) / MPB);
 }
 template <int LPM>
-__device__ __forceinline__ bool lj_eval_first(int block, int nblocks, const LjArgs &A)
+__device__ __forceinline__ int lj_eval_block(int block, int nblocks, const LjArgs &A)
 {
     constexpr int MPB = 256 / LPM;
-    return xcd_remap(block, nblocks) % ((A.n_mols + MPB - 1) / MPB) == 0;
+    return xcd_remap(block, nblocks) % ((A.n_mols + MPB - 1) / MPB);
 }
 template <bool VIR, int LPM>
 __device__ __forceinline__ void lj_block(double *sh, int block, int nblocks, const LjArgs &A)

@@ -934,7 +934,8 @@ struct NlArgs {
     int *flag;
     double *nreb;
     int *point, *fpoint, *list, *flist, *status;
-    int keep_disp;  // leave a rebuilt bead's displacements for a later launch to zero
+    unsigned long long *bm;  // one-stream form: row bitmaps and counts of rebuilt beads
+    int *cnt;
     HeatArgs heat;
 };
 struct NlLds {
@@ -982,6 +983,18 @@ __device__ __forceinline__ int list_flag(double *s1, double *s2, int *flag, int 
     __syncthreads();
     return *flag;
 }
+// The heat sum of a thermostatted step, by the first wave of a block.
+__device__ __forceinline__ void list_heat(const HeatArgs &heat)
+{
+    if (threadIdx.x >= 64) return;
+    const double ke = wave_sum_array(heat.part, heat.ntile);
+    const double h = wave_sum_array(heat.hpart, heat.nh);
+    if (threadIdx.x == 0) {
+        const double ret = ke + h;
+        heat.heat_step[0] = ret;
+        heat.heat_acc[0] -= ret;
+    }
+}
 // Bead `block` of nblocks by NT threads.
 template <int NT>
 __device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, const NlArgs &A)
@@ -999,18 +1012,9 @@ __device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, co
     int *__restrict__ list = A.list;
     int *__restrict__ flist = A.flist;
     int *__restrict__ status = A.status;
-    const HeatArgs &heat = A.heat;
     const int b = block, tid = threadIdx.x;
-    if (heat.part && b == nblocks - 1) {  // the extra last block: the heat sum only
-        if (tid < 64) {
-            const double ke = wave_sum_array(heat.part, heat.ntile);
-            const double h = wave_sum_array(heat.hpart, heat.nh);
-            if (tid == 0) {
-                const double ret = ke + h;
-                heat.heat_step[0] = ret;
-                heat.heat_acc[0] -= ret;
-            }
-        }
+    if (A.heat.part && b == nblocks - 1) {  // the extra last block: the heat sum only
+        list_heat(A.heat);
         return;
     }
     double *D = disp + (long)b * 3 * NMP;
@@ -1082,8 +1086,7 @@ __device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, co
     int *L = list + (long)b * list_size;
     int *FL = flist + (long)b * fcap;
     for (int k = nh_tot + tid; k < list_size; k += NT) L[k] = 0;
-    if (!A.keep_disp)
-        for (int t = tid; t < 3 * NMP; t += NT) D[t] = 0.0;
+    for (int t = tid; t < 3 * NMP; t += NT) D[t] = 0.0;
     // --- fill
     for (int i = w; i < n_mols; i += NT / 64) {
         const double xi = Q[3 * i], yi = Q[NAP + 3 * i], zi = Q[2 * NAP + 3 * i];
@@ -1119,6 +1122,131 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(const NlArgs A)
     nlist_block<1024>(L, blockIdx.x, gridDim.x, A);
 }
 
+// The same rebuild in the launches of the one-stream phase, spread over the
+// chip: list_rows leaves a flagged bead's row bitmaps and counts, NL_ROWS rows
+// a block; list_fill, in the block of the next launch that needs the rows,
+// their offsets and entries.  A step that rebuilds lists took this much longer
+// with one block of 256 threads a bead: 2.4 ms at 990 molecules (k_nlist_bead,
+// 1024 threads: 1.4), 110 us at 216.  Now 21 and 13 us.
+constexpr int NL_ROWS = 64;
+struct NlRowLds {
+    double s1[4], s2[4];
+    int flag;
+};
+// grid share: P * ceil(n_mols / NL_ROWS) blocks of 256 threads, and one more
+// with a heat sum.
+__device__ __forceinline__ void list_rows(NlRowLds &S, int block, int nblocks, const NlArgs &A)
+{
+    if (A.heat.part && block == nblocks - 1) {
+        list_heat(A.heat);
+        return;
+    }
+    const int n = A.n_mols, NAP = A.NAP, nw = (n + 63) >> 6;
+    const int nsub = (n + NL_ROWS - 1) / NL_ROWS;
+    const int b = block / nsub, sub = block - b * nsub;
+    const int f = list_flag<256>(S.s1, S.s2, &S.flag, b, A);
+    if (sub == 0 && threadIdx.x == 0) {
+        A.flag[b] = f;
+        if (f && A.nreb) A.nreb[b] += 1.0;
+    }
+    if (!f) return;
+    const double *Q = A.q + (long)b * 3 * NAP;
+    const double Lx = A.box.L[0], Ly = A.box.L[1], Lz = A.box.L[2];
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // one row at a time: four that share their partners' loads raise the
+    // kernel's register use, and all its other roles slow down by 4 %
+    for (int i = sub * NL_ROWS + w; i < min(n, (sub + 1) * NL_ROWS); i += 4) {
+        const double x = Q[3 * i], y = Q[NAP + 3 * i], z = Q[2 * NAP + 3 * i];
+        unsigned long long word = 0ull;
+        int nh = 0, nf = 0;
+        for (int k = 0; k < nw; ++k) {
+            const int j = 64 * k + lane, jj = min(j, n - 1);
+            const double rx = mimg_exact(x - Q[3 * jj], Lx);
+            const double ry = mimg_exact(y - Q[NAP + 3 * jj], Ly);
+            const double rz = mimg_exact(z - Q[2 * NAP + 3 * jj], Lz);
+            const bool in = rx * rx + ry * ry + rz * rz < A.r_skin_sq && j < n && j != i;
+            const unsigned long long m = __ballot(in);
+            if (lane == k) word = m;
+            nf += __popcll(m);
+            nh += __popcll(__ballot(in && j > i));
+        }
+        if (lane < nw) A.bm[((long)b * n + i) * nw + lane] = word;
+        if (lane == 0) {
+            A.cnt[2L * b * n + i] = nh;
+            A.cnt[(2L * b + 1) * n + i] = nf;
+        }
+    }
+}
+// Rows m0 ... m0 + nrow - 1 of rebuilt bead b from the bitmaps: offsets,
+// entries and the bead's share part / nparts of the unused tail of its half
+// list.  256 threads; the block may read its rows afterwards.
+__device__ __forceinline__ void list_fill(int (*sh)[4], int b, int m0, int nrow, int part, int nparts,
+                                          const NlArgs &A)
+{
+    const int n = A.n_mols, nw = (n + 63) >> 6, tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int *ch = A.cnt + (2L * b) * n, *cf = ch + n;
+    // rows before m0 and all rows: half, full
+    int v[4] = {0, 0, 0, 0};
+    for (int i = tid; i < n; i += 256) {
+        const int h = ch[i], f = cf[i];
+        v[2] += h;
+        v[3] += f;
+        if (i < m0) {
+            v[0] += h;
+            v[1] += f;
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        for (int o = 32; o > 0; o >>= 1) v[k] += __shfl_xor(v[k], o, 64);
+        if (lane == 0) sh[w][k] = v[k];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = sh[0][k] + sh[1][k] + sh[2][k] + sh[3][k];
+    int *PT = A.point + (long)b * n, *FP = A.fpoint + (long)b * (n + 1);
+    int *L = A.list + (long)b * A.list_size, *FL = A.flist + (long)b * A.fcap;
+    const unsigned long long below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+    for (int r = w; r < nrow; r += 4) {
+        const int i = m0 + r;
+        // this row's offsets and, lane r, its counts
+        int h = lane <= r ? ch[m0 + lane] : 0, f = lane <= r ? cf[m0 + lane] : 0;
+        const int nhr = __shfl(h, r, 64), nfr = __shfl(f, r, 64);
+        for (int o = 32; o > 0; o >>= 1) {
+            h += __shfl_xor(h, o, 64);
+            f += __shfl_xor(f, o, 64);
+        }
+        int kh = v[0] + h - nhr;
+        long kf = v[1] + f - nfr;
+        if (lane == 0) {
+            PT[i] = kh;
+            FP[i] = (int)kf;
+            FP[i + 1] = (int)kf + nfr;  // the next row's block writes the same
+        }
+        const unsigned long long *bm = A.bm + ((long)b * n + i) * nw;
+        for (int k = 0; k < nw; ++k) {
+            const unsigned long long m = bm[k];
+            const unsigned long long mh =
+                64 * k > i ? m : 64 * k + 63 <= i ? 0ull : m & ~((2ull << (i & 63)) - 1ull);
+            if ((m >> lane) & 1ull) {
+                const long pos = kf + __popcll(m & below);
+                if (pos < A.fcap) FL[pos] = 64 * k + lane;
+            }
+            if ((mh >> lane) & 1ull) {
+                const int pos = kh + __popcll(mh & below);
+                if (pos < A.list_size) L[pos] = 64 * k + lane;
+            }
+            kf += __popcll(m);
+            kh += __popcll(mh);
+        }
+    }
+    for (int k = v[2] + part * 256 + tid; k < A.list_size; k += nparts * 256) L[k] = 0;
+    if (part == 0 && tid == 0 && (v[2] > A.list_size || (long)v[3] > A.fcap)) atomicOr(A.status, 1);
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // A force phase in three launches on one stream (the third is k_kforce_mf).
 // With the k-space and LJ kernels on a second stream a phase spent 5 us on the
@@ -1138,8 +1266,8 @@ __global__ __launch_bounds__(1024) void k_nlist_bead(const NlArgs A)
 // blocks otherwise (512 x 32 409 against 418).
 // The LJ blocks here of a step's first phase (n_nl > 0) test their bead's
 // displacements themselves: a bead whose lists this launch rebuilds is left to
-// k_phase_reduce, which also zeroes its displacements (nothing may change
-// them while both roles read them).
+// k_phase_reduce, which also fills the lists and zeroes the displacements
+// (nothing may change them while both roles read them).
 constexpr int PH_CAP = 2;   // k_ksum_mf's CAP here: few accumulators, so that six
                             // waves fit a SIMD (four: 512 x 32 469 us a step)
 constexpr int PH_SUB = 32;  // sites whose factor tables are staged at a time: about
@@ -1162,7 +1290,7 @@ __global__ __launch_bounds__(256, 6) void k_phase_pairs(const RsArgs rs, const K
     extern __shared__ double smem[];
     int b = blockIdx.x;
     if (b < n_nl) {
-        nlist_block<256>(*(NlLds *)smem, b, n_nl, nl);
+        list_rows(*(NlRowLds *)smem, b, n_nl, nl);
         return;
     }
     b -= n_nl;
@@ -1183,7 +1311,8 @@ __global__ __launch_bounds__(256, 6) void k_phase_pairs(const RsArgs rs, const K
 }
 // Second launch, 256 threads: n_lj blocks for the LJ and intramolecular terms,
 // of every bead or (rebuilt_only) of the beads whose lists the first launch
-// rebuilt; the rest: reduction of the structure factors.  n_nl > 0: a step's
+// rebuilt, whose rows it fills first; the rest: reduction of the structure
+// factors.  n_nl > 0: a step's
 // first phase, whose rebuilt beads' displacements are zeroed here.
 template <bool VIR, int LPM>
 __global__ __launch_bounds__(256) void k_phase_reduce(const SrArgs sr, const LjArgs lj, const NlArgs nl,
@@ -1195,10 +1324,14 @@ __global__ __launch_bounds__(256) void k_phase_reduce(const SrArgs sr, const LjA
         sreduce_block(sh, b - n_lj, sr);
         return;
     }
-    const int e = lj_eval<LPM>(b, n_lj, lj);
+    __shared__ int cs[4][4];
+    constexpr int MPB = 256 / LPM;
+    const int e = lj_eval<LPM>(b, n_lj, lj), mb = lj_eval_block<LPM>(b, n_lj, lj);
     const bool rebuilt = n_nl > 0 && nl.flag[e];
+    if (rebuilt)
+        list_fill(cs, e, mb * MPB, min(MPB, lj.n_mols - mb * MPB), mb, (lj.n_mols + MPB - 1) / MPB, nl);
     if (rebuilt || !rebuilt_only) lj_block<VIR, LPM>(sh, b, n_lj, lj);
-    if (rebuilt && lj_eval_first<LPM>(b, n_lj, lj))
+    if (rebuilt && mb == 0)
         for (int t = threadIdx.x; t < 3 * nl.NMP; t += 256) nl.disp[(long)e * 3 * nl.NMP + t] = 0.0;
 }
 

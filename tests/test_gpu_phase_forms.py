@@ -89,3 +89,32 @@ def test_one_stream_form_is_bitwise_the_kernels_one_by_one(nside, P, thermo):
     assert all(np.array_equal(x, y) for x, y in zip(a[1], b[1]))
     assert a[2] == b[2]
     assert all(np.array_equal(x, y) for x, y in zip(a[3], b[3]))
+
+
+@pytest.mark.parametrize("nside,P", [
+    ((4, 4, 4), 4), ((4, 4, 5), 2), ((8, 8, 8), 1), ((8, 9, 9), 2), ((9, 10, 11), 2), ((8, 8, 16), 1)])
+def test_spread_rebuild_is_the_one_block_rebuild(nside, P):
+    """Lists rebuilt inside the one-stream phase (bitmaps, then offsets and
+    rows, over many blocks) against k_nlist_bead's: rows up to the largest
+    molecule count, whole and ragged words and blocks of rows."""
+    from qtip4pf_water_amd import Water
+    q0, box, L = _box(nside, 21)
+    n = q0.size // 9
+    beta_n = 1.0 / (cfg.K2AU * 298.0) / P
+    q = cfg.free_ring_polymer_beads(q0, P, beta_n, seed=22) if P > 1 else q0
+    p = cfg.sample_momenta(n, P, beta_n, seed=23)
+    out = []
+    for timing in (False, True):
+        with Water(n, P, box, lj_rcut=cfg.lj_rcut_for(min(L))) as w:
+            w.set_lists("allpairs", 2)
+            w.set_tuning(rs_registers=1)
+            w.set_seed(3)
+            w.enable_timing(timing)
+            w.set_state(q, p)
+            w.run(5)
+            s = w.scalars()
+            assert s["status"] == 0 and s["rebuilds"] == 2 * P
+            out.append((w.get_lists(), w.get_state()))
+    a, b = out
+    for x, y in zip(a[0] + a[1], b[0] + b[1]):
+        assert np.array_equal(x, y)
