@@ -113,8 +113,10 @@ def test_spread_rebuild_is_the_one_block_rebuild(nside, P):
             w.set_state(q, p)
             w.run(5)
             s = w.scalars()
-            assert s["status"] == 0 and s["rebuilds"] == 2 * P
-            out.append((w.get_lists(), w.get_state()))
+            # every second step, and where the beads moved far enough
+            assert s["status"] == 0 and s["rebuilds"] >= 2 * P
+            out.append((w.get_lists(), w.get_state(), s))
     a, b = out
+    assert a[2] == b[2]
     for x, y in zip(a[0] + a[1], b[0] + b[1]):
         assert np.array_equal(x, y)
