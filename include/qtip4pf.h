@@ -321,7 +321,7 @@ int qtp_run_observed(qtp_ctx *ctx, int n_steps, int is_nvt, int every, double *t
  * propagation as one LDS-staged kernel per step where the thermostat allows
  * it: for systems of 256 or more 64-dof tiles (-1), always (1), never (0;
  * the results are the same bit for bit), waves per real-space tile block (2
- * or 4), eighths of the real-space tiles launched on the second stream after
+ * or 4; no effect in boxes so wide that tiles are skipped), eighths of the real-space tiles launched on the second stream after
  * the LJ/intramolecular kernel (0-4), site chunks per structure-factor block
  * of the matrix-core path (1, 2, 4, 8, 16; 0 by launch size)}.
  * Every configuration gives the same forces up to summation order. */

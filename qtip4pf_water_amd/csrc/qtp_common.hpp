@@ -167,38 +167,33 @@ __device__ __forceinline__ double eval_energy(const double *__restrict__ epart, 
 }
 
 // Coefficients of the real-space special functions: the erfcx rational and
-// the e^r Taylor series (e[k] = 1/k!).  As literals (LitCoef) they sit in
-// VGPRs across the pair loop; passed as a kernel argument (RsCoef) they are
-// loaded into SGPRs, which frees about 40 VGPRs (more waves per SIMD).
+// e^r on |r| <= ln2/2 (1 + r + r^2/2 + r^3 g(r), g interpolated at the ten
+// Chebyshev points: error 1e-18; Taylor's series to degree 13, a term longer,
+// had 5e-18).  As literals (LitCoef) they sit in VGPRs across the pair loop;
+// read from RS_COEF by scalar loads they take SGPRs, which frees about 40
+// VGPRs (more waves per SIMD).
+#define QTP_EXP_E                                                                                  \
+    1.0, 1.0, 0.5, 0.16666666666666669, 0.041666666666666664, 0.008333333333330065,               \
+        0.0013888888888886554, 0.00019841269863040559, 2.4801587317135174e-05,                     \
+        2.7557268480289716e-06, 2.755728298404137e-07, 2.51003758422237e-08, 2.091122973665872e-09
+constexpr int EXP_DEG = 12;
 struct RsCoef {
-    double p[QTP_ERFCX_DEG + 1], q[QTP_ERFCX_DEG + 1], e[14];
+    double p[QTP_ERFCX_DEG + 1], q[QTP_ERFCX_DEG + 1], e[EXP_DEG + 1];
 };
 struct LitCoef {
     static constexpr double p[QTP_ERFCX_DEG + 1] = {QTP_ERFCX_P};
     static constexpr double q[QTP_ERFCX_DEG + 1] = {QTP_ERFCX_Q};
-    static constexpr double e[14] = {1.0, 1.0, 0.5, 1.0 / 6.0, 1.0 / 24.0, 1.0 / 120.0,
-                                     1.0 / 720.0, 1.0 / 5040.0, 1.0 / 40320.0, 1.0 / 362880.0,
-                                     1.0 / 3628800.0, 1.0 / 39916800.0, 1.0 / 479001600.0,
-                                     1.0 / 6227020800.0};
+    static constexpr double e[EXP_DEG + 1] = {QTP_EXP_E};
 };
-// the argument form, filled on the host with the same values
-inline RsCoef rs_coef()
-{
-    RsCoef c;
-    for (int k = 0; k <= QTP_ERFCX_DEG; ++k) {
-        c.p[k] = LitCoef::p[k];
-        c.q[k] = LitCoef::q[k];
-    }
-    for (int k = 0; k < 14; ++k) c.e[k] = LitCoef::e[k];
-    return c;
-}
+__constant__ RsCoef RS_COEF = {{QTP_ERFCX_P}, {QTP_ERFCX_Q}, {QTP_EXP_E}};
 
 // erfc(x) = exp(-x^2) erfcx(x) with erfcx from the P8/Q8 rational of
 // qtp_erfcx.h (relative error < 9e-16 on [0, 6.2]; the host guarantees
 // kappa * r_c <= 6.2, so every in-cutoff pair is in range).  ex = exp(-x^2)
 // is passed in (the force needs it too).  The quotient uses the hardware
-// reciprocal refined by two Newton steps and one residual correction
-// (Q >= 1 on the range: no scaling cases).
+// reciprocal (relative error below 2^-22) refined by one Newton step, to
+// 2^-44, and one residual correction, which leaves only the rounding (Q >= 1
+// on the range: no scaling cases).
 template <class C>
 __device__ __forceinline__ double erfc_via_erfcx(double x, double ex, const C &c)
 {
@@ -209,7 +204,6 @@ __device__ __forceinline__ double erfc_via_erfcx(double x, double ex, const C &c
         q = fma(q, x, c.q[k]);
     }
     double r = __builtin_amdgcn_rcp(q);
-    r = fma(fma(-q, r, 1.0), r, r);
     r = fma(fma(-q, r, 1.0), r, r);
     double y = p * r;
     y = fma(fma(-q, y, p), r, y);
@@ -229,8 +223,8 @@ __device__ __forceinline__ double rsqrt_pos(double x)
 // e^x for -708 <= x <= 0 (no overflow, no subnormal results in the range the
 // real-space kernel uses, x >= -(kappa r_c)^2 >= -38.5): Cody-Waite reduction
 // x = n ln2 + r, |r| <= ln2/2, with ln2 split as hi (its first 32 significant
-// bits, so n hi is exact) + lo; e^r by its Taylor series to degree 13
-// (truncation below 5e-18); then 2^n.  Under one ulp over [-40, 0].
+// bits, so n hi is exact) + lo; e^r by the polynomial c.e; then 2^n.  Under
+// one ulp over [-40, 0].
 template <class C>
 __device__ __forceinline__ double exp_nonpos(double x, const C &c)
 {
@@ -240,9 +234,9 @@ __device__ __forceinline__ double exp_nonpos(double x, const C &c)
     const double n = rint(x * L2E);
     double r = fma(-n, LN2_HI, x);
     r = fma(-n, LN2_LO, r);
-    double p = c.e[13];
+    double p = c.e[EXP_DEG];
 #pragma unroll
-    for (int k = 12; k >= 0; --k) p = fma(p, r, c.e[k]);
+    for (int k = EXP_DEG - 1; k >= 0; --k) p = fma(p, r, c.e[k]);
     return ldexp(p, (int)n);
 }
 

@@ -65,7 +65,6 @@ static RsArgs rs_args(const qtp_ctx *ctx, const double *pos, double *vp)
     a.ep_stride = ctx->ep_stride;
     a.ep_off = ctx->ep_real;
     a.vpart = vp;
-    a.cf = rs_coef();
     a.sites = ctx->rs_sites;
     a.bbox = ctx->rs_box;
     a.rfar = ctx->rs_far;
@@ -229,24 +228,30 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
         TimeScope ts(ctx, "realspace");
         ra.t0 = t0;
         ra.nt = nt;
-#define QTP_RS_LAUNCH_W(VIR, CARG, CULL, W) k_realspace<VIR, CARG, CULL, W><<<E * nt, 64 * W, 0, st>>>(ra)
-#define QTP_RS_LAUNCH(VIR, CARG, CULL)                                                             \
+#define QTP_RS_LAUNCH(VIR, CARG)                                                                   \
     do {                                                                                           \
-        if (ctx->rs_waves == 2) QTP_RS_LAUNCH_W(VIR, CARG, CULL, 2);                              \
-        else QTP_RS_LAUNCH_W(VIR, CARG, CULL, 4);                                                  \
+        if (ctx->rs_waves == 2) k_realspace<VIR, CARG, 2><<<E * nt, 128, 0, st>>>(ra);             \
+        else k_realspace<VIR, CARG, 4><<<E * nt, 256, 0, st>>>(ra);                                \
     } while (0)
         if (ctx->rs_cull) {
-            if (vout) QTP_RS_LAUNCH(true, true, true);
-            else QTP_RS_LAUNCH(false, true, true);
+            // tiles a block, while the blocks fill the chip several times over
+            ra.gs = (int)std::min(16L, std::max(1L, (long)E * nt / RS_CULL_WAVES));
+            const int grid = E * ((nt + ra.gs - 1) / ra.gs);
+            if (ra.fx.cubic) {
+                if (vout) k_realspace_cull<true, true><<<grid, 64 * RS_CW, 0, st>>>(ra);
+                else k_realspace_cull<false, true><<<grid, 64 * RS_CW, 0, st>>>(ra);
+            } else {
+                if (vout) k_realspace_cull<true, false><<<grid, 64 * RS_CW, 0, st>>>(ra);
+                else k_realspace_cull<false, false><<<grid, 64 * RS_CW, 0, st>>>(ra);
+            }
         } else if (vout) {
-            if (carg) QTP_RS_LAUNCH(true, true, false);
-            else QTP_RS_LAUNCH(true, false, false);
+            if (carg) QTP_RS_LAUNCH(true, true);
+            else QTP_RS_LAUNCH(true, false);
         } else {
-            if (carg) QTP_RS_LAUNCH(false, true, false);
-            else QTP_RS_LAUNCH(false, false, false);
+            if (carg) QTP_RS_LAUNCH(false, true);
+            else QTP_RS_LAUNCH(false, false);
         }
 #undef QTP_RS_LAUNCH
-#undef QTP_RS_LAUNCH_W
     };
     // the culling form's site tables and skip flags, ahead of the fork: on
     // their own the two small kernels take a few microseconds, behind the

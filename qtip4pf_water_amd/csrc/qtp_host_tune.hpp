@@ -149,7 +149,8 @@ std::vector<TuneCfg> tune_candidates(const qtp_ctx *ctx)
 {
     std::vector<TuneCfg> out;
     const int umax = std::min(4, std::max(1, ctx->ks_nslot / ((ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES)));
-    for (int rsw : {4, 2})
+    // (tile-culling boxes: k_realspace_cull, neither of the two has an effect)
+    for (int rsw : ctx->rs_cull ? std::vector<int>{RS_WAVES} : std::vector<int>{4, 2})
         for (int lpm : {16, 64})
             for (int kmf = ctx->kf_mf_ok ? 1 : 0; kmf >= 0; --kmf)
                 for (int carg : ctx->rs_cull ? std::vector<int>{-1} : std::vector<int>{0, 1}) {

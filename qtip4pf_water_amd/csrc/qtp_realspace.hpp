@@ -31,25 +31,14 @@ namespace qtp {
 // slots and partials).
 // VIR: also accumulate the pair virial r_ij (x) f_ij (6 components) into
 // vpart[(e*6 + c)*ep_stride + ep_off + tile].
-// CARG: the special functions' coefficients come from the argument cf (SGPRs)
-// instead of literals (VGPRs); the host picks it for large grids.
-// CULL: the sites come from k_sites (x, y, z, q per site and bounding boxes
-// per 64-site block and per 8-site cluster).  A tile whose two blocks' boxes
-// are more than r_c apart under every periodic image holds no pair within the
-// cutoff: k_tilefar marks it in rfar[e * ntile + tile] and zeroes its energy
-// partial, and its block here returns after reading the flag, writing no slot
-// entries (k_kforce_mf and k_kforce read none of a tile so marked).  In the
-// other tiles the cutoff test runs only over pairs of clusters whose boxes
-// lie within r_c (4096 H2O, r_c 9 A: a third of the cluster pairs of the near
-// tiles), one lane per site pair.  The same pairs are evaluated either way.
-// The host picks it for boxes several r_c wide, where most tiles are far
-// (4096 H2O, r_c 9 A: 76% of the tiles, sites in molecule order).
+// CARG: the special functions' coefficients come from RS_COEF (SGPRs) instead
+// of literals (VGPRs); the host picks it for large grids.
 // W: two waves per tile halve the block and double each lane's share of the
 // queue; a launch then holds fewer waves (216 H2O x 32 beads: 4224, which
 // the chip holds at once, against 8448 in two rounds with four).
 constexpr int RS_WAVES = 4;  // the default W
 constexpr long RS_CARG_BLOCKS = 16384;  // grids at least this large use CARG
-// boxes at least this many r_c wide use CULL.  x 32 beads, steps/s of the
+// boxes at least this many r_c wide use k_realspace_cull.  x 32 beads, steps/s of the
 // first culling form (block boxes only, zeroed slots) against the plain one
 // at the reference's Ewald point: 216 H2O (2.06 r_c) -8%, 1000 (2.66) +7%,
 // 1728 (2.91) +7%, 4096 (3.36) +21%
@@ -137,8 +126,8 @@ constexpr int RS_BOX = 6 + 6 * 8;
 
 // Sites of each 64-site block as (x, y, z, q) (M from O, H, H; forces.cpp:
 // 558-564), the block's bounding box and those of its 8-site clusters
-// (RS_BOX layout), for the CULL form of k_realspace.  A cluster holding no
-// site gets an empty box (lo > hi); k_realspace never tests one.
+// (RS_BOX layout), for k_realspace_cull.  A cluster holding no
+// site gets an empty box (lo > hi); k_realspace_cull never tests one.
 // grid: E * nblk, 64 threads.
 __global__ __launch_bounds__(64) void k_sites(const double *__restrict__ pos, long pstride,
                                               const double *__restrict__ charge, int n_atoms,
@@ -187,7 +176,7 @@ __global__ __launch_bounds__(64) void k_sites(const double *__restrict__ pos, lo
 // Skip flags of the CULL form, one thread per (evaluation, tile): tile (I, J)
 // is skipped (rfar = 1) when its two blocks' boxes are more than r_c apart
 // under every periodic image; its energy partial (and virial partials, when
-// vpart is given) are zeroed here, so its k_realspace block only reads the
+// vpart is given) are zeroed here, so k_realspace_cull only reads the
 // flag.  grid: ceil(E * ntile / 256), 256 threads.
 __global__ __launch_bounds__(256) void k_tilefar(const int2 *__restrict__ tiles, int ntile, int nblk,
                                                 int E, const double *__restrict__ bbox, Box box,
@@ -241,12 +230,12 @@ struct RsArgs {
     double gamma, half1mg;
     const int2 *tiles;
     int ntile, t0, nt;
+    int gs;  // k_realspace_cull: tiles a wave
     Box box;
     Ewald ew;
     double *rpart, *epart;
     int ep_stride, ep_off;
     double *vpart;
-    RsCoef cf;
     const double4 *sites;
     const double *bbox;
     const unsigned char *rfar;
@@ -254,149 +243,34 @@ struct RsArgs {
 };
 
 // The tile of block `block` of nblocks (XCD-remapped), by its 64 W threads.
-template <bool VIR, bool CARG, bool CULL, int W>
-__device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, const RsArgs &A)
+// Pass 2 over the queue entries q0 ... q1 - 1 of this lane: rows il (site i0 +
+// il) and columns jl (site j0 + jl; coordinates sJ[jl], reaction fj[.][jo +
+// jl]).  Adds to fi, fj, the energy and (VIR) the virial.  near: the tile may
+// hold pairs of one molecule.
+template <bool VIR, bool CARG>
+__device__ __forceinline__ void rs_pairs(const double4 *sI, const double4 *sJ, double (*fi)[64],
+                                         double (*fj)[64], int jo, const unsigned short *qe, int q0,
+                                         int q1, bool near, int i0, int j0, const RsArgs &A, double &en,
+                                         double (&v6)[6])
 {
-    static_assert(W == 2 || W == 4, "two or four waves per tile");
-    constexpr int CPW = 64 / W;  // columns per wave
-    const int n_atoms = A.n_atoms, NAP = A.NAP, nblk = A.nblk, ntile = A.ntile, t0 = A.t0, nt = A.nt;
-    const int ep_stride = A.ep_stride, ep_off = A.ep_off;
-    const double gamma = A.gamma, half1mg = A.half1mg;
     const Box &box = A.box;
     const Ewald &ew = A.ew;
-    const RsCoef &cf = A.cf;
-    const RsFix &fx = A.fx;
-    const double *__restrict__ charge = A.charge;
-    const double4 *__restrict__ sites = A.sites;
-    const double *__restrict__ bbox = A.bbox;
-    double *__restrict__ rpart = A.rpart;
-    double *__restrict__ epart = A.epart;
-    double *__restrict__ vpart = A.vpart;
-    auto &sI = L.sI;
-    auto &sJ = L.sJ;
-    auto &uJ = L.uJ;
-    auto &uI = L.uI;
-    auto &fj = L.fj;
-    auto &fi = L.fi;
-    auto &qe = L.qe;
-    auto &ewv = L.ewv;
-    auto &wv = L.wv;
-    const int bid = xcd_remap(block, nblocks);
-    const int e = bid / nt, t = t0 + (bid - e * nt);
-    // a tile k_tilefar skipped (its partials zeroed there)
-    if (CULL && A.rfar[(long)e * ntile + t]) return;
-    const int I = A.tiles[t].x, J = A.tiles[t].y;
-    const int l = threadIdx.x & 63;
-    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const double *X = A.pos + (long)e * A.pstride;
-    const long base_e = (long)e * nblk * 3 * NAP;
-    // CULL: the live 8 x 8 cluster pairs of the wave's columns, from the
-    // cluster boxes alone, so their loads overlap the staging of the sites:
-    // lane l tests row cluster l & 7 against column cluster l >> 3 (boxes
-    // more than r_c apart under every image hold no pair within the cutoff)
-    unsigned long long todo = 0ull;
-    if constexpr (CULL) {
-        const int ci = l & 7, cj = l >> 3;
-        const double *cI = bbox + ((long)e * nblk + I) * RS_BOX + 6;
-        const double *cJ = bbox + ((long)e * nblk + J) * RS_BOX + 6;
-        double gsq = 0.0;
-        for (int d = 0; d < 3; ++d) {
-            const double g = periodic_gap(cI[8 * d + ci], cI[8 * (3 + d) + ci], cJ[8 * d + cj],
-                                          cJ[8 * (3 + d) + cj], box.L[d], box.inv[d]);
-            gsq = fma(g, g, gsq);
-        }
-        const bool live = gsq <= ew.rcut_sq * (1.0 + 1e-9) && I * 64 + 8 * ci < n_atoms &&
-                          J * 64 + 8 * cj < n_atoms && (I != J || cj >= ci);
-        todo = __ballot(live) & (((CPW == 64 ? 0ull : 1ull << CPW) - 1ull) << (CPW * w));
-    }
-    if (w < 2) {
-        const int s = (w == 0 ? J : I) * 64 + l;
-        double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
-        if (CULL)
-            v = sites[(long)e * nblk * 64 + s];
-        else if (s < n_atoms)
-            v = make_double4(site_coord(X, NAP, s, 0, gamma, half1mg),
-                             site_coord(X, NAP, s, 1, gamma, half1mg),
-                             site_coord(X, NAP, s, 2, gamma, half1mg), charge[s]);
-        (w == 0 ? sJ : sI)[l] = v;
-        uint4 *us = w == 0 ? uJ : uI;
-        const uint4 u = rs_fixed(v.x, v.y, v.z, box, fx.cubic);
-        if (fx.cubic)
-            ((uint2 *)us)[l] = make_uint2(u.x, u.y);
-        else
-            us[l] = u;
-        if (w == 0) {
-            fj[0][l] = 0.0;
-            fj[1][l] = 0.0;
-            fj[2][l] = 0.0;
-        }
-    }
-    fi[w][0][l] = 0.0;
-    fi[w][1][l] = 0.0;
-    fi[w][2][l] = 0.0;
-    __syncthreads();
-    const int c0 = CPW * w;
-    int total = 0;
-    // append the pairs of `in` (one per lane) to the wave's queue
-    auto push = [&](unsigned long long bal, int il, int c) {
-        if ((bal >> l) & 1ull) {
-            const int r = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
-                                                    __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
-            qe[w][total + r] = (unsigned short)(il | (c << 6));
-        }
-        total += __popcll(bal);
-    };
-    if constexpr (CULL) {
-        // pass 1 over the live cluster pairs: each one's 64 site pairs take
-        // one lane each; the queue holds a cluster pair's entries by column,
-        // rows within a column
-        while (todo) {
-            const int bit = __builtin_ctzll(todo);
-            todo &= todo - 1ull;
-            const int il = 8 * (bit & 7) + (l & 7);
-            const int jl = 8 * (bit >> 3) + (l >> 3);
-            const bool close = fx.cubic ? rs_near16(((const uint2 *)uI)[il], ((const uint2 *)uJ)[jl], fx.r2u)
-                                        : rs_near32(uI[il], uJ[jl], fx);
-            const int ii = I * 64 + il, j = J * 64 + jl;
-            push(__ballot(close && j > ii && j < n_atoms), il, jl - c0);
-        }
-    } else {
-        // pass 1, column by column: rows that exist, j > i in diagonal tiles
-        const int nrow = min(64, n_atoms - I * 64), ncol = n_atoms - J * 64;
-        const unsigned long long rows = nrow == 64 ? ~0ull : (1ull << nrow) - 1ull;
-        auto keep = [&](unsigned long long bal, int jl) {
-            if (I == J) bal &= (1ull << jl) - 1ull;
-            return jl < ncol ? bal & rows : 0ull;
-        };
-        if (fx.cubic) {
-            const uint2 a = ((const uint2 *)uI)[l];
-#pragma unroll
-            for (int c = 0; c < CPW; ++c)
-                push(keep(__ballot(rs_near16(a, ((const uint2 *)uJ)[c0 + c], fx.r2u)), c0 + c), l, c);
-        } else {
-            const uint4 a = uI[l];
-#pragma unroll
-            for (int c = 0; c < CPW; ++c)
-                push(keep(__ballot(rs_near32(a, uJ[c0 + c], fx)), c0 + c), l, c);
-        }
-    }
-    __syncthreads();
-    // pass 2: lane l takes queue entries [l*S, l*S + S)
-    const bool near = J - I <= 1;
-    const int S = (total + 63) >> 6;
-    const int q0 = min(l * S, total), q1 = min(q0 + S, total);
-    double gx = 0.0, gy = 0.0, gz = 0.0, en = 0.0;
-    double vxx = 0.0, vyy = 0.0, vzz = 0.0, vxy = 0.0, vxz = 0.0, vyz = 0.0;
+    // at an offset the compiler cannot see through: loaded here, not held
+    // in scalar registers by the code around
+    int o = 0;
+    asm volatile("" : "+s"(o));
+    const RsCoef &cf = *(const RsCoef *)((const char *)&RS_COEF + o);
+    double gx = 0.0, gy = 0.0, gz = 0.0;
     int jcur = -1;
     double4 b = make_double4(0.0, 0.0, 0.0, 0.0);
     for (int q = q0; q < q1; ++q) {
-        const int ent = qe[w][q];
-        const int il = ent & 63, jl = c0 + (ent >> 6);
+        const int ent = qe[q];
+        const int il = ent & 63, jl = ent >> 6;
         if (jl != jcur) {
             if (jcur >= 0) {
-                atomicAdd(&fj[0][jcur], gx);
-                atomicAdd(&fj[1][jcur], gy);
-                atomicAdd(&fj[2][jcur], gz);
+                atomicAdd(&fj[0][jo + jcur], gx);
+                atomicAdd(&fj[1][jo + jcur], gy);
+                atomicAdd(&fj[2][jo + jcur], gz);
             }
             gx = gy = gz = 0.0;
             jcur = jl;
@@ -428,7 +302,7 @@ __device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, con
         }
         // same molecule: -erf (forces.cpp:158-166); a molecule's three sites
         // lie in one 64-site block or two consecutive ones
-        if (near && (I * 64 + il) / 3 == (J * 64 + jl) / 3) ec -= 1.0;
+        if (near && (i0 + il) / 3 == (j0 + jl) / 3) ec -= 1.0;
         const double ep = qq * rinv * ec;
         const double pf = (ep + qq * ew.pref2k * ex) * (rinv * rinv);
         en += ep;
@@ -436,26 +310,113 @@ __device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, con
         gy = fma(-pf, dy, gy);
         gz = fma(-pf, dz, gz);
         if (VIR) {
-            vxx = fma(pf * dx, dx, vxx);
-            vyy = fma(pf * dy, dy, vyy);
-            vzz = fma(pf * dz, dz, vzz);
-            vxy = fma(pf * dx, dy, vxy);
-            vxz = fma(pf * dx, dz, vxz);
-            vyz = fma(pf * dy, dz, vyz);
+            v6[0] = fma(pf * dx, dx, v6[0]);
+            v6[1] = fma(pf * dy, dy, v6[1]);
+            v6[2] = fma(pf * dz, dz, v6[2]);
+            v6[3] = fma(pf * dx, dy, v6[3]);
+            v6[4] = fma(pf * dx, dz, v6[4]);
+            v6[5] = fma(pf * dy, dz, v6[5]);
         }
-        atomicAdd(&fi[w][0][il], pf * dx);
-        atomicAdd(&fi[w][1][il], pf * dy);
-        atomicAdd(&fi[w][2][il], pf * dz);
+        atomicAdd(&fi[0][il], pf * dx);
+        atomicAdd(&fi[1][il], pf * dy);
+        atomicAdd(&fi[2][il], pf * dz);
     }
     if (jcur >= 0) {
-        atomicAdd(&fj[0][jcur], gx);
-        atomicAdd(&fj[1][jcur], gy);
-        atomicAdd(&fj[2][jcur], gz);
+        atomicAdd(&fj[0][jo + jcur], gx);
+        atomicAdd(&fj[1][jo + jcur], gy);
+        atomicAdd(&fj[2][jo + jcur], gz);
     }
+}
+
+template <bool VIR, bool CARG, int W>
+__device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, const RsArgs &A)
+{
+    static_assert(W == 2 || W == 4, "two or four waves per tile");
+    constexpr int CPW = 64 / W;  // columns per wave
+    const int n_atoms = A.n_atoms, NAP = A.NAP, nblk = A.nblk, ntile = A.ntile, t0 = A.t0, nt = A.nt;
+    const int ep_stride = A.ep_stride, ep_off = A.ep_off;
+    const double gamma = A.gamma, half1mg = A.half1mg;
+    const Box &box = A.box;
+    const Ewald &ew = A.ew;
+    const RsFix &fx = A.fx;
+    const double *__restrict__ charge = A.charge;
+    double *__restrict__ rpart = A.rpart;
+    double *__restrict__ epart = A.epart;
+    double *__restrict__ vpart = A.vpart;
+    auto &sI = L.sI;
+    auto &sJ = L.sJ;
+    auto &uJ = L.uJ;
+    auto &uI = L.uI;
+    auto &fj = L.fj;
+    auto &fi = L.fi;
+    auto &qe = L.qe;
+    auto &ewv = L.ewv;
+    auto &wv = L.wv;
+    const int bid = xcd_remap(block, nblocks);
+    const int e = bid / nt, t = t0 + (bid - e * nt);
+    const int I = A.tiles[t].x, J = A.tiles[t].y;
+    const int l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const double *X = A.pos + (long)e * A.pstride;
+    const long base_e = (long)e * nblk * 3 * NAP;
+    if (w < 2) {
+        const int s = (w == 0 ? J : I) * 64 + l;
+        double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (s < n_atoms)
+            v = make_double4(site_coord(X, NAP, s, 0, gamma, half1mg),
+                             site_coord(X, NAP, s, 1, gamma, half1mg),
+                             site_coord(X, NAP, s, 2, gamma, half1mg), charge[s]);
+        (w == 0 ? sJ : sI)[l] = v;
+        uint4 *us = w == 0 ? uJ : uI;
+        const uint4 u = rs_fixed(v.x, v.y, v.z, box, fx.cubic);
+        if (fx.cubic)
+            ((uint2 *)us)[l] = make_uint2(u.x, u.y);
+        else
+            us[l] = u;
+        if (w == 0) {
+            fj[0][l] = 0.0;
+            fj[1][l] = 0.0;
+            fj[2][l] = 0.0;
+        }
+    }
+    fi[w][0][l] = 0.0;
+    fi[w][1][l] = 0.0;
+    fi[w][2][l] = 0.0;
+    __syncthreads();
+    const int c0 = CPW * w;
+    int total = 0;
+    // append column c's pairs to the wave's queue; pass 1, column by column:
+    // rows that exist, j > i in diagonal tiles
+    const int nrow = min(64, n_atoms - I * 64), ncol = n_atoms - J * 64;
+    auto push = [&](bool close, int c) {
+        const int lim = c0 + c >= ncol ? 0 : I == J ? min(nrow, c0 + c) : nrow;
+        const bool in = close && l < lim;
+        const unsigned long long bal = __ballot(in);
+        if (in) {
+            const int r = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                                    __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+            qe[w][total + r] = (unsigned short)(l | (c << 6));
+        }
+        total += __popcll(bal);
+    };
+    if (fx.cubic) {
+        const uint2 a = ((const uint2 *)uI)[l];
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) push(rs_near16(a, ((const uint2 *)uJ)[c0 + c], fx.r2u), c);
+    } else {
+        const uint4 a = uI[l];
+#pragma unroll
+        for (int c = 0; c < CPW; ++c) push(rs_near32(a, uJ[c0 + c], fx), c);
+    }
+    __syncthreads();
+    // pass 2: lane l takes queue entries [l*S, l*S + S)
+    const int S = (total + 63) >> 6;
+    const int q0 = min(l * S, total), q1 = min(q0 + S, total);
+    double en = 0.0, v6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    rs_pairs<VIR, CARG>(sI, sJ + c0, fi[w], fj, c0, qe[w], q0, q1, J - I <= 1, I * 64, J * 64 + c0, A, en, v6);
     en = wave_sum(en);
     if (l == 0) ewv[w] = en;
     if (VIR) {
-        const double v6[6] = {vxx, vyy, vzz, vxy, vxz, vyz};
         for (int cc = 0; cc < 6; ++cc) {
             const double v = wave_sum(v6[cc]);
             if (l == 0) wv[w][cc] = v;
@@ -489,11 +450,200 @@ __device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, con
     }
 }
 
-template <bool VIR, bool CARG, bool CULL, int W>
+template <bool VIR, bool CARG, int W>
 __global__ __launch_bounds__(64 * W) void k_realspace(const RsArgs A)
 {
     __shared__ RsLds<W> L;
-    rs_tile<VIR, CARG, CULL, W>(L, blockIdx.x, gridDim.x, A);
+    rs_tile<VIR, CARG, W>(L, blockIdx.x, gridDim.x, A);
+}
+
+// The culling form.  The sites come from k_sites (x, y, z, q per site and
+// bounding boxes per 64-site block and per 8-site cluster).  A tile whose two
+// blocks' boxes are more than r_c apart under every periodic image holds no
+// pair within the cutoff: k_tilefar marks it in rfar[e * ntile + tile] and
+// zeroes its energy partial; no slot entries are written for it (k_kforce_mf
+// and k_kforce read none of a tile so marked).  In the other tiles the cutoff
+// test runs only over pairs of clusters whose boxes lie within r_c (4096 H2O,
+// r_c 9 A: a third of the cluster pairs of the near tiles), one lane per site
+// pair.  The same pairs are evaluated as by k_realspace.
+// RS_CW waves take A.gs consecutive tiles of the list and work off the live
+// ones, each wave its columns; the rows' sites stay in LDS while I is the same.
+// Few blocks are launched for tiles that hold nothing (4096 x 32: three of
+// four), and a tile's few hundred pairs (4096 H2O: 400) fill the lanes of two
+// waves better than those of four.  Pass 1 takes RS_UNROLL cluster pairs at a
+// time, their LDS reads in flight together; the queue is worked off, in whole
+// rounds of the lanes, when it holds RS_QUEUE pairs.  RS_COEF is read after
+// pass 1, whose scalars would be spilled otherwise.  Vector units and LDS are
+// each busy two thirds of the time; of the 4096 x 32 launch pass 2 takes 58 %,
+// pass 1 20 %.  us, a block of four waves per tile (of two) before -> now: 4096
+// x 32 836 (703) -> 610, 1728 x 16 at r_c 12.9 A 323 (309) -> 301, 1000 x 32 183
+// (168) -> 156, 2197 x 1 28 -> 29.  One wave a tile: 593, 324, 161, 36.
+// grid: E * ceil(nt / gs), 64 RS_CW threads.
+constexpr int RS_CW = 2, RS_UNROLL = 4, RS_QUEUE = 1024;
+constexpr long RS_CULL_WAVES = 16384;  // blocks of a launch at which gs grows past 1
+template <bool CUBIC>
+struct RsU {
+    using type = uint2;
+};
+template <>
+struct RsU<false> {
+    using type = uint4;
+};
+template <bool CUBIC>
+struct RsCullLds {
+    double4 sI[64], sJ[64];
+    typename RsU<CUBIC>::type uI[64], uJ[64];
+    double fj[3][64], fi[RS_CW][3][64];
+    double ewv[RS_CW], wv[RS_CW][6];
+    unsigned short qe[RS_CW][RS_QUEUE + 64 * RS_UNROLL];
+};
+template <bool VIR, bool CUBIC>
+__global__ __launch_bounds__(64 * RS_CW, 5) void k_realspace_cull(const RsArgs A)
+{
+    __shared__ RsCullLds<CUBIC> L;
+    constexpr int W = RS_CW, CPW = 64 / W;  // columns per wave
+    using U = typename RsU<CUBIC>::type;
+    const int n_atoms = A.n_atoms, NAP = A.NAP, nblk = A.nblk, ntile = A.ntile, nt = A.nt;
+    const int ep_stride = A.ep_stride, ep_off = A.ep_off;
+    const Box &box = A.box;
+    const RsFix &fx = A.fx;
+    const int ng = (nt + A.gs - 1) / A.gs;
+    const int bid = xcd_remap(blockIdx.x, gridDim.x);
+    const int e = bid / ng, g0 = (bid - e * ng) * A.gs;
+    const int l = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const double4 *sites = A.sites + (long)e * nblk * 64;
+    const double *bbox = A.bbox + (long)e * nblk * RS_BOX + 6;
+    double *rp = A.rpart + (long)e * nblk * 3 * NAP;
+    // the live tiles of the group (gs <= 64)
+    const int tl = A.t0 + g0 + l;
+    unsigned long long tiles = __ballot(l < A.gs && g0 + l < nt && !A.rfar[(long)e * ntile + min(tl, ntile - 1)]);
+    int Icur = -1;
+    while (tiles) {
+        const int t = A.t0 + g0 + __builtin_ctzll(tiles);
+        tiles &= tiles - 1ull;
+        const int I = A.tiles[t].x, J = A.tiles[t].y;
+        // the first wave stages the sites of J, the last those of a new I
+        const bool newI = I != Icur;
+        Icur = I;
+        double4 v = make_double4(0.0, 0.0, 0.0, 0.0);
+        if (w == 0 || newI) v = sites[(w == 0 ? J : I) * 64 + l];
+        const int ci = l & 7, cj = l >> 3;
+        const double *cI = bbox + (long)I * RS_BOX, *cJ = bbox + (long)J * RS_BOX;
+        double gsq = 0.0;
+        for (int d = 0; d < 3; ++d) {
+            const double gap = periodic_gap(cI[8 * d + ci], cI[8 * (3 + d) + ci], cJ[8 * d + cj],
+                                            cJ[8 * (3 + d) + cj], box.L[d], box.inv[d]);
+            gsq = fma(gap, gap, gsq);
+        }
+        // the live 8 x 8 cluster pairs: lane l tests row cluster l & 7 against
+        // column cluster l >> 3
+        unsigned long long todo = __ballot(gsq <= A.ew.rcut_sq * (1.0 + 1e-9) && I * 64 + 8 * ci < n_atoms &&
+                                           J * 64 + 8 * cj < n_atoms && (I != J || cj >= ci)) &
+                                  (((1ull << CPW) - 1ull) << (CPW * w));
+        __syncthreads();
+        auto put = [&](double4 *s4, U *u) {
+            s4[l] = v;
+            const uint4 x = rs_fixed(v.x, v.y, v.z, box, CUBIC);
+            if constexpr (CUBIC) u[l] = make_uint2(x.x, x.y);
+            else u[l] = x;
+        };
+        if (w == 0) {
+            put(L.sJ, L.uJ);
+            for (int d = 0; d < 3; ++d) L.fj[d][l] = 0.0;
+        }
+        if (w == W - 1 && newI) put(L.sI, L.uI);
+        for (int d = 0; d < 3; ++d) L.fi[w][d][l] = 0.0;
+        __syncthreads();
+        double en = 0.0, v6[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+        unsigned short *qe = L.qe[w];
+        // a tile that holds places without a pair
+        const bool edge = I == J || J * 64 + 64 > n_atoms;
+        int total = 0;
+        do {
+            // pass 1 over the live cluster pairs: each one's 64 site pairs
+            // take one lane each; the queue holds a cluster pair's entries by
+            // column, rows within a column
+            while (todo && total < RS_QUEUE) {
+                int il[RS_UNROLL], jl[RS_UNROLL];
+                bool in[RS_UNROLL];
+#pragma unroll
+                for (int u = 0; u < RS_UNROLL; ++u) {
+                    in[u] = todo != 0ull;
+                    const int bit = in[u] ? __builtin_ctzll(todo) : 0;
+                    todo &= todo - 1ull;
+                    il[u] = 8 * (bit & 7) + (l & 7);
+                    jl[u] = 8 * (bit >> 3) + (l >> 3);
+                }
+#pragma unroll
+                for (int u = 0; u < RS_UNROLL; ++u) {
+                    if constexpr (CUBIC) in[u] = in[u] && rs_near16(L.uI[il[u]], L.uJ[jl[u]], fx.r2u);
+                    else in[u] = in[u] && rs_near32(L.uI[il[u]], L.uJ[jl[u]], fx);
+                }
+                if (edge) {
+#pragma unroll
+                    for (int u = 0; u < RS_UNROLL; ++u)
+                        in[u] = in[u] && J * 64 + jl[u] > I * 64 + il[u] && J * 64 + jl[u] < n_atoms;
+                }
+#pragma unroll
+                for (int u = 0; u < RS_UNROLL; ++u) {
+                    const unsigned long long bal = __ballot(in[u]);
+                    if (in[u]) {
+                        const int r = __builtin_amdgcn_mbcnt_hi((unsigned)(bal >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((unsigned)bal, 0u));
+                        qe[total + r] = (unsigned short)(il[u] | (jl[u] << 6));
+                    }
+                    total += __popcll(bal);
+                }
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            // all of it, or whole rounds of the lanes when more is to come
+            const int n = todo ? total & ~63 : total;
+            const int S = (n + 63) >> 6;
+            const int q0 = min(l * S, n), q1 = min(q0 + S, n);
+            rs_pairs<VIR, true>(L.sI, L.sJ, L.fi[w], L.fj, 0, qe, q0, q1, J - I <= 1, I * 64, J * 64, A, en, v6);
+            total -= n;
+            if (total > 0) {
+                const unsigned short keep = qe[n + l];
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                if (l < total) qe[l] = keep;
+            }
+        } while (todo || total > 0);
+        en = wave_sum(en);
+        if (l == 0) L.ewv[w] = en;
+        if (VIR) {
+            for (int c = 0; c < 6; ++c) {
+                const double x = wave_sum(v6[c]);
+                if (l == 0) L.wv[w][c] = x;
+            }
+        }
+        __syncthreads();
+        if (threadIdx.x < 6 && VIR) {
+            double x = 0.0;
+#pragma unroll
+            for (int k = 0; k < W; ++k) x += L.wv[k][threadIdx.x];
+            A.vpart[((long)e * 6 + threadIdx.x) * ep_stride + ep_off + t] = x;
+        }
+        if (threadIdx.x == 0) {
+            double x = 0.0;
+#pragma unroll
+            for (int k = 0; k < W; ++k) x += L.ewv[k];
+            A.epart[(long)e * ep_stride + ep_off + t] = x;
+        }
+        for (int k = threadIdx.x; k < 192; k += 64 * W) {
+            const int d = k >> 6, ll = k & 63;
+            double si = 0.0;
+#pragma unroll
+            for (int x = 0; x < W; ++x) si += L.fi[x][d][ll];
+            const double sj = L.fj[d][ll];
+            if (I == J) {
+                rp[((long)I * 3 + d) * NAP + I * 64 + ll] = si + sj;
+            } else {
+                rp[((long)J * 3 + d) * NAP + I * 64 + ll] = si;  // slot J
+                rp[((long)I * 3 + d) * NAP + J * 64 + ll] = sj;  // slot I
+            }
+        }
+    }
 }
 
 }  // namespace qtp

@@ -1296,7 +1296,7 @@ __global__ __launch_bounds__(256, 6) void k_phase_pairs(const RsArgs rs, const K
     b -= n_nl;
     const bool rs_last = n_ks + n_lj + n_rs <= PH_RESIDENT;
     if (rs_last ? b >= n_ks + n_lj : b < n_rs) {
-        rs_tile<VIR, true, false, 4>(*(RsLds<4> *)smem, rs_last ? b - n_ks - n_lj : b, n_rs, rs);
+        rs_tile<VIR, true, 4>(*(RsLds<4> *)smem, rs_last ? b - n_ks - n_lj : b, n_rs, rs);
         return;
     }
     if (!rs_last) b -= n_rs;

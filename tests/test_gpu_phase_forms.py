@@ -120,3 +120,43 @@ def test_spread_rebuild_is_the_one_block_rebuild(nside, P):
     assert a[2] == b[2]
     for x, y in zip(a[0] + a[1], b[0] + b[1]):
         assert np.array_equal(x, y)
+
+
+def _ewald(box, rc_angs, n_max=6):
+    rc = rc_angs * A
+    return {"kappa": 2.9 / rc, "rcut": rc, "k_max": n_max,
+            "k_cut": 2.0 * np.pi * n_max / max(box) * (1.0 + 1e-9)}
+
+
+@pytest.mark.parametrize("nside,edge,P", [((7, 10, 14), 3.107, 32), ((8, 8, 8), 2.6, 2), ((6, 7, 8), 3.107, 4)])
+def test_culled_tiles_in_groups(nside, edge, P, oracle_mod):
+    """Boxes past the culling threshold: several tiles a block with a ragged
+    last group (980 H2O x 32: 1081 tiles, two a block; one bead alone: one a
+    block), boxes that are and are not cubic, and more pairs in a wave's half
+    of a tile than its queue holds (512 at 2.6 A a molecule)."""
+    from qtip4pf_water_amd import Water
+    q0, box, L = _box(nside, 31, edge)
+    n = q0.size // 9
+    rc = min(L) / 2.51
+    lj = cfg.lj_rcut_for(min(L))
+    if edge < 3.0:  # molecules in lattice order: close blocks of 64 sites
+        x = q0.reshape(3 * n, 3)
+        most = 0
+        for J in range(1, 8):
+            d = x[64 * (J - 1):64 * J, None] - x[None, 64 * J:64 * J + 32]
+            d -= np.array(box) * np.rint(d / np.array(box))
+            most = max(most, int(np.count_nonzero((d * d).sum(-1) < (rc * A) ** 2)))
+        assert most > 1024
+    q = cfg.replicate_beads(q0, P) + np.random.default_rng(32).normal(0, 0.03, P * 9 * n)
+    o = oracle_mod.Oracle(n, P, box, ewald=_ewald(box, rc), lj_rcut=lj)
+    point, lst, _ = o.all_lists(q)
+    with Water(n, P, box, ewald=_ewald(box, rc), lj_rcut=lj) as w:
+        F, f = np.zeros_like(q), np.zeros_like(q)
+        w.force_eval_sc_nospline(q, F, o.charge, o.mass, point, lst, fphys=f)
+        for b in (0, P - 1):
+            sl = slice(9 * n * b, 9 * n * (b + 1))
+            F1, Fr = np.zeros_like(q), np.zeros_like(q)
+            w.get_forces_nospline(q, F1, o.charge, point, lst, b)
+            o.get_forces(q, Fr, point, lst, b)
+            assert rel_atom_err(F1[sl], Fr[sl]) < 1e-10
+            assert rel_atom_err(f[sl], F1[sl]) < 1e-10
