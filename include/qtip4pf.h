@@ -318,12 +318,13 @@ int qtp_run_observed(qtp_ctx *ctx, int n_steps, int is_nvt, int every, double *t
  * coefficients in scalar registers (1), as literals (0) or by grid size (-1),
  * 16-wave k-space force blocks (1), 8-wave (0) or by block count (-1),
  * structure-factor blocks per 64-site chunk (1-4; 0 by launch size),
- * propagation as one LDS-staged kernel per step where the thermostat allows
- * it: for systems of 256 or more 64-dof tiles (-1), always (1), never (0;
- * the results are the same bit for bit), waves per real-space tile block (2
- * or 4; no effect in boxes so wide that tiles are skipped), eighths of the real-space tiles launched on the second stream after
- * the LJ/intramolecular kernel (0-4), site chunks per structure-factor block
- * of the matrix-core path (1, 2, 4, 8, 16; 0 by launch size)}.
+ * propagation as one launch per step where the thermostat allows it (up to 64
+ * beads): by default (-1), yes (1), no (0; the results are the same bit for
+ * bit), waves per real-space tile block (2 or 4; no effect in boxes so wide
+ * that tiles are skipped), eighths of the real-space tiles launched on the
+ * second stream after the LJ/intramolecular kernel (0-4), site chunks per
+ * structure-factor block of the matrix-core path (1, 2, 4, 8, 16; 0 by launch
+ * size)}.
  * Every configuration gives the same forces up to summation order. */
 int qtp_get_tuning(const qtp_ctx *ctx, int cfg[9]);
 /* Sets cfg (QTP_ERR_ARG for values the context cannot run); with a state set,

@@ -70,9 +70,8 @@ struct qtp_ctx {
     // a list check the SC step leaves to the next force phase's second stream
     bool lists_defer = false, lists_heat = false;
     const unsigned long long *lists_ctr = nullptr;
-    // propagation as one LDS-staged kernel per step (k_prop_tile) where the
-    // thermostat allows it: -1 for systems of PT_MIN_TILES tiles or more,
-    // 1 always, 0 never (k_prop_fwd + k_prop_inv)
+    // propagation as one launch per step (k_prop_dofs) where the thermostat
+    // and the bead count allow it: -1 and 1 yes, 0 no (k_prop_fwd + k_prop_inv)
     int prop_fused = -1;
     int ep_cap = 0;   // allocated stride of the energy partials
     int mf_Mp = 0, mf_nks = 0, mf_nrt = 0, mf_nrt_small = 0, ks_nslot = 0, ks_cap = 6, ks_nslot_ph = 0;

@@ -150,7 +150,7 @@ static HeatArgs heat_args(const qtp_ctx *ctx, bool with_heat)
         h.heat_acc = ctx->heat;
         h.heat_step = ctx->heat_step;
         h.ntile = ctx->ptile;
-        h.nh = ctx->P * ctx->ptile;
+        h.nh = ctx->P * ctx->ptile * HP_PARTS;
     }
     return h;
 }
@@ -568,14 +568,12 @@ static int run_sc_step(qtp_ctx *ctx, int nvt, int host_dev, unsigned long long *
     hipStream_t s = ctx->stream;
     PropArgs A = prop_args(ctx, nvt, host_dev);
     const int grid = ctx->ptile * ctx->P;
-    // one kernel per tile, the beads staged in LDS, when the centroid needs
-    // no rescale over the whole system between the two transforms
+    // one launch when the centroid needs no rescale over the whole system
+    // between the two transforms
     const bool bussi = nvt && A.cthermo == 0 && A.cmode != 2;
-    const bool big = ctx->ptile >= PT_MIN_TILES;
-    if ((ctx->prop_fused == 1 || (ctx->prop_fused == -1 && big)) && !bussi &&
-        !(nvt && host_dev) && ctx->P <= PT_WAVES * PT_PER_WAVE) {
+    if (ctx->prop_fused != 0 && !bussi && !(nvt && host_dev) && ctx->P <= PD_MAX_BEADS) {
         TimeScope ts(ctx, "prop");
-        k_prop_tile<<<ctx->ptile, 64 * PT_WAVES, prop_tile_lds(ctx->P), s>>>(
+        k_prop_dofs<<<HP_PARTS * ctx->ptile, HP_DOFS * ctx->P, prop_dofs_lds(ctx->P), s>>>(
             A, ctx->Cm, ctx->mode, ctx->ms, ctx->q, ctx->p, ctx->F, ctx->m_atom, ctx->sqm_atom,
             ctx->ppart, ctx->hpart, ctx->disp, ctx->NMP, ctr);
     } else {

@@ -311,6 +311,22 @@ __device__ __forceinline__ void cayley_half(double &uq, double &up, double m, do
     uq = temp;
 }
 
+// A lane's heat of mode k into the partials of the tile's groups of HP_DOFS
+// dofs, hpart[(k * ntile + tile) * HP_PARTS + group] (every form of the
+// propagation sums in the same order).
+constexpr int HP_DOFS = 16, HP_PARTS = 64 / HP_DOFS;
+__device__ __forceinline__ double heat_group(double h)
+{
+    for (int o = HP_DOFS / 2; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
+    return h;
+}
+__device__ __forceinline__ void heat_part(double h, double *hpart, int k, int tile, int ntile)
+{
+    const int lane = threadIdx.x & 63;
+    h = heat_group(h);
+    if (lane % HP_DOFS == 0) hpart[((long)k * ntile + tile) * HP_PARTS + lane / HP_DOFS] = h;
+}
+
 // Kick, forward normal-mode transform and first half step for mode k of 64
 // planar dofs; modes k >= 1 also get their Langevin step and second half
 // step here (they do not wait for the centroid).  One wavefront per
@@ -318,7 +334,7 @@ __device__ __forceinline__ void cayley_half(double &uq, double &up, double m, do
 // grid: ntile * P (tile-major, XCD-remapped), 64 threads.
 // part[tile] = centroid KE after the first half step (tile partial);
 // part[ntile + tile] = chi-square partial (device random numbers);
-// hpart[k * ntile + tile] = KE before - KE after of mode k's Langevin step.
+// hpart: KE before - KE after of mode k's Langevin step (heat_part).
 __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__restrict__ Cm,
                                                  const double4 *__restrict__ mode,
                                                  const double2 *__restrict__ mscale,
@@ -377,13 +393,12 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
         np[f] = up;
         ke0 = wave_sum(ke0);
         chi = wave_sum(chi);
-        h = wave_sum(h);
         if (lane == 0) {
             part[tile] = ke0;
             part[A.ntile + tile] = chi;
-            // the centroid's heat slot: PILE-L's here, PILE-G's in k_prop_inv
-            if (A.nvt && !pile_g) hpart[tile] = h;
         }
+        // the centroid's heat slot: PILE-L's here, PILE-G's in k_prop_inv
+        if (A.nvt && !pile_g) heat_part(h, hpart, 0, tile, A.ntile);
         return;
     }
     cayley_half(uq, up, m, A.halfdt, md);
@@ -397,8 +412,7 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
             up = md.z * up + sqm_atom[at] * md.w * xi;
             h -= 0.5 * up * up / m;
         }
-        h = wave_sum(h);
-        if (lane == 0) hpart[(long)k * A.ntile + tile] = h;
+        heat_part(h, hpart, k, tile, A.ntile);
     }
     cayley_half(uq, up, m, A.halfdt, md);
     nq[k * N3 + f] = uq;
@@ -408,7 +422,7 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
 // Centroid rescale (Bussi, tau -> 0), its second half step, inverse
 // transform to bead b and displacement tracking.  One wavefront per
 // (dof tile, bead).   grid: ntile * P (tile-major, XCD-remapped), 64 threads.
-// hpart[tile] (mode-0 slot) = - centroid KE after the rescale (bead-0 waves).
+// hpart (mode 0) = - centroid KE after the rescale (bead-0 waves).
 __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__restrict__ Cm,
                                                  const double4 *__restrict__ mode,
                                                  const double *__restrict__ nq,
@@ -452,8 +466,7 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
         u0p *= alpha;
         if (b == 0) {
             double h = va ? -0.5 * u0p * u0p / m : 0.0;
-            h = wave_sum(h);
-            if (lane == 0) hpart[tile] = h;
+            heat_part(h, hpart, 0, tile, A.ntile);
         }
     }
     cayley_half(u0q, u0p, m, A.halfdt, mode[0]);
@@ -471,24 +484,24 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
     if (va && (at % 3) == 0) disp[((long)b * 3 + d) * NMP + at / 3] += xq - qold;
 }
 
-// The whole propagation of a step for one 64-dof tile when the centroid needs
-// no global rescale (NVE, PILE-L, or the centroid held fixed): kick, forward
+// The whole propagation of a step in one launch when the centroid needs no
+// global rescale (NVE, PILE-L, or the centroid held fixed): kick, forward
 // normal-mode transform, sqrt-Cayley half steps around the Langevin steps of
 // every mode, inverse transform, displacement tracking (update.cpp:281-352,
-// thermostat.cpp:114-129).  The tile's P beads are read from HBM once and
-// staged in LDS ([P][64] positions and kicked momenta, then the modes in the
-// same space); the arithmetic and its order are k_prop_fwd's and
-// k_prop_inv's, so the results are the same bit for bit.
-// grid: ntile (XCD-remapped), 64 * PT_WAVES threads, 2 P 64 doubles of LDS;
-// P <= PT_WAVES * PT_PER_WAVE.
-constexpr int PT_WAVES = 8, PT_PER_WAVE = 8;
-// Below this many tiles (one block per CU) the two-kernel form, with a wave
-// per (tile, mode), has more parallelism and is faster (216 x 32: 33 tiles,
-// 25.6 us fused against 16.4 us for the pair; 4096 x 32: 576 tiles, 69
-// against 124 us).
-constexpr int PT_MIN_TILES = 256;
-inline size_t prop_tile_lds(int P) { return (size_t)2 * P * 64 * sizeof(double); }
-__global__ __launch_bounds__(64 * PT_WAVES) void k_prop_tile(
+// thermostat.cpp:114-129).  HP_DOFS dofs per block, a thread per (mode, dof),
+// then per (bead, dof); the beads' positions and kicked momenta and the matrix
+// are staged in LDS, so that HBM is read and written once.  Bound by the chain
+// of load, P multiply-adds, random numbers, P multiply-adds and store.  The
+// arithmetic and its order are k_prop_fwd's and k_prop_inv's.  us, k_prop_fwd +
+// k_prop_inv -> this: 216 x 32 7.7 + 6.9 -> 7.5, 512 x 32 13.4 + 11.1 -> 13.1,
+// 990 x 16 8.7 + 8.8 -> 8.4, 4096 x 32 64 + 44 -> 38 (a block of 64 dofs and
+// 512 threads, eight modes a thread: 84).  With 64-byte pieces (eight dofs)
+// instead of 128 a block would share its cache lines with the next.
+// grid: HP_PARTS * ntile (XCD-remapped), HP_DOFS * P threads,
+// prop_dofs_lds(P); P <= PD_MAX_BEADS.
+constexpr int PD_MAX_BEADS = 64;
+inline size_t prop_dofs_lds(int P) { return (size_t)(2 * P * HP_DOFS + P * (P + 1)) * sizeof(double); }
+__global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     PropArgs A, const double *__restrict__ Cm, const double4 *__restrict__ mode,
     const double2 *__restrict__ mscale, double *__restrict__ q, double *__restrict__ p,
     const double *__restrict__ F, const double *__restrict__ m_atom,
@@ -496,102 +509,65 @@ __global__ __launch_bounds__(64 * PT_WAVES) void k_prop_tile(
     double *__restrict__ disp, int NMP, const unsigned long long *__restrict__ step_ctr)
 {
     extern __shared__ double S[];
-    const int P = A.P;
-    double *SQ = S, *SP = S + (long)P * 64;
-    const int tile = xcd_remap(blockIdx.x, gridDim.x);
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int P = A.P, CP = P + 1;
+    double *SQ = S, *SP = S + P * HP_DOFS, *C = S + 2 * P * HP_DOFS;  // C: [P][P + 1]
+    const int blk = xcd_remap(blockIdx.x, gridDim.x);
+    const int tid = threadIdx.x, k = tid / HP_DOFS, i = tid % HP_DOFS;  // mode or bead, dof
+    const int tile = blk / HP_PARTS, group = blk % HP_PARTS;
     const long N3 = 3L * A.NAP;
-    const int f = tile * 64 + lane;
+    const int f = blk * HP_DOFS + i;
     const int at = f % A.NAP, d = f / A.NAP;
     const bool va = at < A.n_atoms;
-    double qold[PT_PER_WAVE];
-#pragma unroll
-    for (int j = 0; j < PT_PER_WAVE; ++j) {
-        const int b = w + j * PT_WAVES;
-        if (b < P) {
-            const long idx = b * N3 + f;
-            const double qq = q[idx];
-            qold[j] = qq;
-            SQ[b * 64 + lane] = qq;
-            SP[b * 64 + lane] = p[idx] + A.halfdt * F[idx];   // update.cpp:281-287
-        }
-    }
+    const long idx = k * N3 + f;
+    const double qold = q[idx];
+    const double pk = p[idx] + A.halfdt * F[idx];  // update.cpp:281-287
+    const double m0 = va ? m_atom[at] : 1.0, sqm = va ? sqm_atom[at] : 0.0;
+    const double m = va ? m0 * mscale[k].x : 1.0;
+    const double4 md = mode[k];
+    for (int t = tid; t < P * P; t += HP_DOFS * P) C[t / P * CP + t % P] = Cm[t];
+    SQ[tid] = qold;
+    SP[tid] = pk;
     __syncthreads();
-    double rq[PT_PER_WAVE], rp[PT_PER_WAVE];
-#pragma unroll
-    for (int j = 0; j < PT_PER_WAVE; ++j) {
-        const int k = w + j * PT_WAVES;
-        if (k >= P) continue;
-        const double m = va ? m_atom[at] * mscale[k].x : 1.0;
-        const double *cr = Cm + (long)k * P;
-        double uq = 0.0, up = 0.0;
-        for (int b = 0; b < P; ++b) {
-            const double c = cr[b];
-            uq = fma(c, SQ[b * 64 + lane], uq);
-            up = fma(c, SP[b * 64 + lane], up);
-        }
-        const double4 md = mode[k];
-        if (k == 0) {
-            if (A.cmode == 2) up = 0.0;
-            cayley_half(uq, up, m, A.halfdt, md);
-            double h = 0.0;
-            if (A.nvt && A.cthermo == 1 && A.cmode != 2 && va) {
-                h = 0.5 * up * up / m;
-                const double xi = philox_normal(A.seed, *step_ctr, 0u, (uint32_t)(3 * at + d));
-                up = A.c1_0 * up + sqm_atom[at] * A.c2_0 * xi;
-                h -= 0.5 * up * up / m;
-            }
-            h = wave_sum(h);
-            if (lane == 0) {
-                part[tile] = 0.0;
-                part[A.ntile + tile] = 0.0;
-                if (A.nvt) hpart[tile] = h;
-            }
-            cayley_half(uq, up, va ? m_atom[at] : 1.0, A.halfdt, mode[0]);
-        } else {
-            cayley_half(uq, up, m, A.halfdt, md);
-            if (A.nvt) {
-                double h = 0.0;
-                if (va) {
-                    h += 0.5 * up * up / m;
-                    const double xi =
-                        philox_normal(A.seed, *step_ctr, (uint32_t)k, (uint32_t)(3 * at + d));
-                    up = md.z * up + sqm_atom[at] * md.w * xi;
-                    h -= 0.5 * up * up / m;
-                }
-                h = wave_sum(h);
-                if (lane == 0) hpart[(long)k * A.ntile + tile] = h;
-            }
-            cayley_half(uq, up, m, A.halfdt, md);
-        }
-        rq[j] = uq;
-        rp[j] = up;
+    double uq = 0.0, up = 0.0;
+#pragma unroll 8
+    for (int b = 0; b < P; ++b) {
+        const double c = C[k * CP + b];
+        uq = fma(c, SQ[b * HP_DOFS + i], uq);
+        up = fma(c, SP[b * HP_DOFS + i], up);
     }
+    if (k == 0 && A.cmode == 2) up = 0.0;  // centroid held fixed
+    cayley_half(uq, up, m, A.halfdt, md);
+    if (A.nvt) {
+        double h = 0.0;
+        if (va && !(k == 0 && (A.cthermo != 1 || A.cmode == 2))) {
+            // random stream k; the centroid: PILE-L
+            h += 0.5 * up * up / m;
+            const double xi = philox_normal(A.seed, *step_ctr, (uint32_t)k, (uint32_t)(3 * at + d));
+            up = k == 0 ? A.c1_0 * up + sqm * A.c2_0 * xi : md.z * up + sqm * md.w * xi;
+            h -= 0.5 * up * up / m;
+        }
+        h = heat_group(h);
+        if (i == 0) hpart[((long)k * A.ntile + tile) * HP_PARTS + group] = h;
+    }
+    if (tid == 0 && group == 0) {
+        part[tile] = 0.0;
+        part[A.ntile + tile] = 0.0;
+    }
+    cayley_half(uq, up, k == 0 ? m0 : m, A.halfdt, md);
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PT_PER_WAVE; ++j) {
-        const int k = w + j * PT_WAVES;
-        if (k < P) {
-            SQ[k * 64 + lane] = rq[j];
-            SP[k * 64 + lane] = rp[j];
-        }
-    }
+    SQ[tid] = uq;
+    SP[tid] = up;
     __syncthreads();
-#pragma unroll
-    for (int j = 0; j < PT_PER_WAVE; ++j) {
-        const int b = w + j * PT_WAVES;
-        if (b >= P) continue;
-        double xq = Cm[b] * SQ[lane], xp = Cm[b] * SP[lane];
-        for (int k = 1; k < P; ++k) {
-            const double c = Cm[(long)k * P + b];
-            xq = fma(c, SQ[k * 64 + lane], xq);
-            xp = fma(c, SP[k * 64 + lane], xp);
-        }
-        const long idx = b * N3 + f;
-        q[idx] = xq;
-        p[idx] = xp;
-        if (va && (at % 3) == 0) disp[((long)b * 3 + d) * NMP + at / 3] += xq - qold[j];
+    double xq = C[k] * SQ[i], xp = C[k] * SP[i];
+#pragma unroll 8
+    for (int kk = 1; kk < P; ++kk) {
+        const double c = C[kk * CP + k];
+        xq = fma(c, SQ[kk * HP_DOFS + i], xq);
+        xp = fma(c, SP[kk * HP_DOFS + i], xp);
     }
+    q[idx] = xq;
+    p[idx] = xp;
+    if (va && (at % 3) == 0) disp[((long)k * 3 + d) * NMP + at / 3] += xq - qold;
 }
 
 // The thermostat's heat for one step: pile_g's return value (KE before -
@@ -917,7 +893,7 @@ constexpr int NL_FUSED_MAXMOL = 1024;
 // of block 0 here so that it costs no launch of its own.
 struct HeatArgs {
     const double *part;  // centroid KE partials (ntile) then chi partials
-    const double *hpart; // per-(mode, tile) heat partials (nh)
+    const double *hpart; // heat partials of the modes (nh)
     double *heat_acc, *heat_step;
     int ntile, nh;
 };

@@ -160,3 +160,33 @@ def test_culled_tiles_in_groups(nside, edge, P, oracle_mod):
             o.get_forces(q, Fr, point, lst, b)
             assert rel_atom_err(F1[sl], Fr[sl]) < 1e-10
             assert rel_atom_err(f[sl], F1[sl]) < 1e-10
+
+
+@pytest.mark.parametrize("nside,P,thermo,mode", [
+    ((4, 4, 4), 2, "pile_l", None), ((4, 4, 5), 6, None, None), ((6, 6, 6), 32, "pile_l", None),
+    ((4, 5, 6), 64, "pile_l", "pacmd"), ((5, 5, 5), 8, "pile_g", "centroid_fixed")])
+def test_propagation_forms_agree_bitwise(nside, P, thermo, mode):
+    """One launch with a thread per (mode, dof) (the default of small systems)
+    against the two-kernel form: same operations in the same
+    order, the heat included."""
+    from qtip4pf_water_amd import Water
+    q0, box, L = _box(nside, 41)
+    n = q0.size // 9
+    beta_n = 1.0 / (cfg.K2AU * 298.0) / P
+    q = cfg.free_ring_polymer_beads(q0, P, beta_n, seed=42)
+    p = cfg.sample_momenta(n, P, beta_n, seed=43)
+    out = []
+    for fused in (-1, 0, 1):
+        with Water(n, P, box, dtfs=0.1, lj_rcut=cfg.lj_rcut_for(min(L))) as w:
+            if thermo:
+                w.set_thermostat(thermo, 100.0)
+            if mode:
+                w.set_pimd_mode(mode)
+            w.set_tuning(fused_propagation=fused, rs_registers=1)
+            w.set_seed(5)
+            w.set_state(q, p)
+            w.run(4, is_nvt=thermo is not None)
+            out.append((w.get_state(), w.scalars()))
+    for st, sc in out[1:]:
+        assert all(np.array_equal(x, y) for x, y in zip(st, out[0][0]))
+        assert sc == out[0][1]
