@@ -211,7 +211,7 @@ static int nn_train_batch(qtp_nn *nn, hipStream_t s, int f0, int F, int mode, do
     NNCHK(hipMemsetAsync(nn->inter, 0, nn_inter_elems(b) * sizeof(__bf16), s));
     k_nn_train_fwd<<<b.nbo + b.nbh, 64 * MLP_WAVES, TRAIN_LDS, s>>>(g, nn_weights(nn), b.nbo, nn->gt,
                                                                    nn->ut, T);
-    k_nn_wgrad<<<b.nco + b.nch, 64 * WG_WAVES, 0, s>>>(T, b.nco, nn->part);
+    k_nn_wgrad<<<dim3(b.nco + b.nch, WG_TILES / WG_WAVES), 64 * WG_WAVES, 0, s>>>(T, b.nco, nn->part);
     AdamArgs ad{};
     if (mode == 1) {
         nn->adam_t += 1;

@@ -52,9 +52,26 @@ __device__ __forceinline__ float xor_lane(float v, int o)
     return __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(v)));
 }
 
+// The xor tree 32 ... 1 as wave_sum's: no LDS.  block_sums has 40 of these a
+// wave, which kept the LDS busy for about half of k_nn_tan's time.
 __device__ __forceinline__ float wave_sumf(float v)
 {
-    for (int o = 32; o > 0; o >>= 1) v += xor_lane(v, o);
+    {
+        const unsigned u = __float_as_uint(v);
+        const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+    {
+        const unsigned u = __float_as_uint(v);
+        const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+        v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+    }
+#define QTP_ROR(N) v += __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x120 + N, 0xf, 0xf, true))
+    QTP_ROR(8);
+    QTP_ROR(4);
+    QTP_ROR(2);
+    QTP_ROR(1);
+#undef QTP_ROR
     return v;
 }
 
@@ -1051,9 +1068,12 @@ __global__ __launch_bounds__(64 * TRAIN_WAVES) void k_nn_train_fwd(
 // element: part[e][chunk] = [dJ/dW1 (128 x 64) | dJ/dW2 (128 x 128)],
 //   dJ/dW2[m][n] = sum_rows d2t[m] a1t[n] + d2p[m] a1p[n]
 //   dJ/dW1[m][k] = sum_rows d1t[m] a0t[k] + d1p[m] a0p[k]
-// 88 output tiles of 16 x 16 (64 of W2, 24 of W1 for k < 48) over 8 waves.
-// grid: nco + nch blocks (chunks of O, then of H), 512 threads.
-constexpr int WG_WAVES = 8;
+// 88 output tiles of 16 x 16 (64 of W2, 24 of W1 for k < 48), one a wave: a
+// training batch has few chunks (eight frames of 216 H2O: 21), and with all
+// tiles of a chunk in one block the launch took 80 us on 21 CUs, now 9.5.
+// grid: (nco + nch) x 88 / WG_WAVES blocks (chunks of O, then of H; groups of
+// tiles), 512 threads.
+constexpr int WG_WAVES = 8, WG_TILES = 88;
 constexpr int WG_PART = NH * KIN + NH * NH;
 __global__ __launch_bounds__(64 * WG_WAVES) void k_nn_wgrad(NNTrainBuf B, int nco,
                                                             float *__restrict__ part)
@@ -1064,7 +1084,8 @@ __global__ __launch_bounds__(64 * WG_WAVES) void k_nn_wgrad(NNTrainBuf B, int nc
     const int ld = B.rows[e];
     const long r0 = (long)chunk * WG_ROWS;
     float *P = part + (long)blockIdx.x * WG_PART;
-    for (int tt = wv; tt < 88; tt += WG_WAVES) {
+    const int tt = blockIdx.y * WG_WAVES + wv;
+    {
         const bool w2 = tt < 64;
         const int mt = w2 ? tt >> 3 : (tt - 64) / 3, nt = w2 ? tt & 7 : (tt - 64) % 3;
         const __bf16 *At = w2 ? B.d2t[e] : B.d1t[e], *Ap = w2 ? B.d2p[e] : B.d1p[e];
@@ -1126,10 +1147,14 @@ __global__ __launch_bounds__(256) void k_nn_update(int mode, const float *__rest
         if (kind == 0 || kind == 2) {
             const int c0 = e == 0 ? 0 : nco, c1 = e == 0 ? nco : nco + nch;
             const long off = kind == 0 ? (long)n * KIN + k : (long)NH * KIN + (long)n * NH + k;
+#pragma unroll 16
             for (int c = c0; c < c1; ++c) s += (double)part[(long)c * WG_PART + off];
         } else if (kind != 5) {
             const int t0 = e == 0 ? 0 : nto, t1 = e == 0 ? nto : nto + nth;
             const int slot = kind == 1 ? 0 : (kind == 3 ? 1 : 2);
+            // sixteen loads in flight, added in order (one at a time the few
+            // threads of this kind took 55 us for 216 tiles, now 13)
+#pragma unroll 16
             for (int t = t0; t < t1; ++t) s += (double)tp[((long)t * 3 + slot) * NH + n];
         }
         const float gr = (float)(gscale * s);
