@@ -10,8 +10,8 @@
 // converted by one kernel.  Against converting on the host and one pageable,
 // synchronous copy per array (and expanding the lists on the host), one update_sc
 // call of 216 H2O x 32 beads:
-// 4.18 ms before, 0.79 ms now (chunks of 256 KiB: 1.00); get_forces of 64 H2O
-// 206 -> 84 us.
+// 4.18 ms before, 0.64 ms now (chunks of 256 KiB: 0.2 more); get_forces of 64
+// H2O 206 -> 71 us.
 constexpr size_t XFER_CHUNK = 1 << 20;
 constexpr int XFER_SLOTS = 4;  // qtp_ctx::xev
 constexpr int XFER_MAX = 8;  // arrays per call
@@ -193,13 +193,16 @@ static int download_planar(qtp_ctx *ctx, const double *src, int nb, double *ref)
 }
 
 // The caller's half lists of nb beads (point[b][n], entries packed from
-// ent[off[b]]) into the device half and full lists of beads dev_b0 ...: row i of
-// the full list holds its partners j < i (rows that list i) ascending, then
-// its own row.  One block per bead: incoming counts (LDS atomics), offsets, the
-// incoming entries in arrival order, then each row's sorted by rank (equal
-// entries of a caller's list are interchangeable).  n <= 1024: a row's
-// incoming entries fit sixteen registers a lane.
-// grid: nb, 1024 threads.
+// ent[off[b]]) into the device half and full lists: row i of the full list
+// holds its partners j < i (rows that list i) ascending, then its own row.
+// LE_ROWS rows a block: incoming counts of all rows (LDS atomics) and offsets,
+// then a wave per row picks its incoming entries out of all entries in their
+// order, which is by rising row, and looks up the rows.  All reads are
+// coalesced and from L2; one block a bead with its entries in arrival order and
+// sorted afterwards took 187 us for 216 x 32, this 86; 64 H2O 25, this 12.  n <=
+// 1024.
+// grid: nb * ceil(n / LE_ROWS), 1024 threads.
+constexpr int LE_ROWS = 16;
 __global__ __launch_bounds__(1024) void k_list_expand(int n, int list_size, long fcap,
                                                       const int *__restrict__ pt_in,
                                                       const int *__restrict__ ent,
@@ -207,21 +210,23 @@ __global__ __launch_bounds__(1024) void k_list_expand(int n, int list_size, long
                                                       int *__restrict__ point, int *__restrict__ list,
                                                       int *__restrict__ fpoint, int *__restrict__ flist)
 {
-    __shared__ int inc[NL_FUSED_MAXMOL], cur[NL_FUSED_MAXMOL];
+    __shared__ int pt[NL_FUSED_MAXMOL], inc[NL_FUSED_MAXMOL], beg[NL_FUSED_MAXMOL];
     __shared__ int s_tot[16];
-    const int b = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int *pt = pt_in + (long)b * n;
-    const int *L = ent + off[b] - pt[0];  // entries pt[0] ... pt[n-1] - 1
-    int *P = point + (long)b * n, *H = list + (long)b * list_size;
-    int *FP = fpoint + (long)b * (n + 1), *FL = flist + (long)b * fcap;
-    for (int i = tid; i < n; i += 1024) {
-        inc[i] = 0;
-        P[i] = pt[i];
+    const int nparts = (n + LE_ROWS - 1) / LE_ROWS;
+    const int b = blockIdx.x / nparts, part = blockIdx.x - b * nparts;
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    int *H = list + (long)b * list_size, *FL = flist + (long)b * fcap;
+    if (tid < n) {
+        pt[tid] = pt_in[(long)b * n + tid];
+        inc[tid] = 0;
     }
     __syncthreads();
-    for (int k = pt[0] + tid; k < pt[n - 1]; k += 1024) {
+    const int k0 = pt[0], k1 = pt[n - 1];
+    const int *L = ent + off[b] - k0;  // entries k0 ... k1 - 1
+#pragma unroll 4
+    for (int k = k0 + tid; k < k1; k += 1024) {
         const int j = L[k];
-        H[k] = j;
+        if (part == 0) H[k] = j;
         atomicAdd(&inc[j], 1);
     }
     __syncthreads();
@@ -238,46 +243,43 @@ __global__ __launch_bounds__(1024) void k_list_expand(int n, int list_size, long
     int base = s - v;
     for (int ww = 0; ww < w; ++ww) base += s_tot[ww];
     if (tid < n) {
-        cur[tid] = base;
-        FP[tid] = base;
-        if (tid == n - 1) FP[n] = base + v;
+        beg[tid] = base;
+        if (part == 0) {
+            point[(long)b * n + tid] = pt[tid];
+            fpoint[(long)b * (n + 1) + tid] = base;
+            if (tid == n - 1) fpoint[(long)b * (n + 1) + n] = base + v;
+        }
     }
     __syncthreads();
-    for (int i = w; i < n - 1; i += 16)
-        for (int k = pt[i] + lane; k < pt[i + 1]; k += 64) FL[atomicAdd(&cur[L[k]], 1)] = i;
-    __syncthreads();
-    // cur[i] is now the end of row i's incoming entries
-    constexpr int R = NL_FUSED_MAXMOL / 64;
-    for (int i = w; i < n; i += 16) {
-        const int m = inc[i], f0 = cur[i] - m;
-        int e[R], rank[R];
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (64 * r >= m) break;
-            const int t = lane + 64 * r;
-            e[r] = t < m ? FL[f0 + t] : 0;
-            rank[r] = 0;
+    const int i = part * LE_ROWS + w;
+    if (i >= n) return;
+    const int m = inc[i], f0 = beg[i];
+    const unsigned long long below = lane == 0 ? 0ull : ~0ull >> (64 - lane);
+    int at = f0;
+    if (m > 0) {
+#pragma unroll 8
+        for (int c = k0; c < k1; c += 64) {
+            const int k = c + lane;
+            const bool in = k < k1 && L[min(k, k1 - 1)] == i;
+            const unsigned long long bal = __ballot(in);
+            if (in) FL[at + __popcll(bal & below)] = k;
+            at += __popcll(bal);
         }
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            if (64 * q >= m) break;
-            for (int u = 0; u < min(64, m - 64 * q); ++u) {
-                const int x = __builtin_amdgcn_readlane(e[q], u);
-#pragma unroll
-                for (int r = 0; r < R; ++r) {
-                    if (64 * r >= m) break;
-                    rank[r] += x < e[r] || (x == e[r] && u + 64 * q < lane + 64 * r);
-                }
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+        for (int t = lane; t < m; t += 64) {
+            // the row that holds entry k: the last one with pt <= k
+            const int k = FL[f0 + t];
+            int lo = 0, hi = n - 1;  // pt[lo] <= k < pt[hi]
+            while (hi - lo > 1) {
+                const int mid = (lo + hi) >> 1;
+                if (pt[mid] <= k) lo = mid;
+                else hi = mid;
             }
+            FL[f0 + t] = lo;
         }
-#pragma unroll
-        for (int r = 0; r < R; ++r) {
-            if (64 * r >= m) break;
-            if (lane + 64 * r < m) FL[f0 + rank[r]] = e[r];
-        }
-        if (i < n - 1)
-            for (int k = pt[i] + lane; k < pt[i + 1]; k += 64) FL[cur[i] + k - pt[i]] = L[k];
     }
+    if (i < n - 1)
+        for (int k = pt[i] + lane; k < pt[i + 1]; k += 64) FL[f0 + m + k - pt[i]] = L[k];
 }
 
 // Caller's half lists (reference layout) checked: rows rise within list_size,
@@ -368,7 +370,7 @@ static int upload_with_lists(qtp_ctx *ctx, Xfer &x, const int *point, const int 
     }
     CHK(x.up());
     const int *w = (const int *)ctx->xref;
-    k_list_expand<<<nb, 1024, 0, ctx->stream>>>(
+    k_list_expand<<<nb * ((n + LE_ROWS - 1) / LE_ROWS), 1024, 0, ctx->stream>>>(
         n, ctx->list_size, ctx->fcap, w + 2 * at_pt, w + 2 * at_ent, w + 2 * at_off,
         ctx->point + (size_t)dev_b0 * n, ctx->list + (size_t)dev_b0 * ctx->list_size,
         ctx->fpoint + (size_t)dev_b0 * (n + 1), ctx->flist + (size_t)dev_b0 * ctx->fcap);

@@ -71,3 +71,27 @@ def test_caller_lists_in_any_row_order(oracle_mod):
         w.get_forces_nospline(q, F3, o.charge, point, lst, 0)
         w.get_forces_nospline(q, F, o.charge, point, lst, 0)
         assert np.array_equal(F, F3)
+
+
+def test_caller_lists_with_repeated_entries(oracle_mod):
+    """Lists the caller may pass though no builder writes them: a pair listed
+    twice counts twice, a row that many others list, rows left empty."""
+    from qtip4pf_water_amd import Water
+    q, _, box, lj, n = _system((4, 5, 6), 1)
+    o = oracle_mod.Oracle(n, 1, box, lj_rcut=lj)
+    point, lst, _ = o.all_lists(q)
+    full = [list(lst[point[i]:point[i + 1]]) for i in range(n - 1)]
+    rows = [r + r if i % 3 == 0 else [] if i % 7 == 1 else r for i, r in enumerate(full)]
+    # every pair of the second half of the molecules with the last one, often
+    rows = [r + [n - 1] * (20 if i >= n // 2 else 0) for i, r in enumerate(rows)]
+    flat = [j for r in rows for j in r]
+    assert len(flat) <= lst.size and flat.count(n - 1) > 1024
+    lst[:] = 0
+    lst[:len(flat)] = flat
+    point[:] = np.concatenate([[0], np.cumsum([len(r) for r in rows])])
+    Fr, F = np.zeros_like(q), np.zeros_like(q)
+    o.get_forces(q, Fr, point, lst, 0)
+    with Water(n, 1, box, lj_rcut=lj) as w:
+        w.get_forces_nospline(q, F, o.charge, point, lst, 0)
+    d = np.linalg.norm((F - Fr).reshape(-1, 3), axis=1)
+    assert np.max(d / np.linalg.norm(Fr.reshape(-1, 3), axis=1)) < 1e-10
