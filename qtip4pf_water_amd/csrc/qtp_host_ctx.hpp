@@ -38,7 +38,7 @@ struct qtp_ctx {
     int ntile = 0;       // real-space tiles per evaluation
     int nmb = 0;         // LJ/intra blocks per evaluation
     int lj_lpm = 16;     // lanes per molecule in k_ljintra
-    bool rs_cull = false;  // k_realspace skips tiles beyond r_c (boxes >= RS_CULL_MIN_BOX r_c)
+    bool rs_cull = false;  // k_realspace_cull: tiles beyond r_c skipped (boxes >= RS_CULL_MIN_BOX r_c)
     double4 *rs_sites = nullptr;  // CULL: [E][nblk * 64] sites (x, y, z, q)
     double *rs_box = nullptr;     // CULL: [E][nblk][RS_BOX] block and 8-site cluster bounding boxes
     unsigned char *rs_far = nullptr;  // CULL: [E][ntile] 1 = tile skipped this evaluation
