@@ -7,14 +7,24 @@
 // ---------------------------------------------------------------------------
 // force phase: E single-bead evaluations (forces.cpp:468-630)
 // ---------------------------------------------------------------------------
+// Blocks per chunk group of k_ksum_mf that give each wave at most one slot
+// group (contexts with the vector kernels only have no slot groups), and the
+// largest multiple of that count which leaves no block without one.
+static int ksum_mf_blocks(const qtp_ctx *ctx)
+{
+    return std::max(1, (ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES);
+}
+static int ksum_mf_max_mult(const qtp_ctx *ctx)
+{
+    return std::min(4, std::max(1, ctx->ks_nslot / ksum_mf_blocks(ctx)));
+}
 // Launch shape of k_ksum_mf for E evaluations: blocks per chunk group (a
-// multiple of the count that gives each wave at most one slot group, more when
-// the launch has few blocks, or as tuned), chunks per block (as tuned, else
-// the most of 1, 2, 4, 8 that still leaves 2048 blocks), chunk groups.
+// multiple of ksum_mf_blocks, more than once it when the launch has few blocks,
+// or as tuned), chunks per block (as tuned, else the most of 1, 2, 4, 8 that
+// still leaves 2048 blocks), chunk groups.
 static void ksum_mf_shape(const qtp_ctx *ctx, int E, int *usplit, int *cpb, int *ncg)
 {
-    const int req = std::max(1, (ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES);
-    const int umax = std::min(4, std::max(1, ctx->ks_nslot / req));
+    const int req = ksum_mf_blocks(ctx), umax = ksum_mf_max_mult(ctx);
     const int mult = ctx->ks_usplit > 0 ? std::min(ctx->ks_usplit, umax)
                                         : ((long)E * ctx->nac * req < 128 ? umax : 1);
     *usplit = req * mult;

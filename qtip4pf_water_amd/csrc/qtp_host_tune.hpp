@@ -148,7 +148,7 @@ int tune_time(qtp_ctx *ctx, int n, float *ms)
 std::vector<TuneCfg> tune_candidates(const qtp_ctx *ctx)
 {
     std::vector<TuneCfg> out;
-    const int umax = std::min(4, std::max(1, ctx->ks_nslot / ((ctx->ks_nslot + KS_WAVES - 1) / KS_WAVES)));
+    const int umax = ksum_mf_max_mult(ctx);
     // (tile-culling boxes: k_realspace_cull, neither of the two has an effect)
     for (int rsw : ctx->rs_cull ? std::vector<int>{RS_WAVES} : std::vector<int>{4, 2})
         for (int lpm : {16, 64})
