@@ -527,17 +527,7 @@ static int update_sc_impl(qtp_ctx *ctx, double *q, double *p, const double *mass
     res.raw(ctx->out, o, 2);
     res.raw(ctx->heat, &h0, 1);
     CHK(res.down());
-    std::vector<int> fl(P);
-    HIPCHK(hipMemcpy(fl.data(), ctx->flag, P * sizeof(int), hipMemcpyDeviceToHost));
-    for (int b = 0; b < P; ++b)
-        if (fl[b]) {
-            HIPCHK(hipMemcpy(point + (long)b * ctx->n_mols, ctx->point + (size_t)b * ctx->n_mols,
-                             ctx->n_mols * sizeof(int), hipMemcpyDeviceToHost));
-            // the row's used part
-            const int used = point[(long)(b + 1) * ctx->n_mols - 1];
-            HIPCHK(hipMemcpy(list + (long)b * ctx->list_size, ctx->list + (size_t)b * ctx->list_size,
-                             used * sizeof(int), hipMemcpyDeviceToHost));
-        }
+    CHK(download_rebuilt(ctx, point, list));
     if (heat) *heat = h0;
     if (energy) *energy = o[0];
     if (sc_pot) *sc_pot = o[1];
@@ -572,12 +562,7 @@ static int update_class_impl(qtp_ctx *ctx, double *q, double *p, const double *m
     res.disp(ctx->disp, disp, 1);
     res.raw(ctx->out, o, 2);
     CHK(res.down());
-    int fl = 0;
-    HIPCHK(hipMemcpy(&fl, ctx->flag, sizeof(int), hipMemcpyDeviceToHost));
-    if (fl) {
-        HIPCHK(hipMemcpy(point, ctx->point, ctx->n_mols * sizeof(int), hipMemcpyDeviceToHost));
-        HIPCHK(hipMemcpy(list, ctx->list, point[ctx->n_mols - 1] * sizeof(int), hipMemcpyDeviceToHost));
-    }
+    CHK(download_rebuilt(ctx, point, list));
     if (energy) *energy = o[0];
     ctx->state_set = false;
     return QTP_OK;

@@ -378,6 +378,25 @@ static int upload_with_lists(qtp_ctx *ctx, Xfer &x, const int *point, const int 
     return QTP_OK;
 }
 
+// The half lists of the beads that the last step rebuilt: a bead's entries and
+// zeros up to list_size, the row the list kernels write (neighbour.cpp:23-32).
+// Only the entries travel.
+static int download_rebuilt(qtp_ctx *ctx, int *point, int *list)
+{
+    const int n = ctx->n_mols;
+    std::vector<int> fl(ctx->P);
+    HIPCHK(hipMemcpy(fl.data(), ctx->flag, ctx->P * sizeof(int), hipMemcpyDeviceToHost));
+    for (int b = 0; b < ctx->P; ++b) {
+        if (!fl[b]) continue;
+        int *pt = point + (long)b * n, *ls = list + (long)b * ctx->list_size;
+        HIPCHK(hipMemcpy(pt, ctx->point + (size_t)b * n, n * sizeof(int), hipMemcpyDeviceToHost));
+        HIPCHK(hipMemcpy(ls, ctx->list + (size_t)b * ctx->list_size, pt[n - 1] * sizeof(int),
+                         hipMemcpyDeviceToHost));
+        std::fill(ls + pt[n - 1], ls + ctx->list_size, 0);
+    }
+    return QTP_OK;
+}
+
 static int check_finite(qtp_ctx *ctx, const double *a, long n, const char *what)
 {
     constexpr uint64_t EXP = 0x7ff0000000000000ull;
