@@ -241,7 +241,9 @@ int qtp_set_state(qtp_ctx *ctx, const double *q, const double *p, const double *
                   const double *mass);
 /* Download state in reference layout; any pointer may be NULL. */
 int qtp_get_state(qtp_ctx *ctx, double *q, double *p, double *F, double *fphys, double *disp);
-/* Download the half lists in reference layout. */
+/* Download the half lists in reference layout: the resident state's, or those
+ * that the last call on host arrays was given (up to 1024 molecules with zeros
+ * outside the entries, whatever the caller's arrays hold there) or rebuilt. */
 int qtp_get_lists(qtp_ctx *ctx, int *point, int *list);
 
 /* Virial of every bead at the resident positions (as qtp_get_forces_virial):

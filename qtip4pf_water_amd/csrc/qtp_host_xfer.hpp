@@ -193,8 +193,9 @@ static int download_planar(qtp_ctx *ctx, const double *src, int nb, double *ref)
 }
 
 // The caller's half lists of nb beads (point[b][n], entries packed from
-// ent[off[b]]) into the device half and full lists: row i of the full list
-// holds its partners j < i (rows that list i) ascending, then its own row.
+// ent[off[b]]) into the device half lists (zeros around the entries) and full
+// lists: row i of the full list holds its partners j < i (rows that list i)
+// ascending, then its own row.
 // LE_ROWS rows a block: incoming counts of all rows (LDS atomics) and offsets,
 // then a wave per row picks its incoming entries out of all entries in their
 // order, which is by rising row, and looks up the rows.  All reads are
@@ -229,6 +230,9 @@ __global__ __launch_bounds__(1024) void k_list_expand(int n, int list_size, long
         if (part == 0) H[k] = j;
         atomicAdd(&inc[j], 1);
     }
+    // nothing of an earlier list around the entries
+    for (int k = part * 1024 + tid; k < list_size; k += nparts * 1024)
+        if (k < k0 || k >= k1) H[k] = 0;
     __syncthreads();
     // offsets: thread i <-> row i (the last row of a half list is empty)
     int v = 0;

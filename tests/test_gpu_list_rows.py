@@ -57,3 +57,31 @@ def test_rebuilt_rows_come_back_whole(nside, P):
                 assert not disp[3 * n * b:3 * n * (b + 1)].any()
             else:
                 assert np.array_equal(point[rp], point0[rp]) and np.array_equal(lst[rl], lst0[rl])
+
+
+@pytest.mark.parametrize("nside,P", [((4, 4, 4), 1), ((4, 4, 5), 4), ((9, 10, 11), 2), ((10, 11, 10), 2)])
+def test_lists_held_are_the_callers(nside, P):
+    """A call on host arrays replaces the rows that the context held, the part
+    before and behind the entries with them: here rows of half the entries,
+    from list[3] on."""
+    from qtip4pf_water_amd import Water
+    n, q, box, lj = _system(nside, P)
+    with Water(n, P, box, lj_rcut=lj) as w:
+        N = w.list_size
+        point, lst = _lists(w, q, P, n)
+        for b in range(P):
+            pt, row = point[b * n:(b + 1) * n], lst[b * N:(b + 1) * N]
+            rows = [row[pt[i]:(pt[i] + pt[i + 1]) // 2] for i in range(n - 1)]
+            flat = np.concatenate(rows)
+            assert flat.size + 13 < pt[n - 1]
+            row[:] = 0
+            row[3:3 + flat.size] = flat
+            pt[:] = 3 + np.concatenate([[0], np.cumsum([r.size for r in rows])])
+        F = np.zeros_like(q)
+        if P == 1:
+            w.get_forces_nospline(q, F, None, point, lst, 0)
+        else:
+            w.force_eval_sc_nospline(q, F, None, None, point, lst)
+        got_p, got_l = w.get_lists()
+        assert np.array_equal(got_p, point)
+        assert np.array_equal(got_l, lst)
