@@ -160,7 +160,7 @@ static HeatArgs heat_args(const qtp_ctx *ctx, bool with_heat)
         h.heat_acc = ctx->heat;
         h.heat_step = ctx->heat_step;
         h.ntile = ctx->ptile;
-        h.nh = ctx->P * ctx->ptile * HP_PARTS;
+        h.nh = ctx->ptile * HP_PARTS;
     }
     return h;
 }

@@ -369,7 +369,7 @@ static int alloc_all(qtp_ctx *ctx)
     CHK(dalloc(ctx, &ctx->nq, (size_t)P * N3));
     CHK(dalloc(ctx, &ctx->np, (size_t)P * N3));
     CHK(dalloc(ctx, &ctx->ppart, 2 * (size_t)ctx->ptile + 2));
-    CHK(dalloc(ctx, &ctx->hpart, (size_t)ctx->P * ctx->ptile * HP_PARTS + 1));
+    CHK(dalloc(ctx, &ctx->hpart, heat_doubles(ctx->P, ctx->ptile)));
     CHK(dalloc(ctx, &ctx->obs, (size_t)ctx->ptile * 4 + 64));
     CHK(dalloc(ctx, &ctx->obs_out, 4));
     CHK(dalloc(ctx, &ctx->ntrace, 1));

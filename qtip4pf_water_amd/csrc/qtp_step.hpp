@@ -311,20 +311,39 @@ __device__ __forceinline__ void cayley_half(double &uq, double &up, double m, do
     uq = temp;
 }
 
-// A lane's heat of mode k into the partials of the tile's groups of HP_DOFS
-// dofs, hpart[(k * ntile + tile) * HP_PARTS + group] (every form of the
-// propagation sums in the same order).
+// The heat of a step is summed over groups of HP_DOFS dofs, HP_PARTS of them
+// in a 64-dof tile: per mode over the group (heat_group), then over the modes
+// (k_prop_dofs in LDS, k_prop_inv from k_prop_fwd's sums), in the same order in
+// both forms of the propagation.  hpart[tile * HP_PARTS + group] is that sum;
+// behind these, at [(tile * HP_PARTS + group) * P + k], are the sums per mode of
+// the two-launch form.  A partial per mode and group left k_heat's one block
+// 73 728 to read at 4096 x 32, 22.5 us; these 2304 take 5.2, and the propagation
+// as long as before.
 constexpr int HP_DOFS = 16, HP_PARTS = 64 / HP_DOFS;
+__host__ __device__ inline size_t heat_doubles(int P, int ntile)
+{
+    return (size_t)(P + 1) * ntile * HP_PARTS;
+}
 __device__ __forceinline__ double heat_group(double h)
 {
     for (int o = HP_DOFS / 2; o > 0; o >>= 1) h += __shfl_xor(h, o, 64);
     return h;
 }
-__device__ __forceinline__ void heat_part(double h, double *hpart, int k, int tile, int ntile)
+__device__ __forceinline__ void heat_part(double h, double *hpart, int k, int P, int tile, int ntile)
 {
     const int lane = threadIdx.x & 63;
     h = heat_group(h);
-    if (lane % HP_DOFS == 0) hpart[((long)k * ntile + tile) * HP_PARTS + lane / HP_DOFS] = h;
+    if (lane % HP_DOFS == 0)
+        hpart[(long)ntile * HP_PARTS + ((long)tile * HP_PARTS + lane / HP_DOFS) * P + k] = h;
+}
+// Sum over the modes by the HP_DOFS lanes of a group: lane i those with
+// k = i mod HP_DOFS.
+template <class Get>
+__device__ __forceinline__ double heat_modes(int i, int P, Get get)
+{
+    double s = 0.0;
+    for (int k = i; k < P; k += HP_DOFS) s += get(k);
+    return heat_group(s);
 }
 
 // Kick, forward normal-mode transform and first half step for mode k of 64
@@ -334,7 +353,7 @@ __device__ __forceinline__ void heat_part(double h, double *hpart, int k, int ti
 // grid: ntile * P (tile-major, XCD-remapped), 64 threads.
 // part[tile] = centroid KE after the first half step (tile partial);
 // part[ntile + tile] = chi-square partial (device random numbers);
-// hpart: KE before - KE after of mode k's Langevin step (heat_part).
+// hpart: KE before - KE after of mode k's Langevin step, per mode (heat_part).
 __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__restrict__ Cm,
                                                  const double4 *__restrict__ mode,
                                                  const double2 *__restrict__ mscale,
@@ -397,8 +416,8 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
             part[tile] = ke0;
             part[A.ntile + tile] = chi;
         }
-        // the centroid's heat slot: PILE-L's here, PILE-G's in k_prop_inv
-        if (A.nvt && !pile_g) heat_part(h, hpart, 0, tile, A.ntile);
+        // the centroid's heat: PILE-L's here, PILE-G's in k_prop_inv
+        if (A.nvt && !pile_g) heat_part(h, hpart, 0, P, tile, A.ntile);
         return;
     }
     cayley_half(uq, up, m, A.halfdt, md);
@@ -412,7 +431,7 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
             up = md.z * up + sqm_atom[at] * md.w * xi;
             h -= 0.5 * up * up / m;
         }
-        heat_part(h, hpart, k, tile, A.ntile);
+        heat_part(h, hpart, k, P, tile, A.ntile);
     }
     cayley_half(uq, up, m, A.halfdt, md);
     nq[k * N3 + f] = uq;
@@ -422,7 +441,8 @@ __global__ __launch_bounds__(64) void k_prop_fwd(PropArgs A, const double *__res
 // Centroid rescale (Bussi, tau -> 0), its second half step, inverse
 // transform to bead b and displacement tracking.  One wavefront per
 // (dof tile, bead).   grid: ntile * P (tile-major, XCD-remapped), 64 threads.
-// hpart (mode 0) = - centroid KE after the rescale (bead-0 waves).
+// The bead-0 waves sum the tile's heat over the modes; with the rescale the
+// centroid's is - KE after it.
 __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__restrict__ Cm,
                                                  const double4 *__restrict__ mode,
                                                  const double *__restrict__ nq,
@@ -442,8 +462,9 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
     const int at = f % A.NAP, d = f / A.NAP;
     const bool va = at < A.n_atoms;
     const double m = va ? m_atom[at] : 1.0;
-    double u0q = nq[f], u0p = np[f];
-    if (A.nvt && A.cthermo == 0 && A.cmode != 2) {
+    double u0q = nq[f], u0p = np[f], h0 = 0.0;
+    const bool pile_g = A.nvt && A.cthermo == 0 && A.cmode != 2;
+    if (pile_g) {
         const double ke = wave_sum_array(part, A.ntile);
         double R, g2;
         if (A.host_dev) {
@@ -464,10 +485,13 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
             if (R + sqrt(c / ((1.0 - c) * x)) < 0.0) alpha = -alpha;
         }
         u0p *= alpha;
-        if (b == 0) {
-            double h = va ? -0.5 * u0p * u0p / m : 0.0;
-            heat_part(h, hpart, 0, tile, A.ntile);
-        }
+        if (b == 0) h0 = heat_group(va ? -0.5 * u0p * u0p / m : 0.0);
+    }
+    if (A.nvt && b == 0) {
+        const int i = lane % HP_DOFS, part_i = tile * HP_PARTS + lane / HP_DOFS;
+        const double *hm = hpart + (long)A.ntile * HP_PARTS + (long)part_i * P;
+        const double h = heat_modes(i, P, [&](int k) { return k == 0 && pile_g ? h0 : hm[k]; });
+        if (i == 0) hpart[part_i] = h;
     }
     cayley_half(u0q, u0p, m, A.halfdt, mode[0]);
     double xq = Cm[b] * u0q, xp = Cm[b] * u0p;
@@ -500,7 +524,7 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
 // grid: HP_PARTS * ntile (XCD-remapped), HP_DOFS * P threads,
 // prop_dofs_lds(P); P <= PD_MAX_BEADS.
 constexpr int PD_MAX_BEADS = 64;
-inline size_t prop_dofs_lds(int P) { return (size_t)(2 * P * HP_DOFS + P * (P + 1)) * sizeof(double); }
+inline size_t prop_dofs_lds(int P) { return (size_t)(2 * P * HP_DOFS + P * (P + 1) + P) * sizeof(double); }
 __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     PropArgs A, const double *__restrict__ Cm, const double4 *__restrict__ mode,
     const double2 *__restrict__ mscale, double *__restrict__ q, double *__restrict__ p,
@@ -511,6 +535,7 @@ __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     extern __shared__ double S[];
     const int P = A.P, CP = P + 1;
     double *SQ = S, *SP = S + P * HP_DOFS, *C = S + 2 * P * HP_DOFS;  // C: [P][P + 1]
+    double *H = C + P * CP;                                           // heat per mode
     const int blk = xcd_remap(blockIdx.x, gridDim.x);
     const int tid = threadIdx.x, k = tid / HP_DOFS, i = tid % HP_DOFS;  // mode or bead, dof
     const int tile = blk / HP_PARTS, group = blk % HP_PARTS;
@@ -547,7 +572,7 @@ __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
             h -= 0.5 * up * up / m;
         }
         h = heat_group(h);
-        if (i == 0) hpart[((long)k * A.ntile + tile) * HP_PARTS + group] = h;
+        if (i == 0) H[k] = h;
     }
     if (tid == 0 && group == 0) {
         part[tile] = 0.0;
@@ -558,6 +583,10 @@ __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     SQ[tid] = uq;
     SP[tid] = up;
     __syncthreads();
+    if (A.nvt && k == 0) {
+        const double h = heat_modes(i, P, [&](int kk) { return H[kk]; });
+        if (i == 0) hpart[blk] = h;
+    }
     double xq = C[k] * SQ[i], xp = C[k] * SP[i];
 #pragma unroll 8
     for (int kk = 1; kk < P; ++kk) {
@@ -893,7 +922,7 @@ constexpr int NL_FUSED_MAXMOL = 1024;
 // of block 0 here so that it costs no launch of its own.
 struct HeatArgs {
     const double *part;  // centroid KE partials (ntile) then chi partials
-    const double *hpart; // heat partials of the modes (nh)
+    const double *hpart; // heat partials of the dofs (nh)
     double *heat_acc, *heat_step;
     int ntile, nh;
 };
