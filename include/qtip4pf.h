@@ -454,7 +454,11 @@ int qtp_nn_train(qtp_nn *nn, int n_steps, int batch_frames, double lr, uint64_t 
 int qtp_set_nn(qtp_ctx *ctx, qtp_nn *nn);
 
 /* Per-kernel timing of the last qtp_run (HIP events around each launch of the
- * named kernel class on the context's stream); for measurement only. */
+ * named kernel class on the context's stream); for measurement only.  The
+ * kernels are then launched one by one, also those that the one-stream form of
+ * a force phase puts into one launch.  kernel "one_stream_phase": *launches =
+ * force phases queued in that form since qtp_create, timing on or off (a
+ * captured one counts once, however often it is replayed). */
 int qtp_enable_timing(qtp_ctx *ctx, int on);
 int qtp_get_timing(qtp_ctx *ctx, const char *kernel, double *ms_total, int *launches);
 

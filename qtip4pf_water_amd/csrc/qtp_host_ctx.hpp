@@ -70,6 +70,7 @@ struct qtp_ctx {
     // a list check the SC step leaves to the next force phase's second stream
     bool lists_defer = false, lists_heat = false;
     const unsigned long long *lists_ctr = nullptr;
+    int n_one_stream = 0;  // force phases queued (or captured) in the one-stream form
     // propagation as one launch per step (k_prop_dofs) where the thermostat
     // and the bead count allow it: -1 and 1 yes, 0 no (k_prop_fwd + k_prop_inv)
     int prop_fused = -1;

@@ -279,6 +279,7 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
             ctx->epart, ctx->ep_stride, ctx->ep_real, vp);
     }
     if (fused) {
+        ctx->n_one_stream++;
         int usplit, cpb, ncg;
         ksum_mf_shape(ctx, E, &usplit, &cpb, &ncg);
         usplit = (ctx->ks_nslot_ph + 3) / 4;
