@@ -327,6 +327,14 @@ int qtp_run_observed(qtp_ctx *ctx, int n_steps, int is_nvt, int every, double *t
  * second stream after the LJ/intramolecular kernel (0-4), site chunks per
  * structure-factor block of the matrix-core path (1, 2, 4, 8, 16; 0 by launch
  * size)}.
+ * The defaults run a force phase's kernels in three launches on one stream;
+ * a value of its own (not -1, 0 or the default 4) for real-space coefficients
+ * as literals, structure-factor blocks, waves per tile, tiles on the second
+ * stream or site chunks, or the vector k-space kernels, takes two streams and
+ * about twice the launches, also where it names the shape in use (a force
+ * evaluation with two waves per tile: 45 % longer at 512 molecules x 1 bead,
+ * 3 % at 512 x 32; where the large launches gain more from such a value,
+ * qtp_autotune finds it).
  * Every configuration gives the same forces up to summation order. */
 int qtp_get_tuning(const qtp_ctx *ctx, int cfg[9]);
 /* Sets cfg (QTP_ERR_ARG for values the context cannot run); with a state set,
@@ -335,7 +343,8 @@ int qtp_set_tuning(qtp_ctx *ctx, const int cfg[9]);
 /* Times one force evaluation of every bead of the resident state (the force
  * work of one step captured as a graph, replayed between HIP events, median
  * of 5 runs of replays) under each
- * candidate configuration, keeps the fastest and recomputes the state's
+ * candidate configuration (of the one-stream and of the two-stream form, from
+ * whichever the context starts), keeps the fastest and recomputes the state's
  * forces with it.  The choice is cached per system (molecules, beads, box,
  * Ewald and LJ parameters) for the process, so contexts of one shape are
  * timed once; flags & 1 times again.  report[11] (may be NULL): best ms,

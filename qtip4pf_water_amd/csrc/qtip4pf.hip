@@ -1710,34 +1710,40 @@ int qtp_autotune(qtp_ctx *ctx, int flags, double report[11])
         const TuneCfg dflt = current_tuning(ctx);
         st = tune_time(ctx, 5, &dflt_ms);
         best_ms = dflt_ms;
-        for (const TuneCfg &c : tune_candidates(ctx)) {
-            if (st != QTP_OK) break;
+        // the best of the two-stream form by itself: the second search below
+        // varies it, also while the one-stream form leads
+        TuneCfg two = dflt;
+        float two_ms = phase_fused(ctx) ? 0.f : dflt_ms;
+        auto time_cfg = [&](const TuneCfg &c) {
             apply_tuning(ctx, c);
             float ms = 0.f;
             st = tune_time(ctx, 5, &ms);
             ++n_timed;
+            if (st != QTP_OK) return;
             // a candidate has to beat the configuration in hand by TUNE_MARGIN,
             // so that timing noise between near-equal ones does not decide
-            if (st == QTP_OK && ms < best_ms * (1.0f - TUNE_MARGIN)) {
+            if (!phase_fused(ctx) && (two_ms == 0.f || ms < two_ms * (1.0f - TUNE_MARGIN))) {
+                two_ms = ms;
+                two = c;
+            }
+            if (ms < best_ms * (1.0f - TUNE_MARGIN)) {
                 best_ms = ms;
                 best = c;
             }
+        };
+        for (const TuneCfg &c : tune_candidates(ctx)) {
+            if (st != QTP_OK) break;
+            time_cfg(c);
         }
         // then the real-space share of the second stream and the structure-
-        // factor chunks per block, one at a time on the best so far
+        // factor chunks per block, one at a time on the two-stream form's best
+        // so far
         for (int sp = 1; sp <= 4 + 5 && st == QTP_OK; ++sp) {
-            if (sp > 4 && !best.kmf) break;
-            TuneCfg c = best;
+            if (sp > 4 && !two.kmf) break;
+            TuneCfg c = two;
             if (sp <= 4) c.rsplit = sp;
             else c.cpb = 1 << (sp - 5);
-            apply_tuning(ctx, c);
-            float ms = 0.f;
-            st = tune_time(ctx, 5, &ms);
-            ++n_timed;
-            if (st == QTP_OK && ms < best_ms * (1.0f - TUNE_MARGIN)) {
-                best_ms = ms;
-                best = c;
-            }
+            time_cfg(c);
         }
         if (st == QTP_OK) {
             std::lock_guard<std::mutex> g(g_tune_mu);

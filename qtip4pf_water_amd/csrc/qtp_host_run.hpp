@@ -194,11 +194,17 @@ static NlArgs nlist_args(const qtp_ctx *ctx, int force_all, bool with_heat, cons
     return a;
 }
 
-// Whether a phase takes the one-stream form (k_phase_pairs,
-// k_phase_reduce): the default launch choices without tile culling or splines.
+// Whether the context's phases may take the one-stream form (k_phase_pairs,
+// k_phase_reduce), and whether a phase now does: it covers neither tile culling
+// nor splines, and of the launch choices the defaults except lj_lpm and
+// mf_small.
+static bool phase_fused_ok(const qtp_ctx *ctx)
+{
+    return ctx->kf_mf_ok && !ctx->rs_cull && !ctx->spl_on;
+}
 static bool phase_fused(const qtp_ctx *ctx)
 {
-    return !ctx->timing && ctx->kf_mf && !ctx->rs_cull && !ctx->spl_on && ctx->rs_split == 0 &&
+    return phase_fused_ok(ctx) && !ctx->timing && ctx->kf_mf && ctx->rs_split == 0 &&
            ctx->rs_waves == 4 && ctx->rs_carg != 0 && ctx->ks_usplit == 0 && ctx->ks_cpb == 0;
 }
 

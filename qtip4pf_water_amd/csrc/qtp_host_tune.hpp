@@ -149,6 +149,15 @@ std::vector<TuneCfg> tune_candidates(const qtp_ctx *ctx)
 {
     std::vector<TuneCfg> out;
     const int umax = ksum_mf_max_mult(ctx);
+    const int smax = ctx->kforce_mf_lds_small <= 64 * 1024 ? 1 : 0;
+    // the one-stream phase; all others take two streams
+    if (phase_fused_ok(ctx))
+        for (int lpm : {16, 64})
+            for (int small = 0; small <= smax; ++small) {
+                TuneCfg c;
+                c.lpm = lpm, c.kmf = 1, c.small = small, c.fused = ctx->prop_fused;
+                out.push_back(c);
+            }
     // (tile-culling boxes: k_realspace_cull, neither of the two has an effect)
     for (int rsw : ctx->rs_cull ? std::vector<int>{RS_WAVES} : std::vector<int>{4, 2})
         for (int lpm : {16, 64})
@@ -160,7 +169,6 @@ std::vector<TuneCfg> tune_candidates(const qtp_ctx *ctx)
                         out.push_back(c);
                         continue;
                     }
-                    const int smax = ctx->kforce_mf_lds_small <= 64 * 1024 ? 1 : 0;
                     for (int small = 0; small <= smax; ++small)
                         for (int u = 1; u <= umax; u *= 2) {
                             c.small = small, c.usplit = u;

@@ -33,3 +33,23 @@ def test_autotune_without_matrix_kspace(P):
         assert np.max(np.abs(F2 - F)) < 1e-9 * np.max(np.abs(F))
         w.run(5)
         assert w.scalars()["status"] == 0
+
+
+@pytest.mark.parametrize("start", [{}, {"rs_waves": 2}, {"ksum_blocks_per_chunk": 1}])
+@pytest.mark.parametrize("P", [1, 4])
+def test_autotune_times_the_one_stream_form(P, start):
+    """From any starting configuration: the one-stream force phase with both
+    lane counts and both force-block widths is among the candidates."""
+    from qtip4pf_water_amd import Water
+    q, p, box = _state(5, 15.54, P, 61)
+    with Water(125, P, box, lj_rcut=cfg.lj_rcut_for(15.54)) as w:
+        w.set_tuning(**start)
+        w.set_state(q, p)
+        a = w.timing("one_stream_phase")[1]
+        F = w.get_state()[2]
+        r = w.autotune(retime=True)
+        # captured once a candidate: the four, each with every phase of a step
+        assert w.timing("one_stream_phase")[1] - a >= 4 * (2 if P > 1 else 1)
+        assert r["best_ms"] <= r["default_ms"] * 1.001
+        F2 = w.get_state()[2]
+        assert np.max(np.abs(F2 - F)) < 1e-9 * np.max(np.abs(F))
