@@ -168,7 +168,6 @@ int qtp_create(const qtp_params *prm, qtp_ctx **out)
     // a whole wave per molecule when one launch covers few molecules
     set_lj_lanes(ctx, (long)std::max(ctx->P, 1) * ctx->n_mols <= 2048 ? 64 : 16);
     ctx->ptile = (3 * ctx->NAP + 63) / 64;
-    ctx->prop_lds = 0;
     ctx->cells_ok = cell_grid(ctx->drv.r_skin, ctx->box.L, ctx->n_mols, ctx->cg);
     *out = ctx;
 

@@ -21,7 +21,8 @@ struct qtp_ctx {
     qtp_derived drv{};
     std::string err;
     hipStream_t stream = nullptr;
-    // second stream for the k-space half of a force phase (fork/join by events)
+    // second stream for the k-space half of a force phase that does not take
+    // the one-stream form (fork/join by events)
     hipStream_t s2 = nullptr;
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
     // third stream for the learned correction of classical steps
@@ -50,7 +51,7 @@ struct qtp_ctx {
     SplTab spl{};
     double *spl_coef = nullptr, *fspl = nullptr;
     int ptile = 0;       // propagation tiles (64 planar dofs each)
-    size_t kforce_lds = 0, kforce_lds_split = 0, ksum_lds = 0, prop_lds = 0;
+    size_t kforce_lds = 0, kforce_lds_split = 0, ksum_lds = 0;
     int kf_chunk = KF_CHUNK, kf_chunk_split = KF_CHUNK;  // k_kforce record staging
     // split k_kforce in the SC phases when its P * ceil(n_atoms/63) blocks
     // would not fill two per CU (small systems); large ones have blocks enough
@@ -67,7 +68,7 @@ struct qtp_ctx {
     int rs_waves = RS_WAVES;  // waves per k_realspace tile block (2 or 4)
     int rs_split = 0;         // eighths of the real-space tiles on the second stream (0-4)
     int ks_cpb = 0;           // structure-factor chunks per k_ksum_mf block (0: by launch size)
-    // a list check the SC step leaves to the next force phase's second stream
+    // a list check that a step leaves to its first force phase
     bool lists_defer = false, lists_heat = false;
     const unsigned long long *lists_ctr = nullptr;
     int n_one_stream = 0;  // force phases queued (or captured) in the one-stream form

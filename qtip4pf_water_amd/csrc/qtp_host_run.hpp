@@ -221,10 +221,10 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     const double g = ctx->ff.gamma_vs, h = ctx->ff.half1mg;
     double *vp = vout ? ctx->vpart : nullptr;
     // The k-space sums (ksum, sreduce) and the LJ/intramolecular kernel do not
-    // depend on the real-space kernel: they run on the second stream, joined
-    // before kforce, with a share of the real-space tiles after them.  With
-    // per-kernel timing on, everything stays on one stream so each launch is
-    // timed alone.
+    // depend on the real-space kernel.  They share its launches (phase_fused),
+    // or run on the second stream, joined before kforce, with a share of the
+    // real-space tiles after them.  With per-kernel timing on, everything stays
+    // on one stream, a launch per kernel, so that each is timed alone.
     const bool fused = phase_fused(ctx);
     const bool fork = !ctx->timing && !fused;
     hipStream_t sk = fork ? ctx->s2 : s;
@@ -233,10 +233,11 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     // where its kernels leave the chip room beside the first part
     const int nt_b = fork ? (int)((long)ctx->ntile * ctx->rs_split / 8) : 0;
     const int nt_a = ctx->ntile - nt_b;
-    // coefficients in SGPRs (more waves per SIMD) for large grids, where
-    // that measured faster (4096 x 32: 3.42 against 3.60 ms); literals
-    // for small ones (216 x 32: no gain, and the second stream's kernels
-    // lost more than the launch gained)
+    // two streams: coefficients in SGPRs (more waves per SIMD) for large
+    // grids, where that measured faster (4096 x 32: 3.42 against 3.60 ms);
+    // literals for small ones (216 x 32: no gain, and the second stream's
+    // kernels lost more than the launch gained).  k_phase_pairs and
+    // k_realspace_cull always take SGPRs.
     const bool carg = ctx->rs_carg >= 0 ? ctx->rs_carg == 1
                                         : (long)E * ctx->ntile >= RS_CARG_BLOCKS;
     RsArgs ra = rs_args(ctx, pos, vp);
@@ -251,7 +252,7 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
     } while (0)
         if (ctx->rs_cull) {
             // tiles a block, while the blocks fill the chip several times over
-            ra.gs = (int)std::min(16L, std::max(1L, (long)E * nt / RS_CULL_WAVES));
+            ra.gs = (int)std::min(16L, std::max(1L, (long)E * nt / RS_CULL_BLOCKS));
             const int grid = E * ((nt + ra.gs - 1) / ra.gs);
             if (ra.fx.cubic) {
                 if (vout) k_realspace_cull<true, true><<<grid, 64 * RS_CW, 0, st>>>(ra);
@@ -323,73 +324,73 @@ static int run_phase(qtp_ctx *ctx, const double *pos, int E, int lmode, int lbas
         }
 #undef QTP_PHASE
     } else {
-    if (fork) {
-        HIPCHK(hipEventRecord(ctx->ev_fork, s));
-        HIPCHK(hipStreamWaitEvent(sk, ctx->ev_fork, 0));
-    }
-    {
-        TimeScope ts(ctx, "ksum");
-        if (ctx->kf_mf) {
-            int usplit, cpb, ncg;
-            ksum_mf_shape(ctx, E, &usplit, &cpb, &ncg);
-            const KsArgs ka = ks_args(ctx, pos, ctx->AC, cpb * ctx->AC, ncg, usplit);
+        if (fork) {
+            HIPCHK(hipEventRecord(ctx->ev_fork, s));
+            HIPCHK(hipStreamWaitEvent(sk, ctx->ev_fork, 0));
+        }
+        {
+            TimeScope ts(ctx, "ksum");
+            if (ctx->kf_mf) {
+                int usplit, cpb, ncg;
+                ksum_mf_shape(ctx, E, &usplit, &cpb, &ncg);
+                const KsArgs ka = ks_args(ctx, pos, ctx->AC, cpb * ctx->AC, ncg, usplit);
 #define QTP_KS_MF(CAP) k_ksum_mf<CAP><<<E * ncg * usplit, 64 * KS_WAVES, ctx->ksum_mf_lds, sk>>>(ka)
-            switch (ctx->ks_cap) {
-            case 1: QTP_KS_MF(1); break;
-            case 2: QTP_KS_MF(2); break;
-            case 3: QTP_KS_MF(3); break;
-            case 4: QTP_KS_MF(4); break;
-            default: QTP_KS_MF(KS_ACC); break;
-            }
+                switch (ctx->ks_cap) {
+                case 1: QTP_KS_MF(1); break;
+                case 2: QTP_KS_MF(2); break;
+                case 3: QTP_KS_MF(3); break;
+                case 4: QTP_KS_MF(4); break;
+                default: QTP_KS_MF(KS_ACC); break;
+                }
 #undef QTP_KS_MF
-        } else
-            k_ksum<<<E * ctx->ngc * ctx->nac, 256, ctx->ksum_lds, sk>>>(
-                pos, N3, ctx->charge, ctx->n_atoms, ctx->NAP, g, h, ctx->ew, ctx->groups, ctx->G,
-                ctx->AC, ctx->ngc, ctx->nac, ctx->spart);
-    }
-    {
-        TimeScope ts(ctx, "sreduce");
-        // partials per group: one per chunk (vector k_ksum) or chunk group
-        int nparts = ctx->nac;
-        if (ctx->kf_mf) {
-            int usplit, cpb;
-            ksum_mf_shape(ctx, E, &usplit, &cpb, &nparts);
+            } else
+                k_ksum<<<E * ctx->ngc * ctx->nac, 256, ctx->ksum_lds, sk>>>(
+                    pos, N3, ctx->charge, ctx->n_atoms, ctx->NAP, g, h, ctx->ew, ctx->groups, ctx->G,
+                    ctx->AC, ctx->ngc, ctx->nac, ctx->spart);
         }
-        k_sreduce<<<E * ctx->ngr, 256, 0, sk>>>(sr_args(ctx, nparts, vp));
-    }
-    // a list check deferred by the step (only the LJ kernel reads the lists)
-    if (ctx->lists_defer) {
-        ctx->lists_defer = false;
-        CHK(run_lists(ctx, 0, ctx->lists_heat, ctx->lists_ctr, sk));
-    }
-    {
-        TimeScope ts(ctx, "ljintra");
-        const LjArgs la = lj_args(ctx, pos, lmode, lbase, vp);
+        {
+            TimeScope ts(ctx, "sreduce");
+            // partials per group: one per chunk (vector k_ksum) or chunk group
+            int nparts = ctx->nac;
+            if (ctx->kf_mf) {
+                int usplit, cpb;
+                ksum_mf_shape(ctx, E, &usplit, &cpb, &nparts);
+            }
+            k_sreduce<<<E * ctx->ngr, 256, 0, sk>>>(sr_args(ctx, nparts, vp));
+        }
+        // a list check deferred by the step (only the LJ kernel reads the lists)
+        if (ctx->lists_defer) {
+            ctx->lists_defer = false;
+            CHK(run_lists(ctx, 0, ctx->lists_heat, ctx->lists_ctr, sk));
+        }
+        {
+            TimeScope ts(ctx, "ljintra");
+            const LjArgs la = lj_args(ctx, pos, lmode, lbase, vp);
 #define QTP_LJ_LAUNCH(VIR, LPM) k_ljintra<VIR, LPM><<<E * ctx->nmb, 256, 0, sk>>>(la)
-        if (ctx->lj_lpm == 64) {
-            if (vout) QTP_LJ_LAUNCH(true, 64);
-            else QTP_LJ_LAUNCH(false, 64);
-        } else {
-            if (vout) QTP_LJ_LAUNCH(true, 16);
-            else QTP_LJ_LAUNCH(false, 16);
-        }
+            if (ctx->lj_lpm == 64) {
+                if (vout) QTP_LJ_LAUNCH(true, 64);
+                else QTP_LJ_LAUNCH(false, 64);
+            } else {
+                if (vout) QTP_LJ_LAUNCH(true, 16);
+                else QTP_LJ_LAUNCH(false, 16);
+            }
 #undef QTP_LJ_LAUNCH
-    }
-    if (ctx->spl_on) {
-        TimeScope ts(ctx, "spline");
-        if (vout)
-            k_spline<true><<<E * ctx->nblk, 256, 0, sk>>>(
-                pos, N3, ctx->n_atoms, ctx->NAP, ctx->nblk, ctx->box, ctx->spl, ctx->spl_coef,
-                ctx->fspl, ctx->epart, ctx->ep_stride, ctx->ep_spl, vp);
-        else
-            k_spline<false><<<E * ctx->nblk, 256, 0, sk>>>(
-                pos, N3, ctx->n_atoms, ctx->NAP, ctx->nblk, ctx->box, ctx->spl, ctx->spl_coef,
-                ctx->fspl, ctx->epart, ctx->ep_stride, ctx->ep_spl, vp);
-    }
-    if (nt_b > 0) launch_rs(sk, nt_a, nt_b);
-    if (fork) HIPCHK(hipEventRecord(ctx->ev_join, sk));
-    launch_rs(s, 0, nt_a);
-    if (fork) HIPCHK(hipStreamWaitEvent(s, ctx->ev_join, 0));
+        }
+        if (ctx->spl_on) {
+            TimeScope ts(ctx, "spline");
+            if (vout)
+                k_spline<true><<<E * ctx->nblk, 256, 0, sk>>>(
+                    pos, N3, ctx->n_atoms, ctx->NAP, ctx->nblk, ctx->box, ctx->spl, ctx->spl_coef,
+                    ctx->fspl, ctx->epart, ctx->ep_stride, ctx->ep_spl, vp);
+            else
+                k_spline<false><<<E * ctx->nblk, 256, 0, sk>>>(
+                    pos, N3, ctx->n_atoms, ctx->NAP, ctx->nblk, ctx->box, ctx->spl, ctx->spl_coef,
+                    ctx->fspl, ctx->epart, ctx->ep_stride, ctx->ep_spl, vp);
+        }
+        if (nt_b > 0) launch_rs(sk, nt_a, nt_b);
+        if (fork) HIPCHK(hipEventRecord(ctx->ev_join, sk));
+        launch_rs(s, 0, nt_a);
+        if (fork) HIPCHK(hipStreamWaitEvent(s, ctx->ev_join, 0));
     }
     {
         TimeScope ts(ctx, "kforce");
@@ -608,9 +609,9 @@ static int run_sc_step(qtp_ctx *ctx, int nvt, int host_dev, unsigned long long *
     }
     }
     HIPCHK(hipGetLastError());
-    // the one-kernel list check and rebuild: on the first force phase's
-    // second stream, ahead of the LJ kernel, so that the real-space kernel
-    // starts right after the propagation
+    // the list check and rebuild of up to 1024 molecules: in the first force
+    // phase's first launch (phase_fused) or on its second stream ahead of the LJ
+    // kernel, so that the real-space tiles start right after the propagation
     if (ctx->n_mols <= NL_FUSED_MAXMOL && !use_cells(ctx)) {
         ctx->lists_defer = true;
         ctx->lists_heat = nvt != 0;

@@ -28,7 +28,8 @@ __device__ __forceinline__ void kw_table(double2 *row, double r, double bk, doub
 }
 
 // sin and cos of x for the factor tables: x = n pi/2 + r with pi/2 in three
-// parts (each fma rounds once, to the size of the small difference, so r is as
+// parts of 33, 33 and 53 bits (Cody and Waite's scheme with the parts that
+// fdlibm publishes; each fma rounds once, to the size of the small difference, so r is as
 // accurate as x for every n that a double holds exactly), then the Taylor series of sin and
 // cos to degrees 17 and 18 on |r| <= pi/4 (truncation below 1e-17).  About 40
 // vector instructions; the library's reduction for any size of x takes more

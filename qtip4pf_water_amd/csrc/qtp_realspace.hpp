@@ -38,10 +38,19 @@ namespace qtp {
 // the chip holds at once, against 8448 in two rounds with four).
 constexpr int RS_WAVES = 4;  // the default W
 constexpr long RS_CARG_BLOCKS = 16384;  // grids at least this large use CARG
-// boxes at least this many r_c wide use k_realspace_cull.  x 32 beads, steps/s of the
-// first culling form (block boxes only, zeroed slots) against the plain one
-// at the reference's Ewald point: 216 H2O (2.06 r_c) -8%, 1000 (2.66) +7%,
-// 1728 (2.91) +7%, 4096 (3.36) +21%
+// Boxes at least this many r_c wide use k_realspace_cull, with the two-stream
+// phase around it.  Time of a step against the one-stream phase without culling
+// (k_max 8):
+//   molecules x beads   2.3 r_c   2.55    2.8    3.0-3.3
+//   512 x 1              +78 %    +73 %   +70 %
+//   512 x 32             +15 %    +12 %   +13 %   +12 %
+//   1000 x 1                      +54 %   +53 %   +51 %
+//   1000 x 32                      +3 %    -1 %    -7 %
+//   1728 x 1                      +27 %   +26 %
+//   1728 x 16                       0 %    -8 %   -13 %
+// It pays where the launch fills the chip several times over; the line was
+// drawn for 1000 molecules x 32 beads, before the one-stream phase, which gains
+// most where the launch is small.
 constexpr double RS_CULL_MIN_BOX = 2.5;
 
 // Smallest distance between [a0, a1] and the periodic images of [b0, b1]
@@ -230,7 +239,7 @@ struct RsArgs {
     double gamma, half1mg;
     const int2 *tiles;
     int ntile, t0, nt;
-    int gs;  // k_realspace_cull: tiles a wave
+    int gs;  // k_realspace_cull: tiles a block
     Box box;
     Ewald ew;
     double *rpart, *epart;
@@ -242,7 +251,6 @@ struct RsArgs {
     RsFix fx;
 };
 
-// The tile of block `block` of nblocks (XCD-remapped), by its 64 W threads.
 // Pass 2 over the queue entries q0 ... q1 - 1 of this lane: rows il (site i0 +
 // il) and columns jl (site j0 + jl; coordinates sJ[jl], reaction fj[.][jo +
 // jl]).  Adds to fi, fj, the energy and (VIR) the virial.  near: the tile may
@@ -328,6 +336,7 @@ __device__ __forceinline__ void rs_pairs(const double4 *sI, const double4 *sJ, d
     }
 }
 
+// The tile of block `block` of nblocks (XCD-remapped), by its 64 W threads.
 template <bool VIR, bool CARG, int W>
 __device__ __forceinline__ void rs_tile(RsLds<W> &L, int block, int nblocks, const RsArgs &A)
 {
@@ -480,7 +489,7 @@ __global__ __launch_bounds__(64 * W) void k_realspace(const RsArgs A)
 // (168) -> 156, 2197 x 1 28 -> 29.  One wave a tile: 593, 324, 161, 36.
 // grid: E * ceil(nt / gs), 64 RS_CW threads.
 constexpr int RS_CW = 2, RS_UNROLL = 4, RS_QUEUE = 1024;
-constexpr long RS_CULL_WAVES = 16384;  // blocks of a launch at which gs grows past 1
+constexpr long RS_CULL_BLOCKS = 16384;  // a launch has at least this many blocks, or gs = 1
 template <bool CUBIC>
 struct RsU {
     using type = uint2;

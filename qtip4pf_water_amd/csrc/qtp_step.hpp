@@ -950,7 +950,9 @@ struct NlLds {
 };
 // Whether bead b's lists are rebuilt this step: its two largest O
 // displacements (update.cpp:356-385), or forced.  By a block of NT threads;
-// the same value in every thread.
+// the same value in every thread.  k_phase_pairs asks in several blocks (the
+// list blocks and the LJ blocks) and relies on one answer: the library is built
+// without FMA contraction, so every copy rounds the same.
 template <int NT>
 __device__ __forceinline__ int list_flag(double *s1, double *s2, int *flag, int b, const NlArgs &A)
 {
@@ -1000,10 +1002,10 @@ __device__ __forceinline__ void list_heat(const HeatArgs &heat)
         heat.heat_acc[0] -= ret;
     }
 }
-// Bead `block` of nblocks by NT threads.
-template <int NT>
-__device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, const NlArgs &A)
+__global__ __launch_bounds__(1024) void k_nlist_bead(const NlArgs A)
 {
+    __shared__ NlLds S;
+    constexpr int NT = 1024;
     const int n_mols = A.n_mols, NAP = A.NAP, NMP = A.NMP, list_size = A.list_size;
     const double *__restrict__ q = A.q;
     const Box &box = A.box;
@@ -1017,8 +1019,8 @@ __device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, co
     int *__restrict__ list = A.list;
     int *__restrict__ flist = A.flist;
     int *__restrict__ status = A.status;
-    const int b = block, tid = threadIdx.x;
-    if (A.heat.part && b == nblocks - 1) {  // the extra last block: the heat sum only
+    const int b = blockIdx.x, tid = threadIdx.x;
+    if (A.heat.part && b == (int)gridDim.x - 1) {  // the extra last block: the heat sum only
         list_heat(A.heat);
         return;
     }
@@ -1120,11 +1122,6 @@ __device__ __forceinline__ void nlist_block(NlLds &S, int block, int nblocks, co
             kh += __popcll(bh);
         }
     }
-}
-__global__ __launch_bounds__(1024) void k_nlist_bead(const NlArgs A)
-{
-    __shared__ NlLds L;
-    nlist_block<1024>(L, blockIdx.x, gridDim.x, A);
 }
 
 // The same rebuild in the launches of the one-stream phase, spread over the
