@@ -44,13 +44,14 @@ from qtip4pf_water_amd import flops  # noqa: E402
 
 PEAK_FP64_TFLOPS = 78.6   # MI355X FP64 (vector and matrix), AMD published
 KERNELS = ["realspace", "ksum", "sreduce", "kforce", "ljintra", "sites", "finalize", "sc1",
-           "sc2", "prop", "prop_a", "prop_b", "check", "nlist"]
+           "sc2", "prop", "prop_a", "prop_b", "check", "nlist", "tilefar"]
 
 
 def measured_traffic(kernel):
-    """HBM bytes per launch of `kernel` from the committed counter summary
-    (profiles/pmc_traffic_sc_pimd_216x32.txt: FETCH_SIZE and WRITE_SIZE passes
-    of this workload, calibrated against a copy of known size), or None."""
+    """HBM bytes per launch of `kernel` ("step": of all launches of a step) from
+    the committed counter summary (profiles/pmc_traffic_sc_pimd_216x32.txt:
+    read and write counters of this workload, calibrated against a copy of
+    known size), or None."""
     path = os.path.join(ROOT, "profiles", "pmc_traffic_sc_pimd_216x32.txt")
     try:
         with open(path) as f:
@@ -402,13 +403,23 @@ def main():
         "ns_per_day": sps * wl["dtfs"] * 0.0864,
         "algorithmic_tflops": step_flops * sps / 1e12,
         "roofline": {
-            # FP64 vector ALU work (no matrix instructions in this kernel);
-            # MI355X's FP64 vector and matrix peaks are both 78.6 TFLOP/s
-            "bound": "fp64_valu",
-            "kernel": dom,
-            "achieved": achieved,
+            # the whole step as it is timed, one graph launch: vector and
+            # matrix FP64 work, whose peaks are both 78.6 TFLOP/s on MI355X
+            "bound": "fp64",
+            "kernel": "step",
+            "achieved": step_flops * sps / 1e12,
             "peak": PEAK_FP64_TFLOPS,
             "unit": "TFLOP/s",
+            "frac": step_flops * sps / 1e12 / PEAK_FP64_TFLOPS,
+            "traffic": measured_traffic("step") if a.workload == "c2" else None,
+            "flops_per_launch": step_flops,
+            "us_per_launch": 1e6 / sps,
+        },
+        # the longest kernel launched by itself (kernel_us likewise): the timed
+        # steps may run it inside a launch with others
+        "kernel_alone": {
+            "kernel": dom,
+            "achieved": achieved,
             "frac": achieved / PEAK_FP64_TFLOPS,
             "traffic": measured_traffic(dom) if a.workload == "c2" else None,
             "flops_per_launch": fl[dom] * evals_per_launch,
