@@ -336,14 +336,13 @@ __device__ __forceinline__ void heat_part(double h, double *hpart, int k, int P,
     if (lane % HP_DOFS == 0)
         hpart[(long)ntile * HP_PARTS + ((long)tile * HP_PARTS + lane / HP_DOFS) * P + k] = h;
 }
-// Sum over the modes by the HP_DOFS lanes of a group: lane i those with
-// k = i mod HP_DOFS.
-template <class Get>
-__device__ __forceinline__ double heat_modes(int i, int P, Get get)
+// A lane's share of the sum over the modes, by the HP_DOFS lanes of a group:
+// lane i the modes k = i mod HP_DOFS (then heat_group).
+__device__ __forceinline__ double heat_modes(int i, int P, const double *h)
 {
     double s = 0.0;
-    for (int k = i; k < P; k += HP_DOFS) s += get(k);
-    return heat_group(s);
+    for (int k = i; k < P; k += HP_DOFS) s += h[k];
+    return s;
 }
 
 // Kick, forward normal-mode transform and first half step for mode k of 64
@@ -462,8 +461,15 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
     const int at = f % A.NAP, d = f / A.NAP;
     const bool va = at < A.n_atoms;
     const double m = va ? m_atom[at] : 1.0;
-    double u0q = nq[f], u0p = np[f], h0 = 0.0;
+    double u0q = nq[f], u0p = np[f];
     const bool pile_g = A.nvt && A.cthermo == 0 && A.cmode != 2;
+    // the sums per mode are loaded here and added up behind the stores
+    const int i16 = lane % HP_DOFS, group = tile * HP_PARTS + lane / HP_DOFS;
+    double h0 = 0.0, hm = 0.0;
+    if (A.nvt && b == 0) {
+        const double *H = hpart + (long)A.ntile * HP_PARTS + (long)group * P;
+        hm = pile_g && i16 == 0 ? heat_modes(HP_DOFS, P, H) : heat_modes(i16, P, H);
+    }
     if (pile_g) {
         const double ke = wave_sum_array(part, A.ntile);
         double R, g2;
@@ -485,13 +491,7 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
             if (R + sqrt(c / ((1.0 - c) * x)) < 0.0) alpha = -alpha;
         }
         u0p *= alpha;
-        if (b == 0) h0 = heat_group(va ? -0.5 * u0p * u0p / m : 0.0);
-    }
-    if (A.nvt && b == 0) {
-        const int i = lane % HP_DOFS, part_i = tile * HP_PARTS + lane / HP_DOFS;
-        const double *hm = hpart + (long)A.ntile * HP_PARTS + (long)part_i * P;
-        const double h = heat_modes(i, P, [&](int k) { return k == 0 && pile_g ? h0 : hm[k]; });
-        if (i == 0) hpart[part_i] = h;
+        if (b == 0) h0 = va ? -0.5 * u0p * u0p / m : 0.0;
     }
     cayley_half(u0q, u0p, m, A.halfdt, mode[0]);
     double xq = Cm[b] * u0q, xp = Cm[b] * u0p;
@@ -506,6 +506,10 @@ __global__ __launch_bounds__(64) void k_prop_inv(PropArgs A, const double *__res
     q[idx] = xq;
     p[idx] = xp;
     if (va && (at % 3) == 0) disp[((long)b * 3 + d) * NMP + at / 3] += xq - qold;
+    if (A.nvt && b == 0) {
+        const double h = heat_group(pile_g ? h0 + hm : hm);
+        if (i16 == 0) hpart[group] = h;
+    }
 }
 
 // The whole propagation of a step in one launch when the centroid needs no
@@ -583,10 +587,6 @@ __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     SQ[tid] = uq;
     SP[tid] = up;
     __syncthreads();
-    if (A.nvt && k == 0) {
-        const double h = heat_modes(i, P, [&](int kk) { return H[kk]; });
-        if (i == 0) hpart[blk] = h;
-    }
     double xq = C[k] * SQ[i], xp = C[k] * SP[i];
 #pragma unroll 8
     for (int kk = 1; kk < P; ++kk) {
@@ -597,6 +597,10 @@ __global__ __launch_bounds__(HP_DOFS * PD_MAX_BEADS) void k_prop_dofs(
     q[idx] = xq;
     p[idx] = xp;
     if (va && (at % 3) == 0) disp[((long)k * 3 + d) * NMP + at / 3] += xq - qold;
+    if (A.nvt && k == 0) {
+        const double h = heat_group(heat_modes(i, P, H));
+        if (i == 0) hpart[blk] = h;
+    }
 }
 
 // The thermostat's heat for one step: pile_g's return value (KE before -
